@@ -39,6 +39,16 @@ __device__ inline double wave_fmax(double v)
     return uni(v);
 }
 
+// Keeps a value in a vector register at this point: its computation is
+// neither moved past here nor speculated above it.
+template <typename T>
+__device__ inline void pin(T &v)
+{
+#if defined(__HIP_DEVICE_COMPILE__)
+    asm volatile("" : "+v"(v));
+#endif
+}
+
 __device__ inline bool wave_any(bool p) { return __any((int)p) != 0; }
 
 // A lane's own barrier: orders the accesses of its wavefront's threads to
@@ -291,44 +301,66 @@ struct LuFlags {
     uint64_t nonfinite, worst;
 };
 
-// One row of a row program: every thread runs one op of the row's kind on
-// M = [factor slots | solve vector], in the factor precision R. Rows run in
-// order within the wavefront (LDS accesses of one wavefront complete in issue
-// order), so a row sees the results of every earlier row. The peel tests are
-// computed in FP64 on the values. kSolve: a solve program (R_MACZ and R_DIV
-// rows), whose R_MACZ and idle rows run one branch-free path: an idle row, or
-// an op whose multiplier is zero, writes its slot's own value back (a row
-// never holds two ops on one slot; idle rows touch slot 0 or pads). The
-// refactor's R_MAC rows keep the plain path, which measured faster there.
-template <typename R, bool kSolve, typename MP>
-__device__ inline void run_row(esl::uint2_t w, MP M, double growth, LuFlags &f)
+// A row's word decoded: the LDS addresses of the thread's operands, its
+// peel-test flags and the row's kind (uniform).
+struct RowOp {
+    uint32_t d, b, c, fl, kind;
+};
+
+// base: the LDS address of M. kLast: the last position of a block, where a
+// chain row may sit (its word holds a length and a segment: its operands
+// become the target's slot). The decoded values are pinned here, ahead of
+// their use, which ends the word's life, so that the word's register can be
+// refilled in place.
+template <typename R, bool kSolve, bool kLast>
+__device__ inline RowOp row_decode(esl::uint2_t w, uint32_t base)
 {
-    const uint32_t kind = __builtin_amdgcn_readfirstlane(esl::row_kind(w.y));
-    const uint32_t d = w.x & 0xffffu, b = w.x >> 16, c = w.y & 0xffffu;
-    if (kind == R_CHAIN) return;   // run after its block of rows (run_chain)
-    if (kSolve && kind != R_DIV) {
-        const R v = M[d], A = M[b], B = M[c];
-        const R p = v - A * B;
-        const bool keep = kind == R_NOP || B == R(0);
-        M[d] = keep ? v : p;
-    } else if (!kSolve && kind == R_MAC) {
-        // (refactor programs hold no R_MACZ rows: checked on the host)
-        const R v = M[d], A = M[b], B = M[c];
-        M[d] = v - A * B;
-    } else if (kind == R_DIV) {
-        const R v = M[d], A = M[b];
-        const R q = v / A;
-        M[d] = q;
-        if (kSolve) return;   // solve programs carry no peel tests (flags 0)
-        const uint32_t fl = esl::row_flags(w.y);
-        const bool u = fl & kFlagUnscaled;
-        const uint64_t nf = dbits((double)(q - q));
-        const bool check_growth = growth > 0;
-        f.bad |= u && check_growth && !(fabs((double)A) >= growth * fabs((double)v));
-        f.nonfinite |= ((u && !check_growth) || (fl & kFlagScaled)) ? nf : 0;
-        const uint64_t lb = u ? dbits(fabs((double)q)) : 0;
-        f.worst = lb > f.worst ? lb : f.worst;
+    RowOp o;
+    o.kind = esl::row_kind((uint32_t)__builtin_amdgcn_readfirstlane((int)w.y));
+    const uint32_t d = w.x & 0xffffu;
+    uint32_t b = w.x >> 16, c = w.y & 0xffffu;
+    if (kLast) {
+        b = o.kind == R_CHAIN ? d : b;
+        c = o.kind == R_CHAIN ? d : c;
     }
+    o.d = base + d * (uint32_t)sizeof(R);
+    o.b = base + b * (uint32_t)sizeof(R);
+    o.c = base + c * (uint32_t)sizeof(R);
+    o.fl = kSolve ? 0u : esl::row_flags(w.y);
+    pin(o.d);
+    pin(o.b);
+    pin(o.c);
+    if (!kSolve) pin(o.fl);
+    return o;
+}
+
+// The arithmetic of one row on the operands just read (v, A, B of slots d,
+// b, c). The peel tests are computed in FP64 on the values. Every row runs a
+// branch-free multiply-subtract, whose zero test (kSolve: R_MACZ) keeps the
+// slot's own value; idle rows and threads work on their pad slots, a chain
+// row (run after its block) keeps its target's value, and a division
+// replaces the result.
+template <typename R, bool kSolve, bool kLast>
+__device__ inline void row_finish(const RowOp &o, R v, R A, R B, double growth, LuFlags &f)
+{
+    R r = v - A * B;
+    if (kSolve) r = B == R(0) ? v : r;
+    if (kLast) r = o.kind == R_CHAIN ? v : r;
+    if (o.kind == R_DIV) {
+        R piv = A;
+        pin(piv);   // a branch: every row would pay for a speculated division
+        r = v / piv;
+        if (!kSolve) {   // solve programs carry no peel tests (flags 0)
+            const bool u = o.fl & kFlagUnscaled;
+            const uint64_t nf = dbits((double)(r - r));
+            const bool check_growth = growth > 0;
+            f.bad |= u && check_growth && !(fabs((double)A) >= growth * fabs((double)v));
+            f.nonfinite |= ((u && !check_growth) || (o.fl & kFlagScaled)) ? nf : 0;
+            const uint64_t lb = u ? dbits(fabs((double)r)) : 0;
+            f.worst = lb > f.worst ? lb : f.worst;
+        }
+    }
+    *(__attribute__((address_space(3))) R *)(uintptr_t)o.d = r;
 }
 
 // One chain row (R_CHAIN word w): the thread's run of len terms on target
@@ -436,40 +468,70 @@ __device__ void run_bchain(esl::uint2_t w, const esl::uint2_t *segs, const uint3
 
 // Runs a row program of `rows` rows, a multiple of kRing (its words
 // followed by at least kRing more rows, which are only loaded), with kRing
-// rows of words in flight. M
-// (R elements) and the words may be address-space qualified pointers. The
-// word loads are pinned in row order (scheduling barriers) and each refills
-// the register its row just used, so the oldest load completes first and a
-// row waits only for its own word, never for the whole ring. A chain row,
-// always a block's last row, runs after the block (segs, cw: the program's
-// chain segments and terms; null for programs without chain rows).
+// rows of words in flight: every thread runs one op of the row's kind on
+// M = [factor slots | solve vector] (R elements), in the factor precision R.
+// Rows run in order within the wavefront (LDS accesses of one wavefront
+// complete in issue order), so a row sees the results of every earlier row.
+// A row is bound by its own LDS round trip (reads, two FP64 operations, the
+// write the next row's reads queue behind), so nothing else stands in it:
+// while a row's reads are in flight its word's register is refilled and the
+// next row's word is decoded (operands and kind), and the only branch is a
+// division's. The word loads are pinned in row order (scheduling barriers)
+// and each refills the register its row just used, so the oldest load
+// completes first and a row waits only for the next row's word. A chain
+// row, always a block's last row, runs after the block (segs, cw: the
+// program's chain segments and terms; null for programs without chain
+// rows), outside the block loop, whose loads its own waits would drain.
+// Measured (a serial RC line of 182 nodes, 928 rows an iteration, one lane a
+// SIMD): 470 -> 228 cycles a row; its transient step loop 43.7 -> 26.0 ms for
+// 1,000 lanes and 200 iterations. The floor is the LDS round trip: a
+// read-multiply-subtract-write chain alone takes 98 cycles a link, a
+// division 78 more.
 template <typename R, bool kSolve = false, typename WP, typename MP>
 __device__ void run_rows(WP words, uint32_t rows, MP M, double growth, LuFlags &f, uint32_t tid, uint32_t pad,
                          const esl::uint2_t *segs = nullptr, const uint32_t *cw = nullptr)
 {
-    const WP w = words + tid;
+    if (rows == 0) return;
+    using lp = const __attribute__((address_space(3))) R *;
+    const uint32_t base = (uint32_t)(uintptr_t)(lp)M;
+    WP w = words + tid;
     esl::uint2_t q[kRing];
 #pragma unroll
     for (int k = 0; k < kRing; k++) {
         q[k] = esl::uint2_t{w[k * kWave].x, w[k * kWave].y};
         __builtin_amdgcn_sched_barrier(0);
     }
-    for (uint32_t row = 0; row < rows; row += kRing) {
-        const esl::uint2_t last = q[kRing - 1];
+    RowOp o = row_decode<R, kSolve, false>(q[0], base);
+    uint32_t row = 0;
+    for (;;) {
+        uint32_t lk;
+        do {
+            w += kRing * kWave;
 #pragma unroll
-        for (int k = 0; k < kRing; k++) {
-            // use the word, then refill its register (no register rotation)
-            run_row<R, kSolve>(q[k], M, growth, f);
-            const size_t at = (size_t)(row + kRing + k) * kWave;
-            q[k] = esl::uint2_t{w[at].x, w[at].y};
-            __builtin_amdgcn_sched_barrier(0);
-        }
-        if (segs && __builtin_amdgcn_readfirstlane(esl::row_kind(last.y)) == R_CHAIN) {
+            for (int k = 0; k < kRing; k++) {
+                const R v = *(lp)(uintptr_t)o.d, A = *(lp)(uintptr_t)o.b, B = *(lp)(uintptr_t)o.c;
+                const RowOp cur = o;
+                __builtin_amdgcn_sched_barrier(0);
+                q[k] = esl::uint2_t{w[k * kWave].x, w[k * kWave].y};
+                o = k + 1 == kRing - 1 ? row_decode<R, kSolve, true>(q[kRing - 1], base)
+                                       : row_decode<R, kSolve, false>(q[(k + 1) % kRing], base);
+                __builtin_amdgcn_sched_barrier(0);
+                if (k == kRing - 1) row_finish<R, kSolve, true>(cur, v, A, B, growth, f);
+                else row_finish<R, kSolve, false>(cur, v, A, B, growth, f);
+                __builtin_amdgcn_sched_barrier(0);
+                if (k == kRing - 1) lk = cur.kind;
+            }
+            row += kRing;
+        } while (row < rows && lk != R_CHAIN);
+        if (segs && lk == R_CHAIN) {
+            const WP lw = words + (size_t)(row - 1) * kWave + tid;
+            const esl::uint2_t last{lw->x, lw->y};
             if (__builtin_amdgcn_readfirstlane(last.y) & kChainBcast)
                 run_bchain<R, kSolve>(last, segs, cw, M, pad, tid);
             else
                 run_chain<R, kSolve>(last, segs, cw, M, tid);
         }
+        if (row >= rows) return;
     }
 }
 

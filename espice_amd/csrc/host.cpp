@@ -518,7 +518,13 @@ class OpGraph {
         // 5. words
         const u32 used = (u32)rows.size();
         const u32 padded = (used + esl::kRing - 1) / esl::kRing * esl::kRing;
-        out.words.assign((size_t)(padded + esl::kRing) * esl::kWave, esl::uint2_t{0, 0});
+        // idle rows: every thread on its pad slot (the kernels run them as
+        // multiply-subtracts)
+        out.words.resize((size_t)(padded + esl::kRing) * esl::kWave);
+        for (size_t k = 0; k < out.words.size(); k++) {
+            const u32 pad = pad_base + (u32)(k % esl::kWave);
+            out.words[k] = esl::uint2_t{pad | (pad << 16), pad | ((u32)esl::R_NOP << 16)};
+        }
         out.seg.clear();
         out.cw.clear();
         out.chains = (u32)chains.size();
@@ -2020,7 +2026,6 @@ bool validate_big(const TapeHostProg &o, u32 n)
             for (u32 t = 0; t < (u32)esl::kWave; t++) {
                 const esl::uint2_t w = o.blk_words[r * esl::kWave + t];
                 if (esl::row_kind(w.y) != kind || (w.y >> 22) != 0) return false;
-                if (kind == esl::R_NOP) continue;
                 const u32 d = w.x & 0xffff, bb = w.x >> 16, c = w.y & 0xffff;
                 if (d >= lim || bb >= lim || c >= lim) return false;
             }
@@ -2125,7 +2130,6 @@ bool validate_tape(const TapeHostProg &o, u32 n, u32 nnz)
                     (w.y & esl::kChainBcast) != bflag)
                     return false;
                 if (solve && esl::row_flags(w.y) != 0) return false;   // no peel tests in the solves
-                if (kind == esl::R_NOP) continue;
                 if (kind == esl::R_CHAIN && bflag) {
                     if ((w.x & 0xffff) >= lim) return false;
                     continue;
