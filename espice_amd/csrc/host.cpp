@@ -309,7 +309,10 @@ bool gp_factor(u32 n, const u32 *col_ptr, const u32 *row_idx, const double *vals
 }
 
 // Minimum degree on the pattern of A + A^T (ties to the lowest index).
-vector<u32> min_degree(u32 n, const vector<u32> &col_ptr, const vector<u32> &row_idx)
+// shallow: the next vertex is instead the one of least 2 * degree + level,
+// level being the longest elimination path that ends in it. depth: the
+// longest path of the order; fill: the entries of L (and of U).
+vector<u32> min_degree(u32 n, const vector<u32> &col_ptr, const vector<u32> &row_idx, bool shallow, u32 &depth, size_t &fill)
 {
     vector<vector<u32>> adj(n);
     for (u32 j = 0; j < n; j++)
@@ -324,22 +327,28 @@ vector<u32> min_degree(u32 n, const vector<u32> &col_ptr, const vector<u32> &row
         a.erase(std::unique(a.begin(), a.end()), a.end());
     }
     vector<char> gone(n, 0);
+    vector<u32> level(n, 0);
+    fill = 0;
     vector<u32> q;
     q.reserve(n);
     vector<u32> merged;
     for (u32 step = 0; step < n; step++) {
         u32 best = NONE;
         size_t bd = SIZE_MAX;
-        for (u32 v = 0; v < n; v++)
-            if (!gone[v] && adj[v].size() < bd) {
-                bd = adj[v].size();
+        for (u32 v = 0; v < n; v++) {
+            const size_t key = shallow ? 2 * adj[v].size() + level[v] : adj[v].size();
+            if (!gone[v] && key < bd) {
+                bd = key;
                 best = v;
             }
+        }
         const u32 v = best;
         q.push_back(v);
         gone[v] = 1;
         const vector<u32> nb = adj[v];
+        fill += nb.size();
         for (u32 u : nb) {
+            level[u] = std::max(level[u], level[v] + 1);
             merged.clear();
             std::set_union(adj[u].begin(), adj[u].end(), nb.begin(), nb.end(), std::back_inserter(merged));
             adj[u].clear();
@@ -348,7 +357,31 @@ vector<u32> min_degree(u32 n, const vector<u32> &col_ptr, const vector<u32> &row
         }
         adj[v].clear();
     }
+    depth = *std::max_element(level.begin(), level.end());
     return q;
+}
+
+// The column order of a deck. Plain minimum degree eats a line of resistors
+// from its ends, one column after another (a 182-node RC line: 366 + 550
+// rows of refactor and solve, all but a thread of each idle); the shallow
+// order takes alternate vertices first and its path is logarithmic (80 + 81
+// rows at 1.9 times the fill). It is taken where it at least halves the
+// depth (lines, stacks); on meshes it saves a quarter of the depth for more
+// fill, and the plain order stays. Decks with transistors keep the plain
+// order too: their stages have gain, so the rounding of another order can
+// move a point's iteration count (inverter chains: 60 % of the points),
+// where two-terminal decks agree to rounding in any order.
+vector<u32> deck_order(u32 n, const vector<u32> &col_ptr, const vector<u32> &row_idx, bool transistors)
+{
+    u32 d0 = 0, d1 = 0;
+    size_t f0 = 0, f1 = 0;
+    vector<u32> q = min_degree(n, col_ptr, row_idx, false, d0, f0);
+    if (transistors || 8 * (size_t)d0 < n) return q;   // a path of n / 8 columns: nothing like a line
+    vector<u32> q1 = min_degree(n, col_ptr, row_idx, true, d1, f1);
+    // a lane holds its factors and about eight n-vectors in LDS: the extra
+    // fill must not cost it the LDS of half a workgroup
+    if ((n + 2 * f1 + 8 * (size_t)n) * 8 > 80 * 1024) return q;
+    return 2 * d1 <= d0 ? q1 : q;
 }
 
 // Row programs. Every update of the refactor or the solve is one op
@@ -1483,7 +1516,9 @@ bool compile_deck(const esl_deck *d, Compiled &c, std::string &err)
         else if (in.kind == esl::kQ)
             for (int e = 0; e < 12; e++) in.slot[e] = find_slot(c, in.t[BJT_ENT[e][0]], in.t[BJT_ENT[e][1]]);
     }
-    c.q = min_degree(n, c.col_ptr, c.row_idx);
+    c.q = deck_order(n, c.col_ptr, c.row_idx,
+                     c.kind_first[esl::kMos] != c.kind_first[esl::kMos + 1] ||
+                         c.kind_first[esl::kQ] != c.kind_first[esl::kQ + 1]);
 
     // per-kind instance arrays
     for (auto &in : c.inst) {
