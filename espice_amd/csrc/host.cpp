@@ -41,6 +41,8 @@ extern "C" hipError_t esl_launch_batch(const void *b, uint32_t grid, uint32_t ld
 extern "C" hipError_t esl_batch_occupancy(uint32_t lds_bytes, int *blocks_per_cu);
 extern "C" hipError_t esl_launch_big(const void *b, hipStream_t s);
 extern "C" hipError_t esl_big_attrs(uint32_t lds_bytes);
+extern "C" hipError_t esl_launch_pack(const double *src, size_t stride, size_t k, uint32_t count, double *out,
+                                      hipStream_t s);
 extern "C" hipError_t esl_launch_gather(const double *x, uint32_t n, const uint32_t *ids, uint32_t k, uint32_t count,
                                         double *out, hipStream_t s);
 
@@ -3608,13 +3610,34 @@ esl_status tran_adaptive_rounds(Engine &E, const esl::TranArgs &ta, const esl::P
     }
     vector<esl::AdaptLane> st(count);
     HIPCHK(hipMemcpyAsync(x, e->x.p, count * n * 8, hipMemcpyDeviceToHost, s));
-    HIPCHK(hipMemcpyAsync(ar.times, e->ttimes.p, count * (size_t)o.max_steps * 8, hipMemcpyDeviceToHost, s));
-    if (o.n_probes)
-        HIPCHK(hipMemcpyAsync(probe_out, e->tprobes.p, count * (size_t)o.max_steps * o.n_probes * 8,
-                              hipMemcpyDeviceToHost, s));
     HIPCHK(hipMemcpyAsync(st.data(), e->tadapt.p, count * sizeof(esl::AdaptLane), hipMemcpyDeviceToHost, s));
     HIPCHK(hipMemcpyAsync(iterations, e->iters.p, count * 4, hipMemcpyDeviceToHost, s));
     HIPCHK(hipStreamSynchronize(s));
+    // the accepted rows only: the device's rows past them hold whatever the
+    // buffers held before
+    size_t top = 0;
+    for (size_t l = 0; l < count; l++)
+        if (reasons[l] == ESL_REASON_OK) top = std::max<size_t>(top, std::min(st[l].steps, o.max_steps));
+    vector<double> rows;
+    auto take = [&](const double *src, double *dst, size_t w) -> hipError_t {
+        if (!top || !w) return hipSuccess;
+        hipError_t er = e->probe_out.ensure(count * top * w * 8);
+        if (er != hipSuccess) return er;
+        er = esl_launch_pack(src, (size_t)o.max_steps * w, top * w, (u32)count, e->probe_out.as<double>(), s);
+        if (er != hipSuccess) return er;
+        rows.resize(count * top * w);
+        er = hipMemcpyAsync(rows.data(), e->probe_out.p, rows.size() * 8, hipMemcpyDeviceToHost, s);
+        if (er != hipSuccess) return er;
+        er = hipStreamSynchronize(s);
+        if (er != hipSuccess) return er;
+        for (size_t l = 0; l < count; l++)
+            if (reasons[l] == ESL_REASON_OK)
+                memcpy(dst + l * o.max_steps * w, rows.data() + l * top * w,
+                       std::min<size_t>(st[l].steps, top) * w * 8);
+        return hipSuccess;
+    };
+    HIPCHK(take(e->ttimes.as<double>(), ar.times, 1));
+    HIPCHK(take(e->tprobes.as<double>(), probe_out, o.n_probes));
     uint64_t lane_it = 0;
     for (size_t l = 0; l < count; l++) {
         if (reasons[l] != ESL_REASON_OK) {   // the operating point failed

@@ -1725,7 +1725,24 @@ __global__ void gather_probes(const double *x, uint32_t n, const uint32_t *ids, 
     out[e] = x[p * n + ids[j]];
 }
 
+// out[p][j] = src[p * stride + j], j < k: the leading part of every lane's rows.
+__global__ void pack_rows(const double *src, size_t stride, size_t k, uint32_t count, double *out)
+{
+    const size_t e = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (e >= (size_t)count * k) return;
+    out[e] = src[e / k * stride + e % k];
+}
+
 }  // namespace esl
+
+extern "C" hipError_t esl_launch_pack(const double *src, size_t stride, size_t k, uint32_t count, double *out,
+                                      hipStream_t s)
+{
+    const size_t total = (size_t)count * k;
+    hipLaunchKernelGGL(esl::pack_rows, dim3((uint32_t)((total + 255) / 256)), dim3(256), 0, s, src, stride, k, count,
+                       out);
+    return hipGetLastError();
+}
 
 extern "C" hipError_t esl_launch_gather(const double *x, uint32_t n, const uint32_t *ids, uint32_t k, uint32_t count,
                                         double *out, hipStream_t s)

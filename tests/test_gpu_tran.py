@@ -206,3 +206,37 @@ def test_adaptive_breakpoint_landing_bitwise_against_oracle(lanes, oracle):
     assert np.array_equal(bits(got["probes"][:, :a]), bits(ref["probes"][:, :a]))
     assert np.min(np.abs(got["times"][0, :a] - 2.5e-9)) <= 1e-19
     eng.close()
+
+
+def test_adaptive_rows_past_the_accepted_ones_stay_the_callers(lanes):
+    """A short adaptive run after a longer one on the same engine leaves the
+    rows past its accepted steps as the caller had them (zeros here)."""
+    fam = circuits.rc_ladder(16, tran=True)
+    vals = fam.sample(5, 9)
+    eng = lanes.Engine(fam.deck.arrays())
+    long = eng.solve_tran_adaptive(vals, 1e-9, 1e-11, probes=[2, 3], max_steps=300)
+    short = eng.solve_tran_adaptive(vals, 2e-10, 1e-11, probes=[2, 3], max_steps=300, dt_max=2e-11)
+    assert (short["reasons"] == 0).all() and (short["accepted"] < long["accepted"]).all()
+    for l, a in enumerate(short["accepted"]):
+        assert (short["times"][l, :a] > 0).all()
+        assert (short["times"][l, a:] == 0).all() and (short["probes"][l, a:] == 0).all()
+    eng.close()
+
+
+@pytest.mark.parametrize("nodes,shallow", [(5, True), (63, True), (64, True), (700, True), (1384, False)])
+def test_lines_take_the_shallow_order_bitwise_against_oracle(lanes, oracle, nodes, shallow):
+    """Lines of resistors take the shallow column order while its fill
+    leaves the lane its LDS; operating points and steps stay bitwise the
+    oracle's in that order."""
+    fam = circuits.rc_ladder(nodes, tran=True)
+    vals = fam.sample(11, 5)
+    eng = lanes.Engine(fam.deck.arrays())
+    _, _, q = eng.pattern()
+    got = eng.solve_tran(vals, 10e-12, 6, probes=[2, 3])
+    if nodes > 5:   # the plain order of a line has about two levels a node
+        assert (eng.info().levels < nodes) == shallow
+    ref = oracle.tran(oracle.Circuit(fam.deck.arrays()), vals, q, 10e-12, 6, probes=[2, 3], threads=5)
+    assert np.array_equal(got["iterations"], ref["iterations"])
+    assert np.array_equal(bits(got["probes"]), bits(ref["probes"]))
+    assert np.array_equal(bits(got["x"]), bits(ref["x"]))
+    eng.close()
