@@ -881,6 +881,206 @@ __device__ inline void priv_load(const PrivLane &G, const uint32_t *col_ptr, con
     for (uint32_t k = tid; k < G.n; k += kWave) L.udiag[k] = G.udiag[k];
 }
 
+// ---- small lanes: the own LU with one row a thread ----
+// A lane of at most 64 unknowns keeps its own factors as a dense n x n array
+// in the LDS tail (column k at F + k n, rows in pivot order: U above the
+// diagonal, the pivots, L below) and each thread keeps one row of the
+// running column (of the solve vector) in a register: a U entry is then a
+// lane broadcast and one multiply-subtract under the row's pattern bit
+// instead of LDS round trips through the sparse column, and the next entry's
+// L column is read meanwhile. Rows outside the pattern are left alone, so
+// every slot takes the replay's operations in the replay's order. Measured
+// on the 16-stage inverter chain (n = 21), cycles an iteration: replay
+// 60.3 k -> @R@, solve 22.6 k -> @S@.
+// Tail layout (doubles): [F n n | row masks of L n | of U n | da nnz u16,
+// row of each pivot step n u16, column order n u16].
+struct PrivDense {
+    double *F;
+    uint64_t *lm, *um;          // [n] bit k of row r: L(r, k) / U(r, k) is in the pattern
+    uint16_t *da, *ip, *q;      // [nnz] F position of each pattern slot; [n] row of step r; [n] column of step k
+};
+
+// Uniform: whether the lane runs dense, and its arrays. Lanes with void
+// pivots (their L columns stay zero) keep the sparse path.
+__device__ inline bool priv_dense(const PrivLane &L, double *tail, uint32_t tail_n, PrivDense &D)
+{
+    const uint32_t n = L.n;
+    if (n > (uint32_t)kWave || uni(L.hdr[2]) != 0) return false;
+    const uint64_t o = (uint64_t)n * n + 2 * n;
+    if (o + ((uint64_t)L.nnz + 2 * n + 3) / 4 > tail_n) return false;
+    D.F = tail;
+    D.lm = reinterpret_cast<uint64_t *>(tail + (size_t)n * n);
+    D.um = D.lm + n;
+    D.da = reinterpret_cast<uint16_t *>(tail + o);
+    D.ip = D.da + L.nnz;
+    D.q = D.ip + n;
+    return true;
+}
+
+// The dense lane's tables from its staged pattern (all threads).
+__device__ inline void priv_dense_build(const PrivLane &L, const PrivDense &D, const uint32_t *col_ptr,
+                                        const uint32_t *q, uint32_t tid)
+{
+    const uint32_t n = L.n;
+    if (tid < n) {
+        D.lm[tid] = 0;
+        D.um[tid] = 0;
+    }
+    wsync();
+    if (tid < n) {
+        const uint32_t k = tid, c = q[k];
+        for (uint32_t p = L.lp[k]; p < L.lp[k + 1]; p++)
+            atomicOr(reinterpret_cast<unsigned long long *>(D.lm + L.li[p]), 1ull << k);
+        for (uint32_t p = L.up[k]; p < L.up[k + 1]; p++)
+            atomicOr(reinterpret_cast<unsigned long long *>(D.um + L.ui[p]), 1ull << k);
+        for (uint32_t p = col_ptr[c]; p < col_ptr[c + 1]; p++) D.da[p] = (uint16_t)(k * n + L.prow[p]);
+        D.ip[L.pinv[k]] = (uint16_t)k;
+        D.q[k] = (uint16_t)c;
+    }
+    wsync();
+}
+
+// A fresh factor's values (in global memory) into the dense array.
+__device__ inline void priv_dense_load(const PrivLane &L, const PrivDense &D, uint32_t tid)
+{
+    const uint32_t n = L.n;
+    if (tid < n) {
+        const uint32_t k = tid;
+        for (uint32_t p = L.lp[k]; p < L.lp[k + 1]; p++) D.F[k * n + L.li[p]] = L.lx[p];
+        for (uint32_t p = L.up[k]; p < L.up[k + 1]; p++) D.F[k * n + L.ui[p]] = L.ux[p];
+        D.F[k * n + k] = L.udiag[k];
+    }
+    wsync();
+}
+
+__device__ inline double lane_value(double v, uint32_t l)
+{
+    const uint64_t b = pl_bits(v);
+    const uint32_t lo = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)b, (int)l);
+    const uint32_t hi = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)(b >> 32), (int)l);
+    return pl_double((uint64_t)hi << 32 | lo);
+}
+
+// The replay (priv_replay's steps and tests in its order); true when a peel
+// test fails. A taken branch costs a lone wavefront about as much as an LDS
+// round trip, so a column has two: U entries run four at a time (the tail on
+// the last column, which has no L rows), and the tests are selects.
+__device__ bool priv_replay_dense(const PrivLane &L, const PrivDense &D, double wide, uint32_t tid)
+{
+    constexpr double kGrowth = 1e-12;
+    constexpr uint32_t kEnt = 4;
+    const uint32_t n = uni(L.n), nnz = uni(L.nnz);
+    const auto F = lptr(D.F);
+    const auto up = lptr(L.up), ui = lptr(L.ui);
+    const auto da = lptr(D.da);
+    const auto ap = gptr(L.ap);
+    const uint32_t row = tid < n ? tid : 0u;
+    const uint64_t lmask = lptr(D.lm)[row], umask = lptr(D.um)[row];
+    const uint32_t fl = gptr(L.flags)[row];   // thread k: the flags of step k
+    for (uint32_t i = tid; i < n * n; i += kWave) F[i] = 0.0;
+    wsync();
+    for (uint32_t p0 = 0; p0 < nnz; p0 += 4 * kWave) {
+        double v[4];
+        uint32_t at[4];
+#pragma unroll
+        for (uint32_t u = 0; u < 4; u++) {
+            const uint32_t p = p0 + u * kWave + tid;
+            at[u] = p < nnz ? da[p] : 0xffffu;
+            v[u] = p < nnz ? ap[p] : 0.0;
+        }
+#pragma unroll
+        for (uint32_t u = 0; u < 4; u++)
+            if (at[u] != 0xffffu) F[at[u]] = v[u];
+    }
+    wsync();
+    uint64_t nonfinite = 0, worst = 0;
+    bool bad = false;
+    const uint64_t scaled_steps = __ballot((fl & kScaledBit) != 0);
+    const uint32_t ups = up[row], upe = up[row + 1];   // thread k: column k's span of ui
+    if (tid < n) {
+        double xn = F[row];
+        for (uint32_t k = 0; k < n; k++) {
+            double x = xn;
+            const uint32_t u0 = (uint32_t)__builtin_amdgcn_readlane((int)ups, (int)k);
+            const uint32_t m = (uint32_t)__builtin_amdgcn_readlane((int)upe, (int)k) - u0;   // at most k
+            const uint32_t e = tid < m ? ui[u0 + tid] : n - 1;
+            xn = F[(k + 1 < n ? k + 1 : k) * n + row];
+            for (uint32_t j = 0; j < m; j += kEnt) {
+                uint32_t i[kEnt];
+                double l[kEnt];
+#pragma unroll
+                for (uint32_t u = 0; u < kEnt; u++) {
+                    // entries past m lie on a thread past m, or past n: none
+                    const uint32_t r = (uint32_t)__builtin_amdgcn_readlane((int)e, (int)(j + u));
+                    i[u] = j + u < m ? r : n - 1;
+                    l[u] = F[i[u] * n + row];
+                }
+#pragma unroll
+                for (uint32_t u = 0; u < kEnt; u++) {
+                    const double t = l[u] * lane_value(x, i[u]);
+                    x = (lmask >> i[u]) & 1u ? x - t : x;
+                }
+            }
+            // the U rows hold their entries, row k the pivot, the L rows
+            // their values before the division
+            const bool in_u = (umask >> k) & 1u, in_l = (lmask >> k) & 1u;
+            const bool scaled = (scaled_steps >> k) & 1u;
+            double d = lane_value(x, k);
+            const bool dead = d == 0 || !(fabs(d) < __builtin_inf());
+            d = dead ? 1.0 : d;
+            const double lv = x / d;
+            const uint64_t vb = dbits(fabs(x)), db = dbits(fabs(d)), lb = dbits(fabs(lv));
+            const bool grown = !(fabs(d) >= kGrowth * bitsd(vb > db ? vb : db));
+            bad = bad | dead | (in_l & !scaled & grown);
+            nonfinite |= in_u ? dbits(x - x) : 0u;
+            nonfinite |= in_l & scaled ? dbits(lv - lv) : 0u;
+            const uint64_t wb = in_l & !scaled ? lb : 0u;
+            worst = wb > worst ? wb : worst;
+            F[k * n + row] = row == k ? d : in_l ? lv : x;
+        }
+    }
+    if (wave_any(nonfinite != 0)) return true;
+    worst = wave_max_u64(worst);
+    return wave_any(bad) || !(bitsd(worst) <= wide);
+}
+
+// dx = -A^-1 rhs from the dense factors (priv_solve's steps in its order);
+// dx in unknown order.
+__device__ void priv_solve_dense(const PrivLane &L, const PrivDense &D, const double *rhs_, double *dx_, uint32_t tid)
+{
+    const uint32_t n = uni(L.n);
+    const auto F = lptr(D.F);
+    const auto rhs = lptr(rhs_);
+    const auto dx = lptr(dx_);
+    const bool mine = tid < n;
+    const uint32_t row = mine ? tid : 0u;
+    const uint64_t lmask = lptr(D.lm)[row], umask = lptr(D.um)[row];
+    const uint32_t qr = lptr(D.q)[row];
+    const double dg = F[row * n + row];
+    double y = -rhs[lptr(D.ip)[row]];
+    double c = F[row];
+#pragma unroll 2
+    for (uint32_t k = 0; k + 1 < n; k++) {
+        const double cn = F[(k + 1) * n + row];
+        const double yk = lane_value(y, k);
+        const double t = c * yk;
+        y = ((lmask >> k) & 1u) & (yk != 0) ? y - t : y;
+        c = cn;
+    }
+    // c is now the last column
+#pragma unroll 2
+    for (uint32_t k = n; k > 0;) {
+        k--;
+        const double cn = F[(k ? k - 1 : 0u) * n + row];
+        const double z = y / dg;
+        const double zk = lane_value(z, k);
+        const double t = c * zk;
+        y = row == k ? zk : ((umask >> k) & 1u) & (zk != 0) ? y - t : y;
+        c = cn;
+    }
+    if (mine) dx[qr] = y;
+}
+
 // Entry points for the lane kernels, called by every thread of the lane's
 // wavefront. lds: the lane's factor-slot area (lds_doubles long); its w is
 // all zero on entry and on return. tail: LDS past the lane's working set
@@ -898,7 +1098,15 @@ __device__ __forceinline__ int priv_factor_at(const PrivLU &P, uint32_t lane, co
     uint32_t *ws = 5 * (uint64_t)L.n <= 2 * (uint64_t)tail_n ? reinterpret_cast<uint32_t *>(tail) : nullptr;
     const int rc = priv_factor_w(L, col_ptr, row_idx, q, 1e-3, ws, tid);
     wsync();
-    if (rc == kPlOk) priv_load(L, col_ptr, q, tail, tail_n, tid);
+    if (rc == kPlOk) {
+        PrivDense D;
+        if (priv_dense(L, tail, tail_n, D)) {
+            priv_dense_build(L, D, col_ptr, q, tid);
+            priv_dense_load(L, D, tid);
+        } else {
+            priv_load(L, col_ptr, q, tail, tail_n, tid);
+        }
+    }
     return rc;
 }
 
@@ -912,6 +1120,13 @@ __device__ __forceinline__ bool priv_replay_at(const PrivLU &P, uint32_t lane, c
                                                uint32_t tail_n, uint32_t tid, bool *resident = nullptr)
 {
     PrivLane L = priv_lane(P, lane, lds, lds_doubles);
+    PrivDense D;
+    if (priv_dense(L, tail, tail_n, D)) {
+        if (resident) *resident = true;
+        const bool failed = priv_replay_dense(L, D, 1.0 / 1e-3, tid);
+        wsync();
+        return failed;
+    }
     const bool res = priv_resident(L, tail, tail_n);
     if (resident) *resident = res;
     const bool failed = res ? priv_replay_res(L, 1e-12, 1.0 / 1e-3, tid)
@@ -935,7 +1150,9 @@ __device__ __forceinline__ void priv_solve_at(const PrivLU &P, uint32_t lane, co
                                               uint32_t tail_n, uint32_t tid)
 {
     PrivLane L = priv_lane(P, lane, lds, lds_doubles);
-    if (priv_resident(L, tail, tail_n)) priv_solve<true>(L, q, rhs, dx, tid);
+    PrivDense D;
+    if (priv_dense(L, tail, tail_n, D)) priv_solve_dense(L, D, rhs, dx, tid);
+    else if (priv_resident(L, tail, tail_n)) priv_solve<true>(L, q, rhs, dx, tid);
     else priv_solve<false>(L, q, rhs, dx, tid);
 }
 
@@ -950,7 +1167,10 @@ __device__ __forceinline__ bool priv_enter(const PrivLU &P, uint32_t lane, const
     PrivLane L = priv_lane(P, lane, lds, lds_doubles);
     for (uint32_t i = tid; i < L.n; i += kWave) L.w[i] = 0.0;
     if (!priv_stage(L, tid, kWave)) return false;
-    if (priv_resident(L, tail, tail_n)) priv_stage_static(L, col_ptr, q, tid);
+    wsync();
+    PrivDense D;
+    if (priv_dense(L, tail, tail_n, D)) priv_dense_build(L, D, col_ptr, q, tid);
+    else if (priv_resident(L, tail, tail_n)) priv_stage_static(L, col_ptr, q, tid);
     return true;
 }
 

@@ -1914,14 +1914,15 @@ u32 device_cu_count();
 // the launch leaves LDS idle (few lanes per CU), room (up to what is idle)
 // past the working set
 // for the lanes' own factor values and the replay's records (room for
-// twice the lead factor's entries), so that their replays and solves run
-// out of LDS; otherwise the working set alone.
-u32 own_lds_bytes(u32 lds, u32 grid, u32 n, u32 nnz_l, u32 nnz_u)
+// twice the lead factor's entries, and for the dense form of lanes of at
+// most 64 unknowns), so that their replays and solves run out of LDS; otherwise the working set alone.
+u32 own_lds_bytes(u32 lds, u32 grid, u32 n, u32 nnz, u32 nnz_l, u32 nnz_u)
 {
     const u32 cu = device_cu_count();
     if (cu == 0 || grid == 0) return lds;
     const size_t per_cu = (grid + cu - 1) / cu;
-    const size_t want = lds + 8 * (2 * (size_t)nnz_l + 4 * (size_t)nnz_u + 3 * (size_t)n + 16);
+    size_t want = lds + 8 * (2 * (size_t)nnz_l + 4 * (size_t)nnz_u + 3 * (size_t)n + 16);
+    if (n <= (u32)esl::kWave) want = std::max(want, lds + 8 * ((size_t)n * n + 2 * n + (nnz + 2 * (size_t)n + 3) / 4));
     const size_t room = std::min<size_t>(65536, 160 * 1024 / per_cu) & ~(size_t)15;
     return (u32)std::max<size_t>(lds, std::min(want, room));
 }
@@ -2969,7 +2970,7 @@ esl_status launch_op(Engine &e, const HostOpArgs &d, u32 grid, hipStream_t s)
         return ESL_FAILED;
     }
     HIPCHK(esl_kernel_attrs(std::max<u32>(lds, 65536)));
-    const u32 lds_run = d.priv.cap ? std::max(lds, own_lds_bytes(lds, grid, e.c.n, e.lead_nl, e.lead_nu)) : lds;
+    const u32 lds_run = d.priv.cap ? std::max(lds, own_lds_bytes(lds, grid, e.c.n, e.c.nnz, e.lead_nl, e.lead_nu)) : lds;
     HIPCHK(esl_launch_op_newton(&d, grid, lds_run, s));
     return ESL_OK;
 }
@@ -3429,7 +3430,7 @@ hipError_t launch_tran(Engine &e, const esl::TranArgs &t, u32 grid, hipStream_t 
         return esl_launch_big(&b, s);
     }
     const u32 lds = tran_lds_bytes(e.c, t.op.tv_cap);
-    const u32 lds_run = t.op.priv.cap ? std::max(lds, own_lds_bytes(lds, grid, e.c.n, e.lead_nl, e.lead_nu)) : lds;
+    const u32 lds_run = t.op.priv.cap ? std::max(lds, own_lds_bytes(lds, grid, e.c.n, e.c.nnz, e.lead_nl, e.lead_nu)) : lds;
     return esl_launch_tran_steps(&t, grid, lds_run, s);
 }
 }  // namespace
@@ -3595,7 +3596,7 @@ esl_status tran_adaptive_rounds(Engine &E, const esl::TranArgs &ta, const esl::P
         {
             const u32 lds = tran_lds_bytes(e->c, cap);
             const u32 lds_run = t.op.priv.cap
-                                    ? std::max(lds, own_lds_bytes(lds, (u32)run.size(), n, e->lead_nl, e->lead_nu))
+                                    ? std::max(lds, own_lds_bytes(lds, (u32)run.size(), n, e->c.nnz, e->lead_nl, e->lead_nu))
                                     : lds;
             HIPCHK(esl_launch_tran_steps(&t, (u32)run.size(), lds_run, s));
         }
@@ -3936,7 +3937,7 @@ esl_status tran_run(esl_engine *h, const double *values, size_t count, const esl
             for (u32 b = b0; b < B; b++) {
                 esl::TranArgs t = block_args(b, cap, 0);
                 t.op.priv = own;
-                const u32 lds_run = std::max(lds, own_lds_bytes(lds, (u32)again.size(), n, e->lead_nl, e->lead_nu));
+                const u32 lds_run = std::max(lds, own_lds_bytes(lds, (u32)again.size(), n, e->c.nnz, e->lead_nl, e->lead_nu));
                 HIPCHK(esl_launch_tran_steps(&t, (u32)again.size(), lds_run, s));
             }
             HIPCHK(hipEventRecord(e->ev1, s));
