@@ -199,16 +199,19 @@ __device__ inline void eval_chunk(const DeckProg &dp, const Chunk &ch, const dou
     }
 }
 
+// The lane's threads are tid = 0 .. kStep - 1: its wavefront, or the team of
+// a big lane (whose callers add a workgroup barrier).
 // Limiting state of a start at x (no junction seeds): the previous terminal
 // voltages are x's own.
 // keep_von: MOS fetlim thresholds stay the von of the last evaluation (an
 // accepted transient step: the predictor's limit pass runs against the
 // accepted point with the von its last load stored, mos1.va:293-297).
+template <uint32_t kStep = kWave>
 __device__ inline void seed_lim_at(const DeckProg &dp, const double *live, const double *x, double *lim,
                                    uint32_t tid, bool keep_von = false)
 {
     const uint32_t nm = dp.n_mos;
-    for (uint32_t j = tid; j < nm; j += kWave) {
+    for (uint32_t j = tid; j < nm; j += kStep) {
         const Mos m = mos_load(dp, j, live);
         const uint32_t *t4 = dp.m_t + 4 * j;
         const double xd = x[t4[0]], xgg = x[t4[1]], xs = x[t4[2]], xb = x[t4[3]];
@@ -217,8 +220,8 @@ __device__ inline void seed_lim_at(const DeckProg &dp, const double *live, const
         lim[2 * nm + j] = m.tp * (xb - xs);
         if (!keep_von) lim[3 * nm + j] = 0.0;
     }
-    for (uint32_t j = tid; j < dp.n_dio; j += kWave) lim[4 * nm + j] = x[dp.d_t[2 * j]] - x[dp.d_t[2 * j + 1]];
-    for (uint32_t j = tid; j < dp.n_bjt; j += kWave) {
+    for (uint32_t j = tid; j < dp.n_dio; j += kStep) lim[4 * nm + j] = x[dp.d_t[2 * j]] - x[dp.d_t[2 * j + 1]];
+    for (uint32_t j = tid; j < dp.n_bjt; j += kStep) {
         const uint32_t *t4 = dp.q_t + 4 * j;
         const double tp = dp.q_par[QF_TYPE * dp.n_bjt + j];
         lim[lim_bjt(dp) + 2 * j] = tp * (x[t4[1]] - x[t4[2]]);
@@ -229,21 +232,21 @@ __device__ inline void seed_lim_at(const DeckProg &dp, const double *live, const
 // One limit pass of a lane's devices at x against its limiting state (MOS1
 // fetlim/limvds/pnjlim, diode and BJT pnjlim, eval.zig limitRange): the
 // thread's part; true when any of its devices moved.
-template <typename X>
+template <uint32_t kStep = kWave, typename X>
 __device__ inline bool limit_pass(const DeckProg &dp, const double *live, X x, double *lim, uint32_t tid)
 {
     const uint32_t nm = dp.n_mos;
     bool limited = false;
-    for (uint32_t j = tid; j < nm; j += kWave) {
+    for (uint32_t j = tid; j < nm; j += kStep) {
         const Mos m = mos_load(dp, j, live);
         const uint32_t *t4 = dp.m_t + 4 * j;
         limited |= mos_limit(m, x[t4[0]], x[t4[1]], x[t4[2]], x[t4[3]], lim + j, nm);
     }
-    for (uint32_t j = tid; j < dp.n_dio; j += kWave) {
+    for (uint32_t j = tid; j < dp.n_dio; j += kStep) {
         const Dio d = dio_load(dp, j, live);
         limited |= dio_limit_v(d, x[dp.d_t[2 * j]], x[dp.d_t[2 * j + 1]], lim[4 * nm + j]);
     }
-    for (uint32_t j = tid; j < dp.n_bjt; j += kWave) {
+    for (uint32_t j = tid; j < dp.n_bjt; j += kStep) {
         const Bjt b = bjt_load(dp, j, live);
         const uint32_t *t4 = dp.q_t + 4 * j;
         double *ql = lim + lim_bjt(dp) + 2 * j;
@@ -256,39 +259,42 @@ __device__ inline bool limit_pass(const DeckProg &dp, const double *live, X x, d
 // iterate) and, except on a resume, its limiting state.
 // A cold start: x = 0 and the limiting state's cold seeds (the initial
 // junction and threshold voltages).
+template <uint32_t kStep = kWave>
 __device__ inline void lane_cold(const DeckProg &dp, const double *live, double *x, double *lim, uint32_t tid)
 {
     const uint32_t n = dp.n, nm = dp.n_mos;
-    for (uint32_t i = tid; i < n; i += kWave) x[i] = 0.0;
-    for (uint32_t j = tid; j < nm; j += kWave) {
+    for (uint32_t i = tid; i < n; i += kStep) x[i] = 0.0;
+    for (uint32_t j = tid; j < nm; j += kStep) {
         const Mos m = mos_load(dp, j, live);
         lim[j] = m.tp * m.vbit + m.gammax * sqrt(m.phit);
         lim[nm + j] = 0.0;
         lim[2 * nm + j] = -1.0;
         lim[3 * nm + j] = 0.0;
     }
-    for (uint32_t j = tid; j < dp.n_dio; j += kWave) lim[4 * nm + j] = dio_load(dp, j, live).vcrit;
-    for (uint32_t j = tid; j < dp.n_bjt; j += kWave) {
+    for (uint32_t j = tid; j < dp.n_dio; j += kStep) lim[4 * nm + j] = dio_load(dp, j, live).vcrit;
+    for (uint32_t j = tid; j < dp.n_bjt; j += kStep) {
         lim[lim_bjt(dp) + 2 * j] = bjt_load(dp, j, live).vcrit;
         lim[lim_bjt(dp) + 2 * j + 1] = 0.0;
     }
     wsync();
 }
 
+template <uint32_t kStep = kWave>
 __device__ inline void lane_init(const OpArgs &a, uint32_t lane, const double *live, double *x, double *lim,
                                  uint32_t tid)
 {
     const DeckProg &dp = a.dp;
     const uint32_t n = dp.n;
     if (a.mode == 0) {
-        lane_cold(dp, live, x, lim, tid);
+        lane_cold<kStep>(dp, live, x, lim, tid);
         return;
     }
     const double *xg = a.x + (size_t)lane * n;
-    for (uint32_t i = tid; i < n; i += kWave) x[i] = xg[i];
+    for (uint32_t i = tid; i < n; i += kStep) x[i] = xg[i];
     wsync();
+    if (kStep != kWave) __syncthreads();
     if (a.mode == 2) return;
-    seed_lim_at(dp, live, x, lim, tid);
+    seed_lim_at<kStep>(dp, live, x, lim, tid);
     wsync();
 }
 

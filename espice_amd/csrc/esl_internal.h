@@ -197,15 +197,26 @@ __host__ __device__ inline uint32_t tran_doubles(uint32_t tv_cap, uint32_t n, ui
     return tv_cap + tran_y_block(n, nw) + 3 * n + n_cslot;
 }
 
+// A lane beyond a workgroup's LDS (a big lane) runs on a team of kTeam
+// wavefronts, one workgroup; its row programs are kTeamThreads wide.
+constexpr uint32_t kTeam = 8;
+constexpr uint32_t kTeamThreads = kTeam * kWave;
+
 // One block of a big tape's replay: a run of consecutive ops of the row
 // program order whose slots fit LDS. The block gathers its m slots
 // (blk_slots[slot_off ...]) into LDS positions 0..m-1, runs its rows (words
-// from row row0 of blk_words, indices into [m slots | 64 pads]), then
-// scatters the first w positions (the slots it writes) back.
+// [row][kTeamThreads] from row row0 of blk_words, indices into [m slots |
+// kTeamThreads pads]), then scatters the first w positions (the slots it
+// writes) back.
 struct BigBlock {
     uint32_t slot_off, m, w, rows;   // rows: a multiple of kRing
     uint32_t row0, pad0, pad1, pad2;
 };
+
+// A word of a big tape's solve program: x = d | c << 16 (solve vector
+// indices, pads from n on), y = factor slot | kSolDiv on rows of divisions:
+// y[d] = y[c] != 0 ? y[d] - tv[slot] * y[c] : y[d], or y[d] = y[d] / tv[slot].
+constexpr uint32_t kSolDiv = 0x80000000u;
 
 struct TapeProg {
     uint32_t n_tv, n_u, n_l, lx0;   // tv = [U | diag | L | discard | void extras | 64 pads]
@@ -238,15 +249,15 @@ struct TapeProg {
     const uint32_t *diag_tv;    // [n] tv slot of each row's diagonal
     const uint32_t *li;         // [n_l] row (pivot step) of each L entry
     // big tapes (lanes whose slots live in HBM): the replay in blocks of at
-    // most blk_m slots; the solves in chunks of columns, each chunk's L
-    // (forward) or U (backward) entries at most sol_cap: columns
-    // fch[c] .. fch[c + 1] and bch[c] .. bch[c + 1]
-    uint32_t n_blk, blk_m, n_fch, n_bch;
-    uint32_t sol_cap, pad5, pad6, pad7;
+    // most blk_m slots, and the solves as sol_rows rows of words
+    // [row][kTeamThreads] (kRing idle rows follow both programs)
+    uint32_t n_blk, blk_m, sol_rows, pad5;
+    uint32_t pad6, pad7, pad8, pad9;
     const BigBlock *blk;        // [n_blk]
     const uint32_t *blk_slots;  // tv slots of each block's LDS positions
-    const uint2_t *blk_words;   // rows of all blocks, [row][64]
-    const uint32_t *fch, *bch;  // [n_fch + 1], [n_bch + 1]
+    const uint2_t *blk_words;   // rows of all blocks, [row][kTeamThreads]
+    const uint2_t *sol_w;
+    const uint2_t *sol_pad;
     // chain segments of the refactor and solve programs: (word offset into
     // the terms, blocks) each, and their terms
     const uint2_t *rseg, *sseg;
@@ -480,37 +491,41 @@ struct LptArgs {
 };
 
 // Arguments of the kernel for lanes whose working set is beyond a
-// workgroup's LDS (big_lanes): one wavefront per lane, workgroup g runs lane
-// ta.op.lane_ids[g], .op (tran == 0: the OpArgs of ta, modes 0-2, dump) or
-// transient steps (tran == 1); a workgroup holds `waves` lanes, one per
-// wavefront. The lane's vectors and factor slots live in HBM at
-// ws + g * ws_stride: tv [tv_cap], then rhs, x, xold, sdiag, q [n
+// workgroup's LDS (big_lanes): workgroup g, a team of kTeam wavefronts, runs
+// lane ta.op.lane_ids[g], .op (tran == 0: the OpArgs of ta, modes 0-2, dump)
+// or transient steps (tran == 1). The lane's vectors and factor slots live
+// in HBM at ws + g * ws_stride: tv [tv_cap], then rhs, x, xold, sdiag, q [n
 // each] and the charge-Jacobian cells [n_cslot]; LDS (lds doubles) holds
-// the staging cells, a block of the replay, or the solve vector and a chunk
-// of factor entries.
-constexpr uint32_t kBigWaves = 4;   // most lanes (wavefronts) per big-lane workgroup
+// the wavefronts' staging cells, a block of the replay, or the solve vector,
+// and last the team's reduction scratch.
 struct BigArgs {
     TranArgs ta;
     double *ws;
     uint64_t ws_stride;
     uint32_t N, tran;
-    uint32_t tv_cap, lds;       // lds: doubles of one lane's LDS area
-    uint32_t waves, pad;        // lanes per workgroup (1..kBigWaves)
+    uint32_t tv_cap, lds;
+    // the deck's reduce tasks by rounds of kTeam chunks: targets
+    // rt_target[rt_round[r] .. rt_round[r + 1]), their cells from
+    // rt_cell[...] on in instance order, cell indices chunk in the round *
+    // kStageDoubles + staging index
+    uint32_t n_rounds, pad;
+    const uint32_t *rt_round, *rt_target, *rt_cell;
+    const uint16_t *rt_cells;
 };
 __host__ __device__ inline size_t big_stride(uint32_t tv_cap, uint32_t n, uint32_t n_cslot)
 {
     const size_t d = (size_t)tv_cap + 5 * (size_t)n + n_cslot;
     return (d + 15) / 16 * 16;   // 128-byte aligned lanes
 }
-// the LDS of a big lane: the staging cells, a replay block of blk_m slots
-// and 64 pads, or the solve vector with a chunk of sol_cap entries and
-// their indices
-__host__ __device__ inline uint32_t big_lds_doubles(uint32_t n, uint32_t blk_m, uint32_t sol_cap)
+// the LDS of a big lane: the staging cells of kTeam chunks, a replay block
+// of blk_m slots and its pads, or the solve vector and its pads; then the
+// reduction scratch
+constexpr uint32_t kTeamScratch = 2 * kTeam;
+__host__ __device__ inline uint32_t big_lds_doubles(uint32_t n, uint32_t blk_m)
 {
-    uint32_t d = blk_m + kWave;
-    const uint32_t s = n + sol_cap + (sol_cap + 1) / 2;
-    d = s > d ? s : d;
-    return kStageDoubles > d ? kStageDoubles : d;
+    uint32_t d = blk_m > n ? blk_m : n;
+    d += kTeamThreads;
+    return (kTeam * kStageDoubles > d ? kTeam * kStageDoubles : d) + kTeamScratch;
 }
 
 // Arguments of the LU-only replay (tape_replay).

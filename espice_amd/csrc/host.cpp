@@ -451,6 +451,44 @@ class OpGraph {
     u32 last(u32 slot) const { return last_[slot]; }
     size_t size() const { return ops_.size(); }
 
+    // rows of at most `width` independent ops of one kind, in an order that
+    // keeps every dependency (a big lane's programs: no chains)
+    void rows_of(u32 width, vector<vector<u32>> &rows) const
+    {
+        const size_t m = ops_.size();
+        rows.clear();
+        vector<u32> height(m, 0), deg = indeg_;
+        for (size_t v = m; v > 0;) {   // ops only depend on earlier ones
+            v--;
+            u32 best = 0;
+            for (u32 x : succ_[v]) best = std::max(best, height[x]);
+            height[v] = best + 1;
+        }
+        auto cmp = [&](u32 a, u32 b) { return height[a] != height[b] ? height[a] < height[b] : a > b; };
+        vector<std::priority_queue<u32, vector<u32>, decltype(cmp)>> ready;
+        for (u32 k = 0; k < esl::R_KINDS; k++) ready.emplace_back(cmp);
+        for (size_t v = 0; v < m; v++)
+            if (deg[v] == 0) ready[ops_[v].kind].push((u32)v);
+        for (size_t done = 0; done < m;) {
+            u32 kind = esl::R_KINDS;
+            for (u32 k = 1; k < esl::R_CHAIN; k++) {
+                if (ready[k].empty()) continue;
+                if (kind == esl::R_KINDS || cmp(ready[kind].top(), ready[k].top())) kind = k;
+            }
+            vector<u32> row;
+            while (!ready[kind].empty() && row.size() < (size_t)width) {
+                row.push_back(ready[kind].top());
+                ready[kind].pop();
+            }
+            done += row.size();
+            for (u32 v : row)
+                for (u32 x : succ_[v])
+                    if (--deg[x] == 0) ready[ops_[x].kind].push(x);
+            rows.push_back(std::move(row));
+        }
+    }
+    const SchedOp &op(u32 i) const { return ops_[i]; }
+
     // pad_base: 64 private pad slots, one per thread
     void schedule(u32 pad_base, RowProgram &out, u32 min_chain = 0) const
     {
@@ -677,8 +715,8 @@ struct TapeHostProg {
     // chunks instead of whole-tape row programs and reduce streams
     bool big = false;
     vector<esl::BigBlock> blk;
-    vector<u32> blk_slots, fch, bch;
-    vector<esl::uint2_t> blk_words;
+    vector<u32> blk_slots;
+    vector<esl::uint2_t> blk_words, sol_w;
     DevBuf buf;
 };
 
@@ -877,36 +915,33 @@ void build_row_programs(const HostTape &t, TapeHostProg &o, u32 min_chain = kMin
     }
 }
 
-// The replay of a big tape (lanes whose factor slots live in HBM): the ops
-// of the refactor row program in the order build_row_programs adds them
-// (column by column; in a column each target's multiply-subtracts in the
-// order of the column replay, an L target then its pivot division), cut
-// into runs that touch at most block_slots slots (by default as many as the
-// LDS the solves need anyway holds, at least kBigBlockSlots); each run is
-// scheduled into rows of its own over LDS positions (the slots it writes
-// first), padded to a multiple of kRing. The runs' rows are stored back to
-// back (a run's prefetches past its end load the next run's words), kRing
-// idle rows after the last. The solves run in chunks of columns of at most
-// sol_cap entries. False when a flop's target lies outside its column.
-constexpr u32 kBigBlockSlots = 4032;
-constexpr u32 kBigSlotLimit = 65536 - esl::kWave;   // 16-bit row-word indices
-constexpr u32 kBigSolveCap = 512;
+// The programs of a big tape (lanes whose factor slots live in HBM), rows of
+// kTeamThreads words. The replay: the ops of the refactor row program in
+// the order build_row_programs adds them (column by column; in a column each
+// target's multiply-subtracts in the order of the column replay, an L target
+// then its pivot division), cut into runs that touch at most block_slots
+// slots; each run is scheduled into rows of its own over LDS positions (the
+// slots it writes first), padded to a multiple of kRing. The runs' rows are
+// stored back to back (a run's prefetches past its end load the next run's
+// words), kRing idle rows after the last. A block as large as a workgroup's
+// LDS leaves the scheduler more columns at once: the 64x64 mesh (2.84 M ops)
+// takes 592 blocks and 87,000 rows of 64 at 4,032 slots, 43 blocks and
+// 10,700 rows of 512 at 18,000. The solves: one program over the solve
+// vector, each factor entry read from its slot. False when a flop's target
+// lies outside its column.
+constexpr u32 kBigBlockSlots = 18944;
+constexpr u32 kBigSlotLimit = 65536 - esl::kTeamThreads;   // 16-bit row-word indices
 
-bool build_big_program(const HostTape &t, TapeHostProg &o, u32 block_slots = 0)
+bool build_big_program(const HostTape &t, TapeHostProg &o, u32 block_slots = kBigBlockSlots,
+                       u32 W = esl::kTeamThreads)
 {
     const u32 n = t.n, nu = t.nnz_u;
-    // solve chunks: forward over L entries, backward over U entries and pivots
-    u32 cap = kBigSolveCap;
-    for (u32 k = 0; k < n; k++) cap = std::max({cap, t.lp[k + 1] - t.lp[k], t.up[k + 1] - t.up[k] + 1});
-    if (block_slots == 0) {
-        const uint64_t solve = (uint64_t)n + cap + (cap + 1) / 2;
-        block_slots = (u32)std::min<uint64_t>(kBigSlotLimit, std::max<uint64_t>(kBigBlockSlots, solve - esl::kWave));
-    }
     const esl::TapeProg &P = o.prog;
     const u32 lx0 = P.lx0, discard = P.discard;
     o.blk.clear();
     o.blk_slots.clear();
     o.blk_words.clear();
+    o.sol_w.clear();
     vector<SchedOp> run;                  // the current block's ops (tv slots)
     vector<u32> stamp(P.n_tv, NONE);      // block id that touched a slot
     vector<u32> local(P.n_tv, NONE);
@@ -929,14 +964,26 @@ bool build_big_program(const HostTape &t, TapeHostProg &o, u32 block_slots = 0)
                     o.blk_slots.push_back(s);
                 }
         b.m = m;
-        OpGraph g(m + esl::kWave);
+        OpGraph g(m);
         for (const SchedOp &op : run) g.add(local[op.d], local[op.b], local[op.c], op.kind, op.flags);
-        RowProgram rp;
-        g.schedule(m, rp);
-        b.rows = rp.rows;
+        vector<vector<u32>> rows;
+        g.rows_of(W, rows);
+        b.rows = ((u32)rows.size() + esl::kRing - 1) / esl::kRing * esl::kRing;
         b.row0 = rows_total;
-        rows_total += rp.rows;
-        o.blk_words.insert(o.blk_words.end(), rp.words.begin(), rp.words.begin() + (size_t)rp.rows * esl::kWave);
+        rows_total += b.rows;
+        for (u32 r = 0; r < b.rows; r++) {
+            const u32 cnt = r < rows.size() ? (u32)rows[r].size() : 0u;
+            const u32 kind = cnt ? g.op(rows[r][0]).kind : (u32)esl::R_NOP;
+            for (u32 th = 0; th < W; th++) {
+                const u32 pad = m + th;
+                esl::uint2_t w{pad | (pad << 16), pad | (kind << 16)};
+                if (th < cnt) {
+                    const SchedOp &op = g.op(rows[r][th]);
+                    w = esl::uint2_t{op.d | (op.b << 16), op.c | (op.kind << 16) | (op.flags << 20)};
+                }
+                o.blk_words.push_back(w);
+            }
+        }
         for (u32 k = b.slot_off; k < (u32)o.blk_slots.size(); k++) local[o.blk_slots[k]] = NONE;
         o.blk.push_back(b);
         run.clear();
@@ -995,32 +1042,53 @@ bool build_big_program(const HostTape &t, TapeHostProg &o, u32 block_slots = 0)
     close();
     // idle rows after the last block: the last rows' prefetches stay inside
     // (a block's prefetches past its end read the next block's words)
-    o.blk_words.resize(o.blk_words.size() + (size_t)esl::kRing * esl::kWave, esl::uint2_t{0, 0});
-    o.fch.assign(1, 0);
-    o.bch.assign(1, 0);
-    u32 cf = 0, cb = 0;
-    for (u32 k = 0; k < n; k++) {
-        const u32 lf = t.lp[k + 1] - t.lp[k], lb = t.up[k + 1] - t.up[k] + 1;
-        if (cf + lf > cap) {
-            o.fch.push_back(k);
-            cf = 0;
+    o.blk_words.resize(o.blk_words.size() + (size_t)esl::kRing * W, esl::uint2_t{0, 0});
+    // the solves (lane_kernels.zig:123-143 by rows), as build_row_programs
+    // orders them: forward terms in ascending k, then backward terms in
+    // descending k and the division
+    {
+        vector<vector<std::pair<u32, u32>>> lrow(n), urow(n);
+        for (u32 k = 0; k < n; k++) {
+            for (u32 qq = t.lp[k]; qq < t.lp[k + 1]; qq++) lrow[t.li[qq]].push_back({k, lx0 + qq});
+            for (u32 p = t.up[k]; p < t.up[k + 1]; p++) urow[t.ui[p]].push_back({k, p});
         }
-        if (cb + lb > cap) {
-            o.bch.push_back(k);
-            cb = 0;
+        OpGraph g(n);
+        vector<vector<u32>> readers(n);
+        for (u32 r = 0; r < n; r++)
+            for (auto &e : lrow[r]) readers[e.first].push_back(g.add(r, e.first, e.first, esl::R_MACZ, e.second));
+        for (u32 i = n; i > 0;) {
+            i--;
+            auto &v = urow[i];
+            std::sort(v.begin(), v.end(), [](auto &a, auto &b) { return a.first > b.first; });
+            bool first = true;
+            for (auto &e : v) {
+                g.add(i, e.first, e.first, esl::R_MACZ, e.second, first ? readers[i] : vector<u32>{});
+                first = false;
+            }
+            g.add(i, i, i, esl::R_DIV, nu + i, first ? readers[i] : vector<u32>{});
         }
-        cf += lf;
-        cb += lb;
+        vector<vector<u32>> rows;
+        g.rows_of(W, rows);
+        const u32 total = ((u32)rows.size() + esl::kRing - 1) / esl::kRing * esl::kRing;
+        for (u32 r = 0; r < total + esl::kRing; r++) {
+            const u32 cnt = r < rows.size() ? (u32)rows[r].size() : 0u;
+            const u32 div = cnt && g.op(rows[r][0]).kind == esl::R_DIV ? esl::kSolDiv : 0u;
+            for (u32 th = 0; th < W; th++) {
+                const u32 pad = n + th;
+                esl::uint2_t w{pad | (pad << 16), div};
+                if (th < cnt) {
+                    const SchedOp &op = g.op(rows[r][th]);
+                    w = esl::uint2_t{op.d | (op.c << 16), op.flags | div};
+                }
+                o.sol_w.push_back(w);
+            }
+        }
+        o.prog.sol_rows = total;
     }
-    o.fch.push_back(n);
-    o.bch.push_back(n);
     esl::TapeProg &Q = o.prog;
     Q.n_blk = (u32)o.blk.size();
     Q.blk_m = 0;
     for (auto &b : o.blk) Q.blk_m = std::max(Q.blk_m, b.m);
-    Q.n_fch = (u32)o.fch.size() - 1;
-    Q.n_bch = (u32)o.bch.size() - 1;
-    Q.sol_cap = cap;
     return true;
 }
 
@@ -1042,7 +1110,7 @@ hipError_t upload_tape_prog(TapeHostProg &o)
     f.push_back(pk.add(o.red_off)); f.push_back(pk.add(o.red_len)); f.push_back(pk.add(o.diag_tv));
     f.push_back(pk.add(o.li));
     f.push_back(pk.add(o.blk)); f.push_back(pk.add(o.blk_slots)); f.push_back(pk.add(o.blk_words));
-    f.push_back(pk.add(o.fch)); f.push_back(pk.add(o.bch));
+    f.push_back(pk.add(o.sol_w));
     f.push_back(pk.add(o.rch.seg)); f.push_back(pk.add(o.sch.seg));
     f.push_back(pk.add(o.rch.cw)); f.push_back(pk.add(o.sch.cw));
     f.push_back(pk.add(o.rsrc));
@@ -1076,8 +1144,7 @@ hipError_t upload_tape_prog(TapeHostProg &o)
     T.blk = reinterpret_cast<const esl::BigBlock *>(P(i++));
     T.blk_slots = P(i++);
     T.blk_words = reinterpret_cast<const esl::uint2_t *>(P(i++));
-    T.fch = P(i++);
-    T.bch = P(i++);
+    T.sol_w = reinterpret_cast<const esl::uint2_t *>(P(i++));
     T.rseg = reinterpret_cast<const esl::uint2_t *>(P(i++));
     T.sseg = reinterpret_cast<const esl::uint2_t *>(P(i++));
     T.rcw = P(i++);
@@ -1171,6 +1238,8 @@ struct Compiled {
     // deck program host arrays
     vector<esl::Chunk> chunks;
     vector<u32> task_target, task_cell;
+    vector<u32> rt_round, rt_target, rt_cell;   // the tasks of rounds of kTeam chunks
+    vector<uint16_t> rt_cells;
     vector<uint16_t> cells;
     vector<u32> r_t, v_t, i_t, m_t;
     vector<double> r_val, v_val, i_val, m_par;
@@ -1677,6 +1746,30 @@ bool compile_deck(const esl_deck *d, Compiled &c, std::string &err)
     }
     c.task_cell.push_back((u32)c.cells.size());
     c.chunks.push_back(esl::Chunk{0, 0, 0, (u32)c.task_target.size()});
+    // rounds of kTeam chunks: each target's cells in chunk order
+    const u32 nch = (u32)c.chunks.size() - 1;
+    for (u32 c0 = 0; c0 < nch; c0 += esl::kTeam) {
+        c.rt_round.push_back((u32)c.rt_target.size());
+        std::map<u32, u32> at;   // target -> position in `lists`
+        vector<std::pair<u32, vector<u32>>> lists;
+        for (u32 k = c0; k < std::min(nch, c0 + esl::kTeam); k++)
+            for (u32 tk = c.chunks[k].task_begin; tk < c.chunks[k + 1].task_begin; tk++) {
+                auto it = at.emplace(c.task_target[tk], (u32)lists.size());
+                if (it.second) lists.push_back({c.task_target[tk], {}});
+                for (u32 cc = c.task_cell[tk]; cc < c.task_cell[tk + 1]; cc++)
+                    lists[it.first->second].second.push_back((k - c0) * esl::kStageDoubles + c.cells[cc]);
+            }
+        // threads take the lists in turn: the longest first
+        std::stable_sort(lists.begin(), lists.end(),
+                         [](auto &a, auto &b) { return a.second.size() > b.second.size(); });
+        for (auto &l : lists) {
+            c.rt_target.push_back(l.first);
+            c.rt_cell.push_back((u32)c.rt_cells.size());
+            for (u32 v : l.second) c.rt_cells.push_back((uint16_t)v);
+        }
+    }
+    c.rt_round.push_back((u32)c.rt_target.size());
+    c.rt_cell.push_back((u32)c.rt_cells.size());
     return true;
 }
 
@@ -1686,6 +1779,10 @@ struct Engine {
     Compiled c;
     DevBuf deck_buf;
     esl::DeckProg dp{};
+    // the reduce tasks by rounds, in deck_buf (BigArgs)
+    u32 n_rounds = 0;
+    const u32 *rt_round = nullptr, *rt_target = nullptr, *rt_cell = nullptr;
+    const uint16_t *rt_cells = nullptr;
     vector<TapeHostProg *> tapes;
     std::map<vector<u32>, u32> tape_index;
     DevBuf tape_table;
@@ -1715,8 +1812,8 @@ struct Engine {
     bool profiling = false;
     vector<unsigned long long> prof_host;
     u32 lds_max = 0;
-    // lanes beyond a workgroup's LDS: every launch runs one thread per lane
-    // with its working set in the workspace bigws (lane-major)
+    // lanes beyond a workgroup's LDS: every launch runs one workgroup per lane
+    // with its working set in the workspace bigws
     bool big = false;
     u32 lds_limit = 0;   // the device's LDS per workgroup
     DevBuf bigws;
@@ -1737,7 +1834,8 @@ hipError_t upload_deck(Engine &e)
     Compiled &c = e.c;
     Packer pk;
     size_t o_chunks = pk.add(c.chunks), o_tt = pk.add(c.task_target), o_tc = pk.add(c.task_cell),
-           o_cells = pk.add(c.cells), o_diag = pk.add(c.diag), o_cur = pk.add(c.current_row),
+           o_rtr = pk.add(c.rt_round), o_rtt = pk.add(c.rt_target), o_rtc = pk.add(c.rt_cell),
+           o_rts = pk.add(c.rt_cells), o_cells = pk.add(c.cells), o_diag = pk.add(c.diag), o_cur = pk.add(c.current_row),
            o_rt = pk.add(c.r_t), o_rv = pk.add(c.r_val), o_rb = pk.add(c.r_bind), o_vt = pk.add(c.v_t),
            o_vv = pk.add(c.v_val), o_vb = pk.add(c.v_bind), o_it = pk.add(c.i_t), o_iv = pk.add(c.i_val),
            o_ib = pk.add(c.i_bind), o_mt = pk.add(c.m_t), o_mp = pk.add(c.m_par), o_mbv = pk.add(c.m_bind_vto),
@@ -1802,6 +1900,11 @@ hipError_t upload_deck(Engine &e)
     dp.chunks = reinterpret_cast<const esl::Chunk *>(b + o_chunks);
     dp.task_target = reinterpret_cast<const u32 *>(b + o_tt);
     dp.task_cell = reinterpret_cast<const u32 *>(b + o_tc);
+    e.n_rounds = (u32)c.rt_round.size() - 1;
+    e.rt_round = reinterpret_cast<const u32 *>(b + o_rtr);
+    e.rt_target = reinterpret_cast<const u32 *>(b + o_rtt);
+    e.rt_cell = reinterpret_cast<const u32 *>(b + o_rtc);
+    e.rt_cells = reinterpret_cast<const uint16_t *>(b + o_rts);
     dp.cells = reinterpret_cast<const uint16_t *>(b + o_cells);
     dp.diag_slot = reinterpret_cast<const u32 *>(b + o_diag);
     dp.current_row = reinterpret_cast<const uint8_t *>(b + o_cur);
@@ -2045,24 +2148,24 @@ void build_reduce_streams(const Compiled &c, TapeHostProg &o)
 // Every index a kernel reads is checked on the host before the first launch,
 // so a malformed program is an error here rather than a GPU memory fault.
 
-// A big tape's blocks and solve chunks.
-bool validate_big(const TapeHostProg &o, u32 n)
+// A big tape's blocks and solve program.
+bool validate_big(const TapeHostProg &o, u32 n, u32 W = esl::kTeamThreads)
 {
     const esl::TapeProg &P = o.prog;
-    if (P.n_blk != o.blk.size() || o.blk_words.size() % esl::kWave) return false;
-    const size_t total_rows = o.blk_words.size() / esl::kWave;
+    if (P.n_blk != o.blk.size() || o.blk_words.size() % W || n > kBigSlotLimit) return false;
+    const size_t total_rows = o.blk_words.size() / W;
     u32 bm = 0;
     for (const esl::BigBlock &b : o.blk) {
         if (b.m == 0 || b.w == 0 || b.w > b.m || b.m > kBigSlotLimit) return false;
         if ((size_t)b.slot_off + b.m > o.blk_slots.size()) return false;
         if (b.rows == 0 || b.rows % esl::kRing || (size_t)b.row0 + b.rows + esl::kRing > total_rows) return false;
         bm = std::max(bm, b.m);
-        const u32 lim = b.m + esl::kWave;
+        const u32 lim = b.m + W;
         for (size_t r = b.row0; r < (size_t)b.row0 + b.rows; r++) {
-            const u32 kind = esl::row_kind(o.blk_words[r * esl::kWave].y);
+            const u32 kind = esl::row_kind(o.blk_words[r * W].y);
             if (kind >= esl::R_KINDS || kind == esl::R_MACZ || kind == esl::R_CHAIN) return false;
-            for (u32 t = 0; t < (u32)esl::kWave; t++) {
-                const esl::uint2_t w = o.blk_words[r * esl::kWave + t];
+            for (u32 t = 0; t < W; t++) {
+                const esl::uint2_t w = o.blk_words[r * W + t];
                 if (esl::row_kind(w.y) != kind || (w.y >> 22) != 0) return false;
                 const u32 d = w.x & 0xffff, bb = w.x >> 16, c = w.y & 0xffff;
                 if (d >= lim || bb >= lim || c >= lim) return false;
@@ -2071,17 +2174,13 @@ bool validate_big(const TapeHostProg &o, u32 n)
     }
     if (bm != P.blk_m) return false;
     for (u32 v : o.blk_slots) if (v >= P.n_tv) return false;
-    auto chunks_ok = [&](const vector<u32> &ch, u32 count, bool fwd) {
-        if (ch.size() != (size_t)count + 1 || ch.front() != 0 || ch.back() != n) return false;
-        for (u32 c = 0; c < count; c++) {
-            if (ch[c] >= ch[c + 1]) return false;
-            size_t e = 0;
-            for (u32 k = ch[c]; k < ch[c + 1]; k++) e += fwd ? o.lp[k + 1] - o.lp[k] : o.up[k + 1] - o.up[k] + 1;
-            if (e > P.sol_cap) return false;
-        }
-        return true;
-    };
-    return chunks_ok(o.fch, P.n_fch, true) && chunks_ok(o.bch, P.n_bch, false);
+    if (P.sol_rows % esl::kRing || o.sol_w.size() != ((size_t)P.sol_rows + esl::kRing) * W) return false;
+    for (size_t k = 0; k < o.sol_w.size(); k++) {
+        const esl::uint2_t w = o.sol_w[k];
+        if ((w.x & 0xffff) >= n + W || (w.x >> 16) >= n + W || (w.y & ~esl::kSolDiv) >= P.n_tv) return false;
+        if ((w.y & esl::kSolDiv) != (o.sol_w[k - k % W].y & esl::kSolDiv)) return false;
+    }
+    return true;
 }
 bool validate_tape(const TapeHostProg &o, u32 n, u32 nnz)
 {
@@ -2263,6 +2362,10 @@ bool validate_deck(const Compiled &c)
     }
     for (u32 v : c.cslot_pat) if (v >= nnz) return false;
     for (u32 v : c.cells) if (v >= (u32)(esl::kWave * esl::kStageEntries)) return false;
+    if (c.rt_round.empty() || c.rt_round.front() != 0 || c.rt_round.back() != c.rt_target.size()) return false;
+    if ((c.rt_round.size() - 1) * esl::kTeam < c.chunks.size() - 1) return false;
+    if (c.rt_cell.size() != c.rt_target.size() + 1 || c.rt_cell.back() != c.rt_cells.size()) return false;
+    for (u32 v : c.rt_cells) if (v >= esl::kTeam * esl::kStageDoubles) return false;
     auto terms_ok = [&](const vector<u32> &t) {
         for (u32 v : t) if (v >= n) return false;
         return true;
@@ -2311,7 +2414,7 @@ u32 device_lds_max()
 // streams, checked. No device calls, so it runs on worker threads.
 // A tape of an engine whose lanes keep their factors in HBM (big), or the
 // first tape of an engine that does not fit a workgroup's LDS (which makes
-// the engine big), gets replay blocks and solve chunks instead of whole-tape
+// the engine big), gets replay blocks and a solve program instead of whole-tape
 // row programs and reduce streams.
 TapeHostProg *build_tape(const Engine &e, const HostTape &t, const char *&err)
 {
@@ -2324,8 +2427,10 @@ TapeHostProg *build_tape(const Engine &e, const HostTape &t, const char *&err)
         tp->big = true;
         tp->diag_tv.assign(n, 0);
         for (u32 i = 0; i < n; i++) tp->diag_tv[i] = tp->amap[e.c.diag[i]];
-        if (!build_big_program(t, *tp)) err = "tape program failed validation";
-        else if ((size_t)esl::big_lds_doubles(n, tp->prog.blk_m, tp->prog.sol_cap) * 8 > e.lds_limit)
+        // blocks as large as the LDS holds beside their pads
+        const u32 room = e.lds_limit / 8 - esl::kTeamThreads - esl::kTeamScratch;
+        if (!build_big_program(t, *tp, std::min(kBigSlotLimit, room))) err = "tape program failed validation";
+        else if ((size_t)esl::big_lds_doubles(n, tp->prog.blk_m) * 8 > e.lds_limit)
             err = "too many unknowns for a lane's solve vector in LDS";
     } else if (!fits) {
         err = "lane state exceeds the LDS of one workgroup";
@@ -2592,17 +2697,20 @@ esl_status esl_debug_big_replay(uint32_t n, const uint32_t *col_ptr, const uint3
     TapeHostProg o;
     build_tape_prog(t, cp, 1e-12, 1.0 / pivot_tol, o);
     o.big = true;
-    if (!build_big_program(t, o, block_slots) || !validate_big(o, n)) return ESL_FAILED;
+    // small blocks (many of them): narrow rows, the same programs otherwise
+    if (block_slots == 0) block_slots = kBigBlockSlots;
+    const u32 W = block_slots < 1024 ? (u32)esl::kWave : esl::kTeamThreads;
+    if (!build_big_program(t, o, block_slots, W) || !validate_big(o, n, W)) return ESL_FAILED;
     const esl::TapeProg &T = o.prog;
     if (sizes) {
         sizes[0] = T.n_blk;
         sizes[1] = T.n_l;
         sizes[2] = T.n_u;
-        sizes[3] = (u32)(o.blk_words.size() / esl::kWave);
+        sizes[3] = (u32)(o.blk_words.size() / W);
     }
     const u32 nnz = cp[n];
     for (u32 l = 0; l < lanes; l++) {
-        vector<double> tv(T.n_tv, 0.0), M(T.blk_m + esl::kWave, 0.0), y(n);
+        vector<double> tv(T.n_tv, 0.0), M(T.blk_m + W, 0.0), y(n);
         for (u32 p = 0; p < nnz; p++) tv[o.amap[p]] = a[(size_t)l * nnz + p];
         bool bad = false;
         uint64_t nonfinite = 0, worst = 0;
@@ -2614,8 +2722,8 @@ esl_status esl_debug_big_replay(uint32_t n, const uint32_t *col_ptr, const uint3
         for (const esl::BigBlock &B : o.blk) {
             for (u32 j = 0; j < B.m; j++) M[j] = tv[o.blk_slots[B.slot_off + j]];
             for (u32 r = B.row0; r < B.row0 + B.rows; r++)
-                for (u32 th = 0; th < (u32)esl::kWave; th++) {
-                    const esl::uint2_t w = o.blk_words[(size_t)r * esl::kWave + th];
+                for (u32 th = 0; th < W; th++) {
+                    const esl::uint2_t w = o.blk_words[(size_t)r * W + th];
                     const u32 kind = esl::row_kind(w.y), d = w.x & 0xffff, b = w.x >> 16, c = w.y & 0xffff;
                     if (kind == esl::R_MAC) {
                         const double m = M[b] * M[c];
@@ -2641,26 +2749,15 @@ esl_status esl_debug_big_replay(uint32_t n, const uint32_t *col_ptr, const uint3
         }
         fail[l] = (bad || nonfinite != 0 || !(dbl(worst) <= T.wide)) ? 1u : 0u;
         for (u32 r = 0; r < n; r++) y[o.pinv[r]] = -rhs[(size_t)l * n + r];
-        for (u32 c = 0; c < T.n_fch; c++)
-            for (u32 k = o.fch[c]; k < o.fch[c + 1]; k++) {
-                const double yk = y[k];
-                for (u32 qq = o.lp[k]; qq < o.lp[k + 1]; qq++) {
-                    const double old = y[o.li[qq]], m = tv[T.lx0 + qq] * yk, sv = old - m;
-                    y[o.li[qq]] = yk != 0.0 ? sv : old;
-                }
+        for (u32 r = 0; r < T.sol_rows; r++)
+            for (u32 th = 0; th < W; th++) {
+                const esl::uint2_t w = o.sol_w[(size_t)r * W + th];
+                const u32 d = w.x & 0xffff, c = w.x >> 16;
+                if (d >= n) continue;
+                const double v = y[d], A = tv[w.y & ~esl::kSolDiv];
+                const double m = A * y[c];
+                y[d] = (w.y & esl::kSolDiv) ? v / A : y[c] != 0.0 ? v - m : v;
             }
-        for (u32 c = T.n_bch; c > 0;) {
-            c--;
-            for (u32 k = o.bch[c + 1]; k > o.bch[c];) {
-                k--;
-                const double zk = y[k] / tv[T.n_u + k];
-                y[k] = zk;
-                for (u32 p = o.up[k]; p < o.up[k + 1]; p++) {
-                    const double old = y[o.ui[p]], m = tv[p] * zk, sv = old - m;
-                    y[o.ui[p]] = zk != 0.0 ? sv : old;
-                }
-            }
-        }
         for (u32 p = 0; p < T.n_u; p++) ux[(size_t)l * T.n_u + p] = tv[p];
         for (u32 k = 0; k < n; k++) udiag[(size_t)l * n + k] = tv[T.n_u + k];
         for (u32 qq = 0; qq < T.n_l; qq++) lx[(size_t)l * T.n_l + qq] = tv[T.lx0 + qq];
@@ -2901,23 +2998,12 @@ esl_status launch_lpt(Engine &e, const HostOpArgs &a, u32 lanes, u32 mode, float
 }
 
 // The LDS of a big engine's lanes: the staging cells, its tapes' largest
-// replay block, or the solve vector with its largest solve chunk.
+// replay block, or the solve vector.
 u32 big_lds(const Engine &e)
 {
-    u32 bm = 0, sc = 0;
-    for (const TapeHostProg *t : e.tapes) {
-        bm = std::max(bm, t->prog.blk_m);
-        sc = std::max(sc, t->prog.sol_cap);
-    }
-    return esl::big_lds_doubles(e.c.n, bm, sc);
-}
-
-// Lanes per big-lane workgroup: as many as the LDS of one workgroup holds,
-// at most kBigWaves.
-u32 big_waves(const Engine &e)
-{
-    const u32 per = big_lds(e) * 8;
-    return std::max<u32>(1, std::min<u32>(esl::kBigWaves, e.lds_limit / per));
+    u32 bm = 0;
+    for (const TapeHostProg *t : e.tapes) bm = std::max(bm, t->prog.blk_m);
+    return esl::big_lds_doubles(e.c.n, bm);
 }
 
 // The workspace of a big engine's launch over `lanes` lanes with up to
@@ -2932,7 +3018,7 @@ esl_status big_room(Engine &e, size_t lanes, u32 tv_cap)
         g_last_error = "too many unknowns for a lane's solve vector in LDS";
         return ESL_FAILED;
     }
-    HIPCHK(esl_big_attrs(big_waves(e) * lds));
+    HIPCHK(esl_big_attrs(lds));
     return ESL_OK;
 }
 
@@ -2946,13 +3032,17 @@ esl::BigArgs big_args(Engine &e, const esl::TranArgs &t, u32 lanes, u32 tran)
     b.tran = tran;
     b.tv_cap = t.op.tv_cap;
     b.lds = big_lds(e);
-    b.waves = big_waves(e);
+    b.n_rounds = e.n_rounds;
+    b.rt_round = e.rt_round;
+    b.rt_target = e.rt_target;
+    b.rt_cell = e.rt_cell;
+    b.rt_cells = e.rt_cells;
     return b;
 }
 
 // Launches the .op kernel over `grid` lanes (e.lane_ids; dump: op_dump):
-// one wavefront per lane with its working set in LDS, or for a big engine
-// one thread per lane with its working set in HBM.
+// one wavefront per lane with its working set in LDS, or for a big engine one
+// workgroup per lane with its factors in HBM.
 esl_status launch_op(Engine &e, const HostOpArgs &d, u32 grid, hipStream_t s)
 {
     if (e.big) {

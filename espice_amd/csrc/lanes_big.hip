@@ -1,16 +1,22 @@
 // Lanes whose working set is beyond a workgroup's LDS (the 64 x 64 RC mesh:
 // 4,099 unknowns and about 137,000 factor slots, 1.1 MB per lane): one
-// wavefront per lane as in the LDS kernels, with the lane's factor slots and
-// vectors in HBM (one contiguous region per lane) and LDS as the staging
-// area of each phase:
-// - assembly: the stamp cells of one chunk of 64 instances; each reduce task
-//   adds its cells into its target in HBM;
-// - refactor: the tape's replay cut into blocks of at most a few thousand
-//   slots; a block gathers its slots into LDS, runs its rows (64 independent
-//   updates per wavefront step, each slot's updates in the order of the
+// workgroup of kTeam wavefronts per lane, with the lane's factor slots and
+// vectors in HBM (one contiguous region per lane) and the whole LDS of a CU
+// as the staging area of each phase:
+// - assembly: the stamp cells of kTeam chunks of 64 instances, one chunk a
+//   wavefront; each reduce task adds its cells into its target in HBM;
+// - refactor: the tape's replay cut into blocks of as many slots as the LDS
+//   holds; a block gathers its slots into LDS, runs its rows (kTeamThreads
+//   independent updates per step, each slot's updates in the order of the
 //   column replay, lane_kernels.zig:49-118) and scatters what it wrote;
-// - solves: the solve vector in LDS, the L (forward) and U (backward)
-//   entries staged a chunk of columns at a time (lane_kernels.zig:123-143).
+// - solves: the solve vector in LDS, the factor entries read from their
+//   slots ahead of use (lane_kernels.zig:123-143).
+// One wavefront per lane and four lanes per CU left each lane a quarter of
+// the LDS: its blocks then hold a few columns at a time, whose dependency
+// chains leave half of 64 threads idle over 87,000 rows an iteration. The
+// team's rows are 10,700 (the mesh), each an LDS round trip and a barrier
+// (about 360 cycles; the refactor is 5.1 M of an iteration's 6.1 M cycles).
+// Measured, 256 lanes x 4 steps: 401 -> 75 ms.
 // The reference's lanes keep these arrays in global memory too, one thread
 // per lane walking the tape serially (lane_kernels.zig:7-8). Every value is
 // bitwise the wavefront kernels' and the oracle's: the same sums in the same
@@ -38,7 +44,24 @@ typedef __attribute__((address_space(3))) uint32_t lu32;
 struct BigLane {
     gdbl *tv, *rhs, *x, *xold, *sdiag, *q, *cq;
     ldbl *sm;
+    ldbl *scratch;   // kTeamScratch doubles: the team's reductions
 };
+
+// The team's reductions: the largest of every thread's v (as bit patterns),
+// and whether any thread's p holds; uniform. They are barriers.
+__device__ inline uint64_t team_max_u64(uint64_t v, ldbl *scratch)
+{
+    auto *s = (__attribute__((address_space(3))) uint64_t *)scratch;
+    const uint64_t w = wave_max_u64(v);
+    if (threadIdx.x % kWave == 0) s[threadIdx.x / kWave] = w;
+    __syncthreads();
+    uint64_t m = s[0];
+#pragma unroll
+    for (uint32_t k = 1; k < kTeam; k++) m = s[k] > m ? s[k] : m;
+    __syncthreads();
+    return uni(m);
+}
+__device__ inline bool team_any(bool p, ldbl *scratch) { return team_max_u64(p ? 1u : 0u, scratch) != 0; }
 
 __device__ inline BigLane big_lane(const BigArgs &b, uint32_t g, ldbl *sm)
 {
@@ -52,6 +75,7 @@ __device__ inline BigLane big_lane(const BigArgs &b, uint32_t g, ldbl *sm)
     L.q = L.sdiag + n;
     L.cq = L.q + n;
     L.sm = sm;
+    L.scratch = sm + (b.lds - kTeamScratch);
     return L;
 }
 
@@ -60,33 +84,39 @@ __device__ inline BigLane big_lane(const BigArgs &b, uint32_t g, ldbl *sm)
 // charges too (row charges into q, charge-Jacobian cells into cq), then the
 // ground pin and the companion A = G + ag0 C, F += ag0 (q - q1) - ag1 i_prev
 // (assemble_tran's arithmetic); otherwise capacitors and charge targets are
-// skipped and only the ground pin follows (assemble_pattern's). The stamp
-// cells of each chunk are staged in LDS.
-__device__ void big_assemble(const DeckProg &dp, const uint32_t *amap_, uint32_t n_slots, const double *live,
+// skipped and only the ground pin follows (assemble_pattern's). A round
+// stages the stamp cells of kTeam chunks in LDS, one chunk a wavefront, and
+// adds each target's cells in instance order.
+__device__ void big_assemble(const BigArgs &b, const uint32_t *amap_, uint32_t n_slots, const double *live,
                              gdbl *x, double *lim, gdbl *M, const BigLane &L, bool tran, double t, double ag0,
                              double ag1, gcdbl *q1, gcdbl *ip, uint32_t tid)
 {
+    const DeckProg &dp = b.ta.op.dp;
     const uint32_t n = dp.n;
     ldbl *st = L.sm;
     gcu32 *amap = amap_ ? gptr(amap_) : nullptr;
-    gcu32 *task_target = gptr(dp.task_target), *task_cell = gptr(dp.task_cell);
-    const __attribute__((address_space(1))) uint16_t *cells = gptr(dp.cells);
-    for (uint32_t i = tid; i < n_slots; i += kWave) M[i] = 0.0;
-    for (uint32_t i = tid; i < n; i += kWave) {
+    gcu32 *rt_target = gptr(b.rt_target), *rt_cell = gptr(b.rt_cell), *rt_round = gptr(b.rt_round);
+    const __attribute__((address_space(1))) uint16_t *cells = gptr(b.rt_cells);
+    const uint32_t wv = uni(tid / kWave), wt = tid % kWave;
+    for (uint32_t i = tid; i < n_slots; i += kTeamThreads) M[i] = 0.0;
+    for (uint32_t i = tid; i < n; i += kTeamThreads) {
         L.rhs[i] = 0.0;
         if (tran) L.q[i] = 0.0;
     }
     if (tran)
-        for (uint32_t k = tid; k < dp.n_cslot; k += kWave) L.cq[k] = 0.0;
-    wsync();
-    for (uint32_t c = 0; c < dp.n_chunks; c++) {
-        const Chunk ch = dp.chunks[c];
-        if (!tran && ch.kind == kC) continue;   // no static stamps
-        eval_chunk(dp, ch, live, x, lim, dp.n_mos, st, tid, t, tran);
-        wsync();
-        const uint32_t t1 = dp.chunks[c + 1].task_begin;
-        for (uint32_t k = ch.task_begin + tid; k < t1; k += kWave) {
-            const uint32_t tgt = task_target[k];
+        for (uint32_t k = tid; k < dp.n_cslot; k += kTeamThreads) L.cq[k] = 0.0;
+    __syncthreads();
+    for (uint32_t r = 0; r < b.n_rounds; r++) {
+        const uint32_t c = r * kTeam + wv;
+        if (c < dp.n_chunks) {
+            const Chunk ch = dp.chunks[c];
+            if (tran || ch.kind != kC)   // capacitors have no static stamps
+                eval_chunk(dp, ch, live, x, lim, dp.n_mos, st + wv * kStageDoubles, wt, t, tran);
+        }
+        __syncthreads();
+        const uint32_t t1 = rt_round[r + 1];
+        for (uint32_t k = rt_round[r] + tid; k < t1; k += kTeamThreads) {
+            const uint32_t tgt = rt_target[k];
             const uint32_t idx = tgt & kTargetMask;
             gdbl *d;
             if (tgt & kRhsBit) {
@@ -98,36 +128,36 @@ __device__ void big_assemble(const DeckProg &dp, const uint32_t *amap_, uint32_t
                 d = &M[amap ? amap[tgt] : tgt];
             }
             double acc = *d;
-            const uint32_t cc1 = task_cell[k + 1];
-            for (uint32_t cc = task_cell[k]; cc < cc1; cc++) acc = acc + st[cells[cc]];
+            const uint32_t cc1 = rt_cell[k + 1];
+            for (uint32_t cc = rt_cell[k]; cc < cc1; cc++) acc = acc + st[cells[cc]];
             *d = acc;
         }
-        wsync();
+        __syncthreads();
     }
     if (tid == 0) {
         const uint32_t d0 = amap ? amap[dp.diag0_slot] : dp.diag0_slot;
         M[d0] = M[d0] + 1.0;
         L.rhs[0] = L.rhs[0] + x[0];
     }
-    wsync();
+    __syncthreads();
     if (!tran) return;
     gcu32 *cslot_pat = gptr(dp.cslot_pat);
-    for (uint32_t k = tid; k < dp.n_cslot; k += kWave) {
+    for (uint32_t k = tid; k < dp.n_cslot; k += kTeamThreads) {
         const uint32_t sl = amap ? amap[cslot_pat[k]] : cslot_pat[k];
         M[sl] = M[sl] + ag0 * L.cq[k];
     }
-    for (uint32_t i = tid; i < n; i += kWave) {
+    for (uint32_t i = tid; i < n; i += kTeamThreads) {
         const double d = ag0 * (L.q[i] - q1[i]);
         const double base = L.rhs[i] + d;
         L.rhs[i] = base - ag1 * ip[i];
     }
-    wsync();
+    __syncthreads();
 }
 
 // Batched moves between HBM and LDS: each thread issues kBatch independent
-// loads before it uses any, so a wavefront has up to 16 x 64 loads in
-// flight instead of waiting on each.
-constexpr uint32_t kBatch = 16;
+// loads before it uses any, so a wavefront has up to 8 x 64 loads in flight
+// instead of waiting on each.
+constexpr uint32_t kBatch = 8;
 
 // dst[j] = src[idx[j]] for j < count (LDS from HBM through an index list).
 // Pipelined: the next batch's indices load while this batch's values do, so
@@ -137,22 +167,22 @@ __device__ inline void gather(ldbl *dst, gcdbl *src, gcu32 *idx, uint32_t count,
     uint32_t id[kBatch];
 #pragma unroll
     for (uint32_t u = 0; u < kBatch; u++) {
-        const uint32_t j = u * kWave + tid;
+        const uint32_t j = u * kTeamThreads + tid;
         id[u] = idx[j < count ? j : 0];
     }
-    for (uint32_t j0 = 0; j0 < count; j0 += kBatch * kWave) {
+    for (uint32_t j0 = 0; j0 < count; j0 += kBatch * kTeamThreads) {
         double v[kBatch];
 #pragma unroll
         for (uint32_t u = 0; u < kBatch; u++) v[u] = src[id[u]];
-        const uint32_t j1 = j0 + kBatch * kWave;
+        const uint32_t j1 = j0 + kBatch * kTeamThreads;
 #pragma unroll
         for (uint32_t u = 0; u < kBatch; u++) {
-            const uint32_t j = j1 + u * kWave + tid;
+            const uint32_t j = j1 + u * kTeamThreads + tid;
             id[u] = idx[j < count ? j : 0];
         }
 #pragma unroll
         for (uint32_t u = 0; u < kBatch; u++) {
-            const uint32_t j = j0 + u * kWave + tid;
+            const uint32_t j = j0 + u * kTeamThreads + tid;
             if (j < count) dst[j] = v[u];
         }
     }
@@ -161,37 +191,55 @@ __device__ inline void gather(ldbl *dst, gcdbl *src, gcu32 *idx, uint32_t count,
 // dst[idx[j]] = src[j] for j < count (HBM from LDS through an index list).
 __device__ inline void scatter(gdbl *dst, gcu32 *idx, const ldbl *src, uint32_t count, uint32_t tid)
 {
-    for (uint32_t j0 = 0; j0 < count; j0 += kBatch * kWave) {
+    for (uint32_t j0 = 0; j0 < count; j0 += kBatch * kTeamThreads) {
         uint32_t id[kBatch];
 #pragma unroll
         for (uint32_t u = 0; u < kBatch; u++) {
-            const uint32_t j = j0 + u * kWave + tid;
+            const uint32_t j = j0 + u * kTeamThreads + tid;
             id[u] = idx[j < count ? j : 0];
         }
 #pragma unroll
         for (uint32_t u = 0; u < kBatch; u++) {
-            const uint32_t j = j0 + u * kWave + tid;
+            const uint32_t j = j0 + u * kTeamThreads + tid;
             if (j < count) dst[id[u]] = src[j];
         }
     }
 }
 
-// dst[j] = src[j] for j < count (LDS from a contiguous HBM range, doubles
-// or 32-bit indices), with the same batching.
-template <typename D, typename S>
-__device__ inline void stage(D *dst, S *src, uint32_t count, uint32_t tid)
+// Between two rows: the team's LDS writes are done and seen.
+__device__ inline void row_sync()
 {
-    for (uint32_t j0 = 0; j0 < count; j0 += kBatch * kWave) {
-        decltype(+src[0]) v[kBatch];
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+    __builtin_amdgcn_s_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+}
+
+// run_rows for a team: rows of kTeamThreads words, a barrier between rows
+// (a row reads what other wavefronts wrote in earlier rows).
+template <typename WP>
+__device__ void run_rows_team(WP words, uint32_t rows, ldbl *M, double growth, LuFlags &f, uint32_t tid)
+{
+    const uint32_t base = (uint32_t)(uintptr_t)M;
+    WP w = words + tid;
+    uint2_t q[kRing];
 #pragma unroll
-        for (uint32_t u = 0; u < kBatch; u++) {
-            const uint32_t j = j0 + u * kWave + tid;
-            v[u] = src[j < count ? j : 0];
-        }
+    for (int k = 0; k < kRing; k++) {
+        q[k] = uint2_t{w[k * kTeamThreads].x, w[k * kTeamThreads].y};
+        __builtin_amdgcn_sched_barrier(0);
+    }
+    RowOp o = row_decode<double, false, false>(q[0], base);
+    for (uint32_t row = 0; row < rows; row += kRing) {
+        w += kRing * kTeamThreads;
 #pragma unroll
-        for (uint32_t u = 0; u < kBatch; u++) {
-            const uint32_t j = j0 + u * kWave + tid;
-            if (j < count) dst[j] = v[u];
+        for (int k = 0; k < kRing; k++) {
+            const double v = *(ldbl *)(uintptr_t)o.d, A = *(ldbl *)(uintptr_t)o.b, B = *(ldbl *)(uintptr_t)o.c;
+            const RowOp cur = o;
+            __builtin_amdgcn_sched_barrier(0);
+            q[k] = uint2_t{w[k * kTeamThreads].x, w[k * kTeamThreads].y};
+            o = row_decode<double, false, false>(q[(k + 1) % kRing], base);
+            __builtin_amdgcn_sched_barrier(0);
+            row_finish<double, false, false>(cur, v, A, B, growth, f);
+            row_sync();
         }
     }
 }
@@ -199,112 +247,103 @@ __device__ inline void stage(D *dst, S *src, uint32_t count, uint32_t tid)
 // The replay on the lane's slots in HBM: void pivots set to 1, the blocks
 // (gather into LDS, rows, scatter), then the peel tests of refactor(). True
 // when the lane must re-pivot.
-__device__ bool big_refactor(const TapeProg &T, uint32_t n, gdbl *tv, ldbl *M, uint32_t tid)
+__device__ bool big_refactor(const TapeProg &T, uint32_t n, gdbl *tv, const BigLane &L, uint32_t tid)
 {
+    ldbl *M = L.sm;
     gcu32 *flags = gptr(T.flags), *amap = gptr(T.amap), *void_slots = gptr(T.void_slots);
     LuFlags f{false, 0, 0};
-    for (uint32_t v = tid; v < T.n_void; v += kWave) f.bad |= tv[amap[void_slots[v]]] != 0.0;
-    for (uint32_t k = tid; k < n; k += kWave)
+    for (uint32_t v = tid; v < T.n_void; v += kTeamThreads) f.bad |= tv[amap[void_slots[v]]] != 0.0;
+    for (uint32_t k = tid; k < n; k += kTeamThreads)
         if (flags[k] & kVoidBit) tv[T.n_u + k] = 1.0;
-    wsync();
+    __syncthreads();
     const __attribute__((address_space(1))) BigBlock *blk = gptr(T.blk);
     for (uint32_t b = 0; b < T.n_blk; b++) {
-        const uint32_t m = blk[b].m, w = blk[b].w, rows = blk[b].rows, row0 = blk[b].row0;
-        gcu32 *sl = gptr(T.blk_slots) + blk[b].slot_off;
+        const uint32_t m = uni(blk[b].m), w = uni(blk[b].w), rows = uni(blk[b].rows), row0 = uni(blk[b].row0);
+        gcu32 *sl = gptr(T.blk_slots) + uni(blk[b].slot_off);
         gather(M, tv, sl, m, tid);
-        wsync();
-        run_rows<double>(gptr(T.blk_words) + (size_t)row0 * kWave, rows, M, T.growth, f, tid, 0u);
-        wsync();
+        __syncthreads();
+        run_rows_team(gptr(T.blk_words) + (size_t)row0 * kTeamThreads, rows, M, T.growth, f, tid);
         scatter(tv, sl, M, w, tid);
-        wsync();
+        __syncthreads();
     }
-    for (uint32_t p = tid; p < T.n_u; p += kWave) {
+    for (uint32_t p = tid; p < T.n_u; p += kTeamThreads) {
         const double u = tv[p];
         f.nonfinite |= dbits(u - u);
     }
-    for (uint32_t k = tid; k < n; k += kWave) {
+    for (uint32_t k = tid; k < n; k += kTeamThreads) {
         if (flags[k] & kVoidBit) continue;
         const double d = tv[T.n_u + k];
         f.bad |= d == 0.0 || !(fabs(d) < __builtin_inf());
     }
-    const uint64_t worst = wave_max_u64(f.worst);
+    const uint64_t worst = team_max_u64(f.worst, L.scratch);
     const bool fail = f.bad || f.nonfinite != 0 || !(bitsd(worst) <= T.wide);
-    return wave_any(fail);
+    return team_any(fail, L.scratch);
 }
 
 // dx = -A^-1 rhs into y (LDS, pivot order; row i's dx is y[qinv[i]]): the
-// forward sweep (L with zero skip) over chunks of columns whose L entries
-// and rows are staged after y, then the backward sweep over chunks whose U
-// entries, rows and pivots are staged (lane_kernels.zig:123-143). Within a
-// column the updated rows are distinct; columns run in order (LDS accesses
-// of one wavefront complete in issue order).
+// tape's solve program. A word and, kAhead rows later, the factor entry it
+// names are read ahead of their row, so a row costs its LDS round trip on
+// the solve vector and a barrier (every row's terms in the order of
+// lane_kernels.zig:123-143, with its zero skip).
 __device__ void big_solve(const TapeProg &T, uint32_t n, gcdbl *tv, gcdbl *rhs, ldbl *y, uint32_t tid)
 {
-    ldbl *sv = y + n;
-    lu32 *si = (lu32 *)(sv + T.sol_cap);
-    gcu32 *pinv = gptr(T.pinv), *lp = gptr(T.lp), *li = gptr(T.li), *up = gptr(T.up), *ui = gptr(T.ui);
-    gcu32 *fch = gptr(T.fch), *bch = gptr(T.bch);
-    for (uint32_t r = tid; r < n; r += kWave) y[pinv[r]] = -rhs[r];
-    wsync();
-    for (uint32_t c = 0; c < T.n_fch; c++) {
-        const uint32_t k0 = fch[c], k1 = fch[c + 1];
-        const uint32_t e0 = lp[k0], e1 = lp[k1];
-        stage(sv, tv + T.lx0 + e0, e1 - e0, tid);
-        stage(si, li + e0, e1 - e0, tid);
-        wsync();
-        for (uint32_t k = k0; k < k1; k++) {
-            const double yk = y[k];
-            const uint32_t q1 = lp[k + 1] - e0;
-            for (uint32_t q = lp[k] - e0 + tid; q < q1; q += kWave) {
-                const uint32_t r = si[q];
-                const double old = y[r];
-                const double m = sv[q] * yk;
-                const double s = old - m;
-                y[r] = yk != 0.0 ? s : old;
-            }
-        }
-        wsync();
+    constexpr int kAhead = kRing / 2;
+    gcu32 *pinv = gptr(T.pinv);
+    for (uint32_t r = tid; r < n; r += kTeamThreads) y[pinv[r]] = -rhs[r];
+    y[n + tid] = 0.0;   // the pads
+    const __attribute__((address_space(1))) uint2_t *w = gptr(T.sol_w) + tid;
+    uint2_t q[kRing];
+    double a[kAhead];
+#pragma unroll
+    for (int k = 0; k < kRing; k++) {
+        q[k] = uint2_t{w[k * kTeamThreads].x, w[k * kTeamThreads].y};
+        __builtin_amdgcn_sched_barrier(0);
     }
-    for (uint32_t c = T.n_bch; c > 0;) {
-        c--;
-        const uint32_t k0 = bch[c], k1 = bch[c + 1];
-        const uint32_t e0 = up[k0], e1 = up[k1], ne = e1 - e0;
-        stage(sv, tv + e0, ne, tid);
-        stage(si, ui + e0, ne, tid);
-        stage(sv + ne, tv + T.n_u + k0, k1 - k0, tid);
-        wsync();
-        for (uint32_t k = k1; k > k0;) {
-            k--;
-            const double zk = y[k] / sv[ne + (k - k0)];
-            if (tid == 0) y[k] = zk;
-            const uint32_t p1 = up[k + 1] - e0;
-            for (uint32_t p = up[k] - e0 + tid; p < p1; p += kWave) {
-                const uint32_t i = si[p];
-                const double old = y[i];
-                const double m = sv[p] * zk;
-                const double s = old - m;
-                y[i] = zk != 0.0 ? s : old;
+#pragma unroll
+    for (int k = 0; k < kAhead; k++) a[k] = tv[q[k].y & ~kSolDiv];
+    __syncthreads();
+    for (uint32_t row = 0; row < T.sol_rows; row += kRing) {
+        w += kRing * kTeamThreads;
+#pragma unroll
+        for (int k = 0; k < kRing; k++) {
+            const uint32_t x = q[k].x, kind = uni(q[k].y) & kSolDiv;
+            const uint32_t d = x & 0xffffu;
+            const double v = y[d], B = y[x >> 16], A = a[k % kAhead];
+            __builtin_amdgcn_sched_barrier(0);
+            // row + k + kAhead's entry, row + k + kRing's word
+            a[k % kAhead] = tv[q[(k + kAhead) % kRing].y & ~kSolDiv];
+            q[k] = uint2_t{w[k * kTeamThreads].x, w[k * kTeamThreads].y};
+            __builtin_amdgcn_sched_barrier(0);
+            const double m = A * B;
+            double r = B != 0.0 ? v - m : v;
+            if (kind) {
+                double piv = A;
+                pin(piv);   // a branch: every row would pay for a speculated division
+                r = v / piv;
             }
+            y[d] = r;
+            row_sync();
         }
-        wsync();
     }
 }
 
 // The plausible limit of a Newton run's first iterate (converger.zig:377-384).
-__device__ inline double big_limit_at(const TapeProg &T, uint32_t n, gcdbl *tv, gcdbl *x, gcdbl *rhs, uint32_t tid)
+__device__ inline double big_limit_at(const TapeProg &T, uint32_t n, const BigLane &L, uint32_t tid)
 {
     gcu32 *diag_tv = gptr(T.diag_tv);
+    gcdbl *tv = L.tv, *x = L.x, *rhs = L.rhs;
     double gm = 1.0;
     uint64_t xm = 0, fm = 0;
-    for (uint32_t i = tid; i < n; i += kWave) {
+    for (uint32_t i = tid; i < n; i += kTeamThreads) {
         gm = fmax(gm, fabs(tv[diag_tv[i]]));
         const uint64_t xb = dbits(fabs(x[i])), fb = dbits(fabs(rhs[i]));
         xm = xb > xm ? xb : xm;
         fm = fb > fm ? fb : fm;
     }
-    gm = wave_fmax(gm);
-    xm = wave_max_u64(xm);
-    fm = wave_max_u64(fm);
+    // gm >= 1: fmax drops a NaN, and non-negative doubles order as their bits
+    gm = bitsd(team_max_u64(dbits(gm), L.scratch));
+    xm = team_max_u64(xm, L.scratch);
+    fm = team_max_u64(fm, L.scratch);
     const double scale = fmin(fmax(bitsd(xm), bitsd(fm) * gm), 1e18);
     return !(1e3 * scale > 1e9) ? 1e9 : 1e3 * scale;
 }
@@ -318,7 +357,7 @@ __device__ inline double big_update(const OpArgs &a, const TapeProg &T, const Bi
     gcu32 *qinv = gptr(T.qinv);
     const __attribute__((address_space(1))) uint8_t *current_row = gptr(dp.current_row);
     uint64_t worst = 0;
-    for (uint32_t i = tid; i < dp.n; i += kWave) {
+    for (uint32_t i = tid; i < dp.n; i += kTeamThreads) {
         const double xo = L.x[i];
         const double d = y[qinv[i]];
         const double xn = xo + d;
@@ -331,13 +370,14 @@ __device__ inline double big_update(const OpArgs &a, const TapeProg &T, const Bi
         const uint64_t sb = dbits(score);
         worst = sb > worst ? sb : worst;
     }
-    return bitsd(wave_max_u64(worst));
+    return bitsd(team_max_u64(worst, L.scratch));
 }
 
 // Limiting after an update (MOS1, diodes, BJTs): true when any limited.
-__device__ __forceinline__ bool big_limit(const DeckProg &dp, const double *live, gcdbl *x, double *lim, uint32_t tid)
+__device__ __forceinline__ bool big_limit(const DeckProg &dp, const double *live, const BigLane &L, double *lim,
+                                          uint32_t tid)
 {
-    return wave_any(limit_pass(dp, live, x, lim, tid));
+    return team_any(limit_pass<kTeamThreads>(dp, live, (gcdbl *)L.x, lim, tid), L.scratch);
 }
 
 // One lane's operating point (op_lane's FP64 path: cold, given or resumed
@@ -346,19 +386,20 @@ __device__ __forceinline__ bool big_limit(const DeckProg &dp, const double *live
 __device__ __forceinline__ void big_op_lane(const BigArgs &b, uint32_t g, uint32_t lane, ldbl *sm)
 {
     const OpArgs &a = b.ta.op;
-    const uint32_t tid = threadIdx.x % kWave;
+    const uint32_t tid = threadIdx.x;
     const DeckProg &dp = a.dp;
     const uint32_t n = dp.n;
     const BigLane L = big_lane(b, g, sm);
     const double *live = a.live + (size_t)lane * dp.n_live;
     double *lim = a.lim + (size_t)lane * lim_width(dp);
     gdbl *xg = gptr(a.x) + (size_t)lane * n;
-    lane_init(a, lane, live, (double *)L.x, lim, tid);
+    lane_init<kTeamThreads>(a, lane, live, (double *)L.x, lim, tid);
+    __syncthreads();
     if (a.dump) {
-        big_assemble(dp, nullptr, dp.nnz, live, L.x, lim, gptr(a.a_out) + (size_t)g * dp.nnz, L, false, 0.0, 0.0,
+        big_assemble(b, nullptr, dp.nnz, live, L.x, lim, gptr(a.a_out) + (size_t)g * dp.nnz, L, false, 0.0, 0.0,
                      0.0, nullptr, nullptr, tid);
         gdbl *f = gptr(a.f_out) + (size_t)g * n;
-        for (uint32_t i = tid; i < n; i += kWave) f[i] = L.rhs[i];
+        for (uint32_t i = tid; i < n; i += kTeamThreads) f[i] = L.rhs[i];
         return;
     }
     const LaneResume rs = a.resume[lane];
@@ -385,15 +426,15 @@ __device__ __forceinline__ void big_op_lane(const BigArgs &b, uint32_t g, uint32
     uint32_t iter = iter0;
     for (; iter - k0 < a.max_iter; iter++) {
         lap(3);
-        big_assemble(dp, T.amap, T.n_tv, live, L.x, lim, L.tv, L, false, 0.0, 0.0, 0.0, nullptr, nullptr, tid);
-        if (iter == k0) limit = big_limit_at(T, n, L.tv, L.x, L.rhs, tid);
-        for (uint32_t i = tid; i < n; i += kWave) L.sdiag[i] = L.tv[T.diag_tv[i]];
-        wsync();
+        big_assemble(b, T.amap, T.n_tv, live, L.x, lim, L.tv, L, false, 0.0, 0.0, 0.0, nullptr, nullptr, tid);
+        if (iter == k0) limit = big_limit_at(T, n, L, tid);
+        for (uint32_t i = tid; i < n; i += kTeamThreads) L.sdiag[i] = L.tv[T.diag_tv[i]];
+        __syncthreads();
         lap(0);
-        const bool repivot = big_refactor(T, n, L.tv, L.sm, tid);
+        const bool repivot = big_refactor(T, n, L.tv, L, tid);
         lap(1);
         if (repivot) {
-            for (uint32_t i = tid; i < n; i += kWave) xg[i] = L.x[i];
+            for (uint32_t i = tid; i < n; i += kTeamThreads) xg[i] = L.x[i];
             if (tid == 0) {
                 LaneResume o{};
                 o.iter = iter;
@@ -406,8 +447,8 @@ __device__ __forceinline__ void big_op_lane(const BigArgs &b, uint32_t g, uint32
             if (a.a_out) {
                 // the Jacobian at this iterate (pattern order) for the host's
                 // re-pivot: the same sums as the failed assembly
-                wsync();
-                big_assemble(dp, nullptr, dp.nnz, live, L.x, lim, gptr(a.a_out) + (size_t)lane * dp.nnz, L, false,
+                __syncthreads();
+                big_assemble(b, nullptr, dp.nnz, live, L.x, lim, gptr(a.a_out) + (size_t)lane * dp.nnz, L, false,
                              0.0, 0.0, 0.0, nullptr, nullptr, tid);
             }
             status = kRepivot;
@@ -415,15 +456,15 @@ __device__ __forceinline__ void big_op_lane(const BigArgs &b, uint32_t g, uint32
             break;
         }
         big_solve(T, n, L.tv, L.rhs, L.sm, tid);
-        wsync();
+        __syncthreads();
         lap(2);
         const double scaled = big_update(a, T, L, tid);
-        wsync();
-        const bool limited = big_limit(dp, live, L.x, lim, tid);
+        __syncthreads();
+        const bool limited = big_limit(dp, live, L, lim, tid);
         bool ok = !limited && iter != k0 && scaled < 1.0;
         if (ok) {
             bool miss = false;
-            for (uint32_t i = tid; i < n; i += kWave) {
+            for (uint32_t i = tid; i < n; i += kTeamThreads) {
                 const double xi = L.x[i];
                 miss |= !(fabs(xi) <= limit);
                 const double s0 = fabs(L.sdiag[i]);
@@ -431,22 +472,22 @@ __device__ __forceinline__ void big_op_lane(const BigArgs &b, uint32_t g, uint32
                 const double rt = fmax(a.residual_tol, 10.0 * s * (a.reltol * fabs(xi) + a.vntol));
                 miss |= !(fabs(L.rhs[i]) <= rt);
             }
-            ok = !wave_any(miss);
+            ok = !team_any(miss, L.scratch);
         }
         if (ok && init_fix) {
             init_fix = false;
         } else if (ok) {
-            for (uint32_t i = tid; i < n; i += kWave) L.x[i] = L.xold[i];
+            for (uint32_t i = tid; i < n; i += kTeamThreads) L.x[i] = L.xold[i];
             status = kConverged;
             iters = iter + 1;
             break;
         }
-        wsync();
+        __syncthreads();
     }
     if (status == kNoConvergence) iters = iter;
-    wsync();
+    __syncthreads();
     if (status != kRepivot)
-        for (uint32_t i = tid; i < n; i += kWave) xg[i] = L.x[i];
+        for (uint32_t i = tid; i < n; i += kTeamThreads) xg[i] = L.x[i];
     lap(3);
     if (tid == 0) {
         a.status[lane] = status;
@@ -464,7 +505,7 @@ __device__ __forceinline__ void big_tran_lane(const BigArgs &b, uint32_t g, uint
 {
     const TranArgs &ta = b.ta;
     const OpArgs &a = ta.op;
-    const uint32_t tid = threadIdx.x % kWave;
+    const uint32_t tid = threadIdx.x;
     if (a.status[lane] != kTranRunning) return;
     uint32_t s = ta.step[lane];
     if (s >= ta.s1) return;
@@ -482,27 +523,27 @@ __device__ __forceinline__ void big_tran_lane(const BigArgs &b, uint32_t g, uint
     const TapeProg T = a.tapes[rs.tape];
     gdbl *aout = gptr(a.a_out) + (size_t)lane * dp.nnz;
     gcu32 *amap = gptr(T.amap);
-    for (uint32_t i = tid; i < n; i += kWave) L.x[i] = xg[i];
-    wsync();
+    for (uint32_t i = tid; i < n; i += kTeamThreads) L.x[i] = xg[i];
+    __syncthreads();
     if (ta.init) {
         // start at the operating point: limiting state at its own voltages,
         // charges from one evaluation there, no dynamic current
-        seed_lim_at(dp, live, (const double *)L.x, lim, tid);
-        for (uint32_t i = tid; i < n; i += kWave) {
+        seed_lim_at<kTeamThreads>(dp, live, (const double *)L.x, lim, tid);
+        for (uint32_t i = tid; i < n; i += kTeamThreads) {
             q1[i] = 0.0;
             ip[i] = 0.0;
             xp[i] = L.x[i];
         }
-        wsync();
-        big_assemble(dp, T.amap, T.n_tv, live, L.x, lim, L.tv, L, true, 0.0, 0.0, 0.0, q1, ip, tid);
-        for (uint32_t i = tid; i < n; i += kWave) q1[i] = L.q[i];
-        wsync();
+        __syncthreads();
+        big_assemble(b, T.amap, T.n_tv, live, L.x, lim, L.tv, L, true, 0.0, 0.0, 0.0, q1, ip, tid);
+        for (uint32_t i = tid; i < n; i += kTeamThreads) q1[i] = L.q[i];
+        __syncthreads();
         if (ta.dump) {
-            big_assemble(dp, nullptr, dp.nnz, live, L.x, lim, aout, L, true, ta.dt, 1.0 / ta.dt, 0.0, q1, ip, tid);
+            big_assemble(b, nullptr, dp.nnz, live, L.x, lim, aout, L, true, ta.dt, 1.0 / ta.dt, 0.0, q1, ip, tid);
             return;
         }
     }
-    wsync();
+    __syncthreads();
     uint32_t iter0 = rs.iter;   // nonzero only when resuming inside a step
     double limit = rs.limit;
     uint32_t status = kTranRunning;
@@ -524,18 +565,18 @@ __device__ __forceinline__ void big_tran_lane(const BigArgs &b, uint32_t g, uint
         uint32_t iter = iter0;
         for (; iter < a.max_iter; iter++) {
             lap(3);
-            big_assemble(dp, T.amap, T.n_tv, live, L.x, lim, L.tv, L, true, t, ag0, ag1, q1, ip, tid);
-            if (iter == 0) limit = big_limit_at(T, n, L.tv, L.x, L.rhs, tid);
-            wsync();
+            big_assemble(b, T.amap, T.n_tv, live, L.x, lim, L.tv, L, true, t, ag0, ag1, q1, ip, tid);
+            if (iter == 0) limit = big_limit_at(T, n, L, tid);
+            __syncthreads();
             lap(0);
-            const bool repivot = big_refactor(T, n, L.tv, L.sm, tid);
+            const bool repivot = big_refactor(T, n, L.tv, L, tid);
             lap(1);
             if (repivot) {
                 // the Jacobian again, read out in pattern order for the
                 // host's re-pivot; resume at this iterate
-                wsync();
-                big_assemble(dp, T.amap, T.n_tv, live, L.x, lim, L.tv, L, true, t, ag0, ag1, q1, ip, tid);
-                for (uint32_t p = tid; p < dp.nnz; p += kWave) aout[p] = L.tv[amap[p]];
+                __syncthreads();
+                big_assemble(b, T.amap, T.n_tv, live, L.x, lim, L.tv, L, true, t, ag0, ag1, q1, ip, tid);
+                for (uint32_t p = tid; p < dp.nnz; p += kTeamThreads) aout[p] = L.tv[amap[p]];
                 if (tid == 0) {
                     LaneResume o = rs;
                     o.iter = iter;
@@ -547,23 +588,23 @@ __device__ __forceinline__ void big_tran_lane(const BigArgs &b, uint32_t g, uint
                 break;
             }
             big_solve(T, n, L.tv, L.rhs, L.sm, tid);
-            wsync();
+            __syncthreads();
             lap(2);
             const double scaled = big_update(a, T, L, tid);
-            wsync();
-            const bool limited = big_limit(dp, live, L.x, lim, tid);
+            __syncthreads();
+            const bool limited = big_limit(dp, live, L, lim, tid);
             bool ok = !limited && iter != 0 && scaled < 1.0;
             if (ok) {
                 bool miss = false;
-                for (uint32_t i = tid; i < n; i += kWave) {
+                for (uint32_t i = tid; i < n; i += kTeamThreads) {
                     miss |= !(fabs(L.x[i]) <= limit);
                     miss |= !(fabs(L.rhs[i]) <= __builtin_inf());
                 }
-                ok = !wave_any(miss);
+                ok = !team_any(miss, L.scratch);
             }
-            wsync();
+            __syncthreads();
             if (ok) {
-                for (uint32_t i = tid; i < n; i += kWave) L.x[i] = L.xold[i];
+                for (uint32_t i = tid; i < n; i += kTeamThreads) L.x[i] = L.xold[i];
                 converged = true;
                 iter++;
                 break;
@@ -578,34 +619,34 @@ __device__ __forceinline__ void big_tran_lane(const BigArgs &b, uint32_t g, uint
         }
         // accept: q holds the charges of the converged point (the last
         // assembly ran at x_old)
-        wsync();
-        for (uint32_t i = tid; i < n; i += kWave) {
+        __syncthreads();
+        for (uint32_t i = tid; i < n; i += kTeamThreads) {
             const double d = ag0 * (L.q[i] - q1[i]);
             ip[i] = d - ag1 * ip[i];
             q1[i] = L.q[i];
         }
-        for (uint32_t k = tid; k < ta.n_probes; k += kWave)
+        for (uint32_t k = tid; k < ta.n_probes; k += kTeamThreads)
             ta.probes[((size_t)lane * ta.steps + s) * ta.n_probes + k] = L.x[ta.probe_ids[k]];
-        wsync();
-        seed_lim_at(dp, live, (const double *)L.x, lim, tid, true);
-        wsync();
+        __syncthreads();
+        seed_lim_at<kTeamThreads>(dp, live, (const double *)L.x, lim, tid, true);
+        __syncthreads();
         // the next step's first iterate: the last two accepted points
         // extrapolated (tran.zig:1131-1137; lane_device.zig:141-153), then
         // one limit pass against the accepted point (tran.zig:1138)
         if (s + 1 < ta.steps) {
-            for (uint32_t i = tid; i < n; i += kWave) {
+            for (uint32_t i = tid; i < n; i += kTeamThreads) {
                 const double cu = L.x[i];
                 L.x[i] = cu + (cu - xp[i]);
                 xp[i] = cu;
             }
-            wsync();
-            limit_pass(dp, live, (gcdbl *)L.x, lim, tid);
-            wsync();
+            __syncthreads();
+            limit_pass<kTeamThreads>(dp, live, (gcdbl *)L.x, lim, tid);
+            __syncthreads();
         }
     }
     lap(3);
     if (status == kTranRunning && s >= ta.steps) status = kConverged;
-    for (uint32_t i = tid; i < n; i += kWave) xg[i] = L.x[i];
+    for (uint32_t i = tid; i < n; i += kTeamThreads) xg[i] = L.x[i];
     if (tid == 0) {
         if (status != kRepivot) {
             LaneResume o = rs;
@@ -620,19 +661,14 @@ __device__ __forceinline__ void big_tran_lane(const BigArgs &b, uint32_t g, uint
     }
 }
 
-// Workgroups of b.waves wavefronts, each wavefront one lane in its own
-// b.lds doubles of the LDS. The lanes of a workgroup start together and do
-// the same work per Newton iteration (the same tape), so they walk the
-// replay's row words nearly in step and share their fetches in the caches;
-// they never wait on one another.
-__global__ __launch_bounds__(kWave * kBigWaves) void big_lanes(BigArgs b)
+// One workgroup per lane: the lanes walk the same tape nearly in step, so
+// the lanes of an XCD share their words' fetches in its L2.
+__global__ __launch_bounds__(kTeamThreads) void big_lanes(BigArgs b)
 {
-    const uint32_t w = threadIdx.x / kWave;
-    const uint32_t g = blockIdx.x * b.waves + w;
-    if (g >= b.N) return;
-    const uint32_t lane = b.ta.op.lane_ids[g];
+    const uint32_t g = blockIdx.x;
+    const uint32_t lane = uni(b.ta.op.lane_ids[g]);
     extern __shared__ double dyn[];
-    ldbl *sm = lptr(dyn) + (size_t)w * b.lds;
+    ldbl *sm = lptr(dyn);
     if (b.tran) big_tran_lane(b, g, lane, sm);
     else big_op_lane(b, g, lane, sm);
 }
@@ -648,8 +684,6 @@ extern "C" hipError_t esl_big_attrs(uint32_t lds_bytes)
 
 extern "C" hipError_t esl_launch_big(const esl::BigArgs *b, hipStream_t s)
 {
-    const uint32_t grid = (b->N + b->waves - 1) / b->waves;
-    hipLaunchKernelGGL(esl::big_lanes, dim3(grid), dim3(esl::kWave * b->waves),
-                       b->waves * b->lds * (uint32_t)sizeof(double), s, *b);
+    hipLaunchKernelGGL(esl::big_lanes, dim3(b->N), dim3(esl::kTeamThreads), b->lds * (uint32_t)sizeof(double), s, *b);
     return hipGetLastError();
 }

@@ -107,3 +107,16 @@ def test_peel_cases_fail_as_serial(lanes, oracle):
     for lead, bad in (([1.0, 0.5, 0.0, 1.0], [1e-4, 1.0, 0.0, 1.0]), ([1.0, 0.5, 0.5, 1.0], [1e-13, 1.0, 0.5, 1.0])):
         got, ok = compare(lanes, oracle, cp, ri, np.array(lead), [0, 1], np.array([lead, bad]), np.ones((2, 2)), 3)
         assert list(got["fail"]) == [0, 1]
+
+
+@pytest.mark.parametrize("k,block_slots", [(5, 1024), (9, 1500), (14, 2048), (14, 18944)])
+def test_team_rows_equal_serial(lanes, oracle, k, block_slots):
+    """Blocks run in rows of 512 words (wide blocks) equal the serial replay:
+    one block, several, and rows with more ops than a wavefront holds."""
+    rng = np.random.default_rng(k)
+    cp, ri, lead = grid_laplacian(rng, k)
+    q = np.arange(k * k, dtype=np.uint32)
+    a = lead * (1 + 0.02 * rng.standard_normal((3, len(lead))))
+    rhs = rng.standard_normal((3, k * k))
+    got, ok = compare(lanes, oracle, cp, ri, lead, q, a, rhs, block_slots)
+    assert ok.all()
