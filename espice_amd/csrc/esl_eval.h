@@ -40,13 +40,26 @@ __device__ inline double wave_fmax(double v)
 }
 
 // Keeps a value in a vector register at this point: its computation is
-// neither moved past here nor speculated above it.
-template <typename T>
-__device__ inline void pin(T &v)
+// neither moved past here nor speculated above it. Only 32-bit operands: the
+// "v" constraint may give a 64-bit one a register pair that starts at an odd
+// register, which gfx950 instructions cannot address.
+__device__ inline void pin(uint32_t &v)
 {
 #if defined(__HIP_DEVICE_COMPILE__)
     asm volatile("" : "+v"(v));
 #endif
+}
+__device__ inline void pin(float &v)
+{
+#if defined(__HIP_DEVICE_COMPILE__)
+    asm volatile("" : "+v"(v));
+#endif
+}
+__device__ inline void pin(double &v)
+{
+    uint32_t lo = (uint32_t)dbits(v);
+    pin(lo);
+    v = bitsd((dbits(v) & 0xffffffff00000000ull) | lo);
 }
 
 __device__ inline bool wave_any(bool p) { return __any((int)p) != 0; }

@@ -161,12 +161,19 @@ constexpr uint32_t kFlagUnscaled = 1;   // R_DIV on an unscaled column: growth +
 constexpr uint32_t kFlagScaled = 2;     // R_DIV on a scaled column: non-finite test
 inline constexpr uint32_t row_kind(uint32_t y) { return (y >> 16) & 0xfu; }
 inline constexpr uint32_t row_flags(uint32_t y) { return (y >> 20) & 0x3u; }
-// Reduce-stream words: a target word sets the accumulator's slot (bit 30:
-// residual row, else factor slot); a cell word adds one staged value.
+// Chain headers of the assembly reduce: a target word names the factor slot
+// or (kRedRhs) the double at rhs + index.
 constexpr uint32_t kRedTarget = 0x80000000u, kRedRhs = 0x40000000u;
-// A reduce stream's padding word: a target word for the lane's scratch
-// double at rhs + 2n (after x), which nothing else reads.
-__host__ __device__ inline uint32_t red_pad(uint32_t n) { return kRedTarget | kRedRhs | (2 * n); }
+// Reduce rows: words {x = target | c0 << 16, y = c1 | c2 << 16}, one per
+// thread of a row: the target takes the staged cells c0, c1, c2 in that
+// order; a target with more cells continues in later rows. target: a factor
+// slot below n_tv, n_tv + i for the double at rhs + i. kRedNone: no cell (it
+// reads as -0, which leaves any sum unchanged). Idle threads add nothing to
+// a scratch double behind the lane's working set, which holds two: that one
+// and the -0.
+constexpr uint32_t kRedNone = 0xffffu;
+constexpr int kRedCells = 3;
+constexpr int kRedRing = 4;    // rows of words in flight; a stream is a multiple of it
 constexpr int kRing = 16;      // rows in flight; streams carry kRing pad rows
 // 16-bit cell indices of a chunk's reduce chains: they fill the 64 pad
 // slots of the factor area
@@ -174,9 +181,9 @@ constexpr uint32_t kRedChainCells = 256;
 
 // Doubles of a lane's working set in LDS: tv_cap factor slots, the Y block
 // (y, sdiag, xold after the assembly; during it the stamp staging areas,
-// one per wavefront of the lane's crew), rhs, x, and a scratch pair that
-// the assembly reduce's padding words write (rhs + 2n). A transient lane's
-// Y block holds y and xold, and q and the charge-Jacobian cells follow x.
+// one per wavefront of the lane's crew), rhs, x, and the assembly reduce's
+// scratch pair. A transient lane's Y block holds y and xold, and q and the
+// charge-Jacobian cells follow x, then the scratch pair.
 constexpr uint32_t kStageDoubles = kWave * kStageEntries;
 __host__ __device__ inline uint32_t lds_y_block(uint32_t n, uint32_t nw = 1)
 {
@@ -194,7 +201,7 @@ __host__ __device__ inline uint32_t tran_y_block(uint32_t n, uint32_t nw = 1)
 }
 __host__ __device__ inline uint32_t tran_doubles(uint32_t tv_cap, uint32_t n, uint32_t n_cslot, uint32_t nw = 1)
 {
-    return tv_cap + tran_y_block(n, nw) + 3 * n + n_cslot;
+    return tv_cap + tran_y_block(n, nw) + 3 * n + n_cslot + 2;
 }
 
 // A lane beyond a workgroup's LDS (a big lane) runs on a team of kTeam
@@ -243,9 +250,9 @@ struct TapeProg {
     // row programs: [rows + kRing][64] words (the kRing tail rows are R_NOP)
     const uint2_t *rw;          // refactor
     const uint2_t *sw;          // forward + backward solve
-    const uint32_t *red;        // assembly reduce words, per chunk [len + kRing][64]
-    const uint32_t *red_off;    // [n_chunks] word offset of each chunk's stream
-    const uint32_t *red_len;    // [n_chunks] rows of each chunk's stream (multiple of kRing)
+    const uint2_t *red;         // assembly reduce rows, per chunk and analysis [len + kRedRing][64]
+    const uint4_t *red_h;       // two per stream (2 c: .op, 2 c + 1: transient): {word offset, rows | chains << 16,
+                                // first chain header, first index word | blocks << 26}, the chunk {kind, first, count}
     const uint32_t *diag_tv;    // [n] tv slot of each row's diagonal
     const uint32_t *li;         // [n_l] row (pivot step) of each L entry
     // big tapes (lanes whose slots live in HBM): the replay in blocks of at
@@ -265,14 +272,12 @@ struct TapeProg {
     // [res_total]: the factor slot each position of a lane's packed FP64
     // Jacobian copies (a pad slot for a row start, whose value is unused)
     const uint32_t *rsrc;
-    // assembly reduce chains: the longest targets of each chunk, one per
-    // thread; headers {target word as in the reduce stream, cells | index
-    // offset << 16} from rc_off[c] (rc_count[c] of them), the chunk's
-    // kRedChainCells 16-bit cell indices from word rc_coff[c], staged in
-    // the pad slots while the chains run, rc_blocks[c] blocks of kChainBlk
+    // assembly reduce chains: the longest targets of each stream, one per
+    // thread; headers {target word, cells | index offset << 16}, the
+    // stream's kRedChainCells 16-bit cell indices, staged in the pad slots
+    // while the chains run, as many blocks of kChainBlk as the longest has
     const uint2_t *rc_head;
     const uint32_t *rc_cells;
-    const uint32_t *rc_off, *rc_count, *rc_coff, *rc_blocks;
 };
 
 // Per-lane results of the Newton kernel.

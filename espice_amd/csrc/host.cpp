@@ -703,12 +703,14 @@ struct TapeHostProg {
     vector<u32> flev_ptr, flev_rows, lrow_ptr, lrow_k, lrow_slot;
     vector<u32> blev_ptr, blev_rows, urow_ptr, urow_k, urow_slot, void_slots;
     RowProgram rch, sch;
-    vector<u32> red, red_off, red_len, diag_tv;
+    vector<esl::uint2_t> red;
+    vector<u32> red_off, red_len, diag_tv;
     // assembly reduce chains: headers {target word, cells | index offset <<
     // 16}, per chunk with chains kRedChainCells 16-bit cell indices, and per
     // chunk its first header, chains, first index word and blocks
     vector<esl::uint2_t> rc_head;
     vector<u32> rc_cells, rc_off, rc_count, rc_coff, rc_blocks;
+    vector<esl::uint4_t> red_h;
     vector<u32> rsrc;   // the factor slot of each position of the packed FP64 Jacobian
     uint64_t flops = 0;
     // lanes beyond a workgroup's LDS: the replay in blocks and the solves in
@@ -1107,7 +1109,7 @@ hipError_t upload_tape_prog(TapeHostProg &o)
     f.push_back(pk.add(o.rch.words));
     f.push_back(pk.add(o.sch.words));
     f.push_back(pk.add(o.red));
-    f.push_back(pk.add(o.red_off)); f.push_back(pk.add(o.red_len)); f.push_back(pk.add(o.diag_tv));
+    f.push_back(pk.add(o.red_h)); f.push_back(pk.add(o.diag_tv));
     f.push_back(pk.add(o.li));
     f.push_back(pk.add(o.blk)); f.push_back(pk.add(o.blk_slots)); f.push_back(pk.add(o.blk_words));
     f.push_back(pk.add(o.sol_w));
@@ -1115,8 +1117,6 @@ hipError_t upload_tape_prog(TapeHostProg &o)
     f.push_back(pk.add(o.rch.cw)); f.push_back(pk.add(o.sch.cw));
     f.push_back(pk.add(o.rsrc));
     f.push_back(pk.add(o.rc_head)); f.push_back(pk.add(o.rc_cells));
-    f.push_back(pk.add(o.rc_off)); f.push_back(pk.add(o.rc_count));
-    f.push_back(pk.add(o.rc_coff)); f.push_back(pk.add(o.rc_blocks));
     hipError_t e = o.buf.ensure(pk.blob.size());
     if (e != hipSuccess) return e;
     e = hipMemcpy(o.buf.p, pk.blob.data(), pk.blob.size(), hipMemcpyHostToDevice);
@@ -1136,9 +1136,8 @@ hipError_t upload_tape_prog(TapeHostProg &o)
     T.sw = reinterpret_cast<const esl::uint2_t *>(P(i++));
     T.rw_rows = o.rch.rows;
     T.sw_rows = o.sch.rows;
-    T.red = P(i++);
-    T.red_off = P(i++);
-    T.red_len = P(i++);
+    T.red = reinterpret_cast<const esl::uint2_t *>(P(i++));
+    T.red_h = reinterpret_cast<const esl::uint4_t *>(P(i++));
     T.diag_tv = P(i++);
     T.li = P(i++);
     T.blk = reinterpret_cast<const esl::BigBlock *>(P(i++));
@@ -1152,10 +1151,6 @@ hipError_t upload_tape_prog(TapeHostProg &o)
     T.rsrc = P(i++);
     T.rc_head = reinterpret_cast<const esl::uint2_t *>(P(i++));
     T.rc_cells = P(i++);
-    T.rc_off = P(i++);
-    T.rc_count = P(i++);
-    T.rc_coff = P(i++);
-    T.rc_blocks = P(i++);
     if (i != f.size()) return hipErrorInvalidValue;
     return hipSuccess;
 }
@@ -2030,25 +2025,24 @@ u32 own_lds_bytes(u32 lds, u32 grid, u32 n, u32 nnz, u32 nnz_l, u32 nnz_u)
     return (u32)std::max<size_t>(lds, std::min(want, room));
 }
 
-
-
-// Assembly reduce streams for one tape: each chunk's reduce tasks with their
-// targets mapped to factor slots, dealt to the 64 threads longest first, each
-// thread's words laid out row by row ([row][64]) so a wavefront reads one
-// coalesced row per step. A step costs the whole wavefront whatever its
-// threads hold, so a target with far more cells than the chunk's average
-// (a supply rail's diagonal and residual row, which collect cells from
-// every device on the rail) would set the stream's length by itself; the
-// longest tasks of a chunk instead become chains, one per thread, which add
-// their cells in order with the target in a register, eight cells a block,
-// their 16-bit cell indices staged in the tape's 64 pad slots (unused
-// during the assembly; room for kRedChainCells indices). The split is
-// chosen per chunk by a cost model of the two loops (cycles per stream step
-// and per chain block, measured).
+// The assembly reduce of each chunk and analysis (.op: the static targets;
+// transient: the charges too): the chunk's reduce tasks, their targets
+// mapped to the lane's working set, as rows of 64 words of up to kRedCells
+// cells each. A target's words sit in successive rows, the longest targets
+// first, so a stream has as many rows as its words need or its longest
+// target has. A supply rail's diagonal and residual row collect cells from
+// every device on the rail; such targets become chains instead, one per
+// thread, which add their cells in order with the target in a register,
+// eight cells a block, their 16-bit cell indices staged in the tape's 64 pad
+// slots (unused during the assembly; room for kRedChainCells indices). The
+// split is chosen per stream by a cost model of the two loops (cycles per
+// row and per chain block, measured).
 void build_reduce_streams(const Compiled &c, TapeHostProg &o)
 {
-    constexpr double kStepCost = 130.0, kChainSetup = 300.0, kBlockCost = 200.0;
+    constexpr double kRowCost = 150.0, kChainSetup = 300.0, kBlockCost = 200.0;
+    constexpr u32 K = esl::kRedCells;
     o.red.clear();
+    o.red_h.clear();
     o.red_off.clear();
     o.red_len.clear();
     o.rc_head.clear();
@@ -2058,64 +2052,87 @@ void build_reduce_streams(const Compiled &c, TapeHostProg &o)
     o.rc_coff.clear();
     o.rc_blocks.clear();
     const size_t nch = c.chunks.size() - 1;
-    for (size_t ci = 0; ci < nch; ci++) {
+    const u32 n = c.n, n_tv = o.prog.n_tv, ncs = (u32)c.cslot_pat.size();
+    for (size_t si = 0; si < 2 * nch; si++) {
+        const size_t ci = si / 2;
+        const bool tran = si % 2 != 0;
         const u32 t0 = c.chunks[ci].task_begin, t1 = c.chunks[ci + 1].task_begin;
         vector<u32> order;
         for (u32 t = t0; t < t1; t++)
-            if (!(c.task_target[t] & (esl::kCBit | esl::kQBit))) order.push_back(t);
-        auto len = [&](u32 t) { return 1 + c.task_cell[t + 1] - c.task_cell[t]; };
-        std::stable_sort(order.begin(), order.end(), [&](u32 a, u32 b) { return len(a) > len(b); });
-        auto word_of = [&](u32 t) {
-            const u32 tg = c.task_target[t];
-            return (tg & esl::kRhsBit) ? (esl::kRedTarget | esl::kRedRhs | (tg & ~esl::kRhsBit))
-                                       : (esl::kRedTarget | o.amap[tg]);
+            if (tran || !(c.task_target[t] & (esl::kCBit | esl::kQBit))) order.push_back(t);
+        auto cells_of = [&](u32 t) { return c.task_cell[t + 1] - c.task_cell[t]; };
+        std::stable_sort(order.begin(), order.end(), [&](u32 a, u32 b) { return cells_of(a) > cells_of(b); });
+        // a target in the working set [factor slots | ... rhs | x | q | cq]:
+        // below n_tv a slot, else n_tv + its distance from rhs
+        auto place = [&](u32 t) {
+            const u32 tg = c.task_target[t], idx = tg & esl::kTargetMask;
+            if (tg & esl::kRhsBit) return n_tv + idx;
+            if (tg & esl::kQBit) return n_tv + 2 * n + idx;
+            if (tg & esl::kCBit) return n_tv + 3 * n + idx;
+            return o.amap[tg];
         };
-        // the stream rows of the tasks from `first` on, dealt longest first
-        // to the least loaded thread
-        auto deal = [&](size_t first, vector<vector<u32>> *words) {
-            vector<size_t> load(esl::kWave, 0);
+        // rows of the tasks from `first` on: each row takes the targets with
+        // most words left
+        auto rows_of = [&](size_t first, vector<vector<std::pair<u32, u32>>> *rows) {   // (task, word)
+            vector<u32> left, at;
+            size_t words = 0;
             for (size_t k = first; k < order.size(); k++) {
-                const u32 t = order[k];
-                size_t best = 0;
-                for (size_t w = 1; w < load.size(); w++)
-                    if (load[w] < load[best]) best = w;
-                load[best] += len(t);
-                if (words) {
-                    (*words)[best].push_back(word_of(t));
-                    for (u32 cc = c.task_cell[t]; cc < c.task_cell[t + 1]; cc++) (*words)[best].push_back(c.cells[cc]);
-                }
+                left.push_back((cells_of(order[k]) + K - 1) / K);
+                words += left.back();
             }
-            size_t L = 0;
-            for (size_t v : load) L = std::max(L, v);
-            return (L + esl::kRing - 1) / esl::kRing * esl::kRing;
+            if (!rows) return std::max<size_t>((words + esl::kWave - 1) / esl::kWave, left.empty() ? 0 : left[0]);
+            at.assign(left.size(), 0);
+            for (size_t done = 0; done < words;) {
+                vector<u32> pick;
+                for (u32 k = 0; k < left.size(); k++)
+                    if (left[k]) pick.push_back(k);
+                std::stable_sort(pick.begin(), pick.end(), [&](u32 a, u32 b) { return left[a] > left[b]; });
+                if (pick.size() > (size_t)esl::kWave) pick.resize(esl::kWave);
+                vector<std::pair<u32, u32>> row;
+                for (u32 k : pick) {
+                    row.push_back({order[first + k], at[k]++});
+                    left[k]--;
+                }
+                done += row.size();
+                rows->push_back(std::move(row));
+            }
+            return rows->size();
         };
-        // chains: the k longest tasks whose indices fit the pads; a task of
-        // few cells never pays
+        // chains: the k longest tasks on slots or rhs whose indices fit the
+        // pads; a task of few cells never pays
         auto aligned = [](u32 cells) { return (cells + esl::kChainBlk - 1) / esl::kChainBlk * esl::kChainBlk; };
         size_t best_k = 0;
-        double best_cost = kStepCost * (double)deal(0, nullptr);
+        double best_cost = kRowCost * (double)rows_of(0, nullptr);
         // every chain thread reads the longest chain's blocks from its own
         // offset on: the last chain's offset plus those must fit the pads
         u32 at_last = 0;
-        for (size_t k = 1; k <= std::min<size_t>(order.size(), esl::kWave) && len(order[k - 1]) > 2 * esl::kRing;
-             k++) {
-            if (k > 1) at_last += aligned(len(order[k - 2]) - 1);
-            if (at_last + aligned(len(order[0]) - 1) > esl::kRedChainCells) break;
-            const double blocks = (double)aligned(len(order[0]) - 1) / esl::kChainBlk;
-            const double cost = kStepCost * (double)deal(k, nullptr) + kChainSetup + kBlockCost * blocks;
+        for (size_t k = 1; k <= std::min<size_t>(order.size(), esl::kWave) && cells_of(order[k - 1]) > 16; k++) {
+            if (c.task_target[order[k - 1]] & (esl::kCBit | esl::kQBit)) break;
+            if (k > 1) at_last += aligned(cells_of(order[k - 2]));
+            if (at_last + aligned(cells_of(order[0])) > esl::kRedChainCells) break;
+            const double blocks = (double)aligned(cells_of(order[0])) / esl::kChainBlk;
+            const double cost = kRowCost * (double)rows_of(k, nullptr) + kChainSetup + kBlockCost * blocks;
             if (cost < best_cost) {
                 best_cost = cost;
                 best_k = k;
             }
         }
-        vector<vector<u32>> words(esl::kWave);
-        const size_t L = deal(best_k, &words);
+        vector<vector<std::pair<u32, u32>>> rows;
+        rows_of(best_k, &rows);
+        const size_t L = (rows.size() + esl::kRedRing - 1) / esl::kRedRing * esl::kRedRing;
         o.red_off.push_back((u32)o.red.size());
         o.red_len.push_back((u32)L);
+        const u32 idle = n_tv + (tran ? 3 * n + ncs : 2 * n);
         const size_t base = o.red.size();
-        o.red.resize(base + (L + esl::kRing) * esl::kWave, esl::red_pad(c.n));
-        for (size_t t = 0; t < words.size(); t++)
-            for (size_t w = 0; w < words[t].size(); w++) o.red[base + w * esl::kWave + t] = words[t][w];
+        o.red.resize(base + (L + esl::kRedRing) * esl::kWave,
+                     esl::uint2_t{idle | (esl::kRedNone << 16), esl::kRedNone | (esl::kRedNone << 16)});
+        for (size_t r = 0; r < rows.size(); r++)
+            for (size_t th = 0; th < rows[r].size(); th++) {
+                const u32 t = rows[r][th].first, c0 = c.task_cell[t] + rows[r][th].second * K;
+                u32 cl[K];
+                for (u32 e = 0; e < K; e++) cl[e] = c0 + e < c.task_cell[t + 1] ? c.cells[c0 + e] : esl::kRedNone;
+                o.red[base + r * esl::kWave + th] = esl::uint2_t{place(t) | (cl[0] << 16), cl[1] | (cl[2] << 16)};
+            }
         // the chains' headers {target word, cells | index offset << 16}, one
         // per thread, and their indices as kRedChainCells 16-bit values
         // (two per word; unused ones 0, a valid staging index)
@@ -2128,8 +2145,10 @@ void build_reduce_streams(const Compiled &c, TapeHostProg &o)
             o.rc_cells.resize(cb + esl::kRedChainCells / 2, 0u);
             u32 at = 0;
             for (size_t k = 0; k < best_k; k++) {
-                const u32 task = order[k], cells = len(task) - 1;
-                o.rc_head.push_back(esl::uint2_t{word_of(task), cells | (at << 16)});
+                const u32 task = order[k], cells = cells_of(task), tg = c.task_target[task];
+                const u32 word = (tg & esl::kRhsBit) ? (esl::kRedTarget | esl::kRedRhs | (tg & ~esl::kRhsBit))
+                                                     : (esl::kRedTarget | o.amap[tg]);
+                o.rc_head.push_back(esl::uint2_t{word, cells | (at << 16)});
                 for (u32 j = 0; j < cells; j++) {
                     const u32 cell = c.cells[c.task_cell[task] + j];
                     o.rc_cells[cb + (at + j) / 2] |= ((at + j) % 2) ? (cell << 16) : cell;
@@ -2139,7 +2158,11 @@ void build_reduce_streams(const Compiled &c, TapeHostProg &o)
             }
         }
         o.rc_blocks.push_back(blocks);
+        const esl::Chunk &ch = c.chunks[ci];
+        o.red_h.push_back({o.red_off.back(), (u32)L | ((u32)best_k << 16), o.rc_off.back(), o.rc_coff.back() | (blocks << 26)});
+        o.red_h.push_back({ch.kind, ch.first, ch.count, 0u});
     }
+    o.red_h.resize(o.red_h.size() + 4, esl::uint4_t{0, 0, 0, 0});   // the last chunk's read ahead
     o.diag_tv.assign(c.n, 0);
     for (u32 i = 0; i < c.n; i++) o.diag_tv[i] = o.amap[c.diag[i]];
 }
@@ -2182,7 +2205,7 @@ bool validate_big(const TapeHostProg &o, u32 n, u32 W = esl::kTeamThreads)
     }
     return true;
 }
-bool validate_tape(const TapeHostProg &o, u32 n, u32 nnz)
+bool validate_tape(const TapeHostProg &o, u32 n, u32 nnz, u32 ncs = 0)
 {
     const esl::TapeProg &P = o.prog;
     if (o.amap.size() != nnz || o.pinv.size() != n || o.qinv.size() != n || o.flags.size() != n) return false;
@@ -2285,15 +2308,24 @@ bool validate_tape(const TapeHostProg &o, u32 n, u32 nnz)
     if (!rows_ok(o.rch, false) || !rows_ok(o.sch, true)) return false;
     for (u32 v : o.rsrc) if (v >= P.n_tv) return false;
     if (!o.red_off.empty()) {
-        if (o.red_len.size() != o.red_off.size()) return false;
-        for (size_t ci = 0; ci < o.red_off.size(); ci++) {
-            if ((size_t)o.red_off[ci] + (size_t)(o.red_len[ci] + esl::kRing) * esl::kWave > o.red.size()) return false;
-            if (o.red_len[ci] % esl::kRing) return false;
+        // up to the transient's scratch double, and 16-bit targets
+        const u32 lim = P.n_tv + 3 * n + ncs;
+        if (o.red_len.size() != o.red_off.size() || o.red_off.size() % 2 || lim >= 0xffff) return false;
+        if (o.red_h.size() != 2 * o.red_off.size() + 4 || o.rc_cells.size() >= (1u << 26)) return false;
+        for (size_t si = 0; si < o.red_off.size(); si++) {
+            const u32 top = si % 2 ? lim : P.n_tv + 2 * n;   // the idle threads' scratch double
+            const size_t rows = (size_t)o.red_len[si] + esl::kRedRing;
+            if (o.red_len[si] > 0xffff || o.red_len[si] % esl::kRedRing || o.red_off[si] + rows * esl::kWave > o.red.size()) return false;
+            for (size_t k = o.red_off[si]; k < o.red_off[si] + rows * esl::kWave; k++) {
+                const u32 cl[3] = {o.red[k].x >> 16, o.red[k].y & 0xffff, o.red[k].y >> 16};
+                if ((o.red[k].x & 0xffff) > top) return false;
+                for (u32 v : cl)
+                    if (v >= esl::kStageDoubles && v != esl::kRedNone) return false;
+            }
         }
-        if (2 * n > 0xfffff) return false;
         auto target_ok = [&](u32 w) {
             const u32 idx = w & 0xfffff;
-            if ((w & esl::kRedRhs) ? (idx >= n && w != esl::red_pad(n)) : idx >= P.n_tv) return false;
+            if ((w & esl::kRedRhs) ? idx >= n : idx >= P.n_tv) return false;
             return (w & ~(esl::kRedTarget | esl::kRedRhs)) <= 0xfffff;
         };
         const size_t nch = o.red_off.size();
@@ -2320,15 +2352,6 @@ bool validate_tape(const TapeHostProg &o, u32 n, u32 nnz)
             if ((w & 0xffff) >= (u32)(esl::kWave * esl::kStageEntries) ||
                 (w >> 16) >= (u32)(esl::kWave * esl::kStageEntries))
                 return false;
-        for (u32 w : o.red) {
-            if (w & esl::kRedTarget) {
-                const u32 idx = w & 0xfffff;
-                if ((w & esl::kRedRhs) ? (idx >= n && w != esl::red_pad(n)) : idx >= P.n_tv) return false;
-                if ((w & ~(esl::kRedTarget | esl::kRedRhs)) > 0xfffff) return false;
-            } else if (w >= (u32)(esl::kWave * esl::kStageEntries)) {
-                return false;
-            }
-        }
     }
     return true;
 }
@@ -2441,7 +2464,7 @@ TapeHostProg *build_tape(const Engine &e, const HostTape &t, const char *&err)
         for (u32 k = 0; k < e.c.res_total; k++)
             tp->rsrc[k] = e.c.res_p[k] == esl::kNoSlot ? tp->prog.pad_slot : tp->amap[e.c.res_p[k]];
     }
-    if (!err && !validate_tape(*tp, n, e.c.nnz)) err = "tape program failed validation";
+    if (!err && !validate_tape(*tp, n, e.c.nnz, (u32)e.c.cslot_pat.size())) err = "tape program failed validation";
     // the residual's chain rows use the FP64 pads while the factors are FP32
     if (!err && !tp->big && !e.c.res_ch.empty() && 2 * (size_t)(tp->prog.n_tv - esl::kWave) < (size_t)tp->prog.n_tv + n)
         err = "tape program failed validation";
@@ -4201,7 +4224,7 @@ void model_job_ns(const BatchItemRun &r, double out[2])
     auto rows = [&](u32 tape) {
         const TapeHostProg &t = *e.tapes[tape];
         double red = 0;
-        for (u32 v : t.red_len) red += v;
+        for (size_t k = 0; k < t.red_len.size(); k += 2) red += t.red_len[k];
         return (double)t.prog.rw_rows + t.prog.sw_rows + red;
     };
     const double chunks = (double)e.c.chunks.size() - 1;

@@ -167,14 +167,71 @@ __device__ inline void add_gmin(double g, const DeckProg &dp, const uint32_t *di
     wsync();
 }
 
-// The LDS double a reduce word reads, without a branch: a target word its
-// factor slot or rhs row (padding words: the lane's scratch double at
-// rhs + 2n), a cell word its staged cell. Branch-free, so the reads of the
-// words ahead stay in flight together.
-__device__ inline double *red_src(uint32_t w, double *tv, double *rhs, double *stc)
+// The LDS double a chain header names.
+__device__ inline double *red_src(uint32_t w, double *tv, double *rhs)
 {
-    double *tb = (w & kRedRhs) ? rhs : tv;
-    return ((int32_t)w < 0 ? tb : stc) + (w & 0xfffffu);
+    return ((w & kRedRhs) ? rhs : tv) + (w & 0xfffffu);
+}
+
+// a tape descriptor in the tape table: fields through the scalar cache (a
+// copy whose address is passed on would live in scratch memory)
+typedef const __attribute__((address_space(4))) TapeProg *ctape;
+
+// A stream's header, read a chunk ahead (its words' address, and the chunk
+// itself, would otherwise wait for a chain of loads), and its first rows,
+// read before the chunk's evaluation.
+struct RedStream {
+    esl::uint4_t a, b;
+    const __attribute__((address_space(1))) esl::uint2_t *w;
+    esl::uint2_t q[kRedRing];
+    uint32_t len;
+};
+__device__ inline void red_head(RedStream &r, ctape T, uint32_t s)
+{
+    const __attribute__((address_space(1))) esl::uint4_t *h = gptr(T->red_h) + 2 * s;
+    r.a = esl::uint4_t{h[0].x, h[0].y, h[0].z, h[0].w};
+    r.b = esl::uint4_t{h[1].x, h[1].y, h[1].z, h[1].w};
+}
+__device__ inline Chunk red_chunk(const RedStream &r) { return Chunk{uni(r.b.x), uni(r.b.y), uni(r.b.z), 0u}; }
+__device__ inline void red_load(RedStream &r, ctape T, uint32_t tid)
+{
+    r.len = uni(r.a.y) & 0xffffu;
+    r.w = gptr(T->red) + uni(r.a.x) + tid;
+#pragma unroll
+    for (int k = 0; k < kRedRing; k++) r.q[k] = esl::uint2_t{r.w[k * kWave].x, r.w[k * kWave].y};
+}
+
+// Runs a stream on the staged cells at st0 (LDS addresses; tv0: the factor
+// slots, rhs8: what a rhs-side index adds to its slot number's address,
+// none: the double holding -0, above every staging cell). A row is bound by
+// its target's LDS round trip and three dependent adds, for up to three
+// cells a thread, where a stream of one word a cell took a round trip for
+// each cell. With the headers read a chunk ahead, cycles an iteration:
+// assembly of the 64-OTA array 106.9 k -> 86.3 k, of the mirror tree of
+// depth 6 109.6 k -> 66.9 k, of 8 diodes 15.9 k -> 9.9 k; the transient of
+// 16 bipolar pairs, whose reduce walked task tables, 7.28 -> 6.42 ms.
+__device__ inline void red_rows(RedStream &r, uint32_t tv0, uint32_t n_tv, uint32_t rhs8, uint32_t st0, uint32_t none)
+{
+    using lp = __attribute__((address_space(3))) double *;
+    auto cell = [&](uint32_t c) {
+        const uint32_t a = st0 + c * 8u;
+        return *(lp)(uintptr_t)(a < none ? a : none);
+    };
+    for (uint32_t row = 0; row < r.len; row += kRedRing) {
+        r.w += kRedRing * kWave;
+#pragma unroll
+        for (int k = 0; k < kRedRing; k++) {
+            const esl::uint2_t w = r.q[k];
+            const uint32_t t = w.x & 0xffffu;
+            const lp d = (lp)(uintptr_t)(tv0 + t * 8u + (t >= n_tv ? rhs8 : 0u));
+            const double v = *d, a0 = cell(w.x >> 16), a1 = cell(w.y & 0xffffu), a2 = cell(w.y >> 16);
+            r.q[k] = esl::uint2_t{r.w[k * kWave].x, r.w[k * kWave].y};
+            double acc = v + a0;
+            acc = acc + a1;
+            acc = acc + a2;
+            *d = acc;
+        }
+    }
 }
 
 // The reduce chains of a chunk: thread k < chains adds its chain's cells
@@ -192,7 +249,7 @@ __device__ inline void red_chains(esl::uint2_t hd, uint32_t nb, const uint32_t *
     const uint32_t len = hd.y & 0xffffu;
     const __attribute__((address_space(3))) uint32_t *ip = lptr(pw) + (hd.y >> 17);
     const __attribute__((address_space(3))) double *sv = lptr(stc);
-    double *tgt = red_src(hd.x, tv, rhs, stc);
+    double *tgt = red_src(hd.x, tv, rhs);
     auto idx = [&](uint32_t b, uint32_t (&ws)[4]) {
 #pragma unroll
         for (int q = 0; q < 4; q++) ws[q] = ip[4 * b + q];
@@ -224,98 +281,75 @@ __device__ inline void red_chains(esl::uint2_t hd, uint32_t nb, const uint32_t *
     *tgt = acc;
 }
 
-// Assembly into the tape's factor slots: every chunk evaluates, then each
-// thread runs its reduce words (coalesced rows, 16 rows in flight), adding
-// each target's cells in instance order into a register. A crew of nw
+// One stream of a staged chunk: its rows, then its chains. idle: the header
+// of a thread without a chain (the scratch double).
+__device__ inline void red_stream(RedStream &r, ctape T, double *tv, double *rhs, double *stc, uint32_t none,
+                                  uint32_t idle, uint32_t tid)
+{
+    using lp = __attribute__((address_space(3))) double *;
+    const uint32_t tv0 = (uint32_t)(uintptr_t)(lp)tv, rhs0 = (uint32_t)(uintptr_t)(lp)rhs;
+    // the chains' cell indices load now, ahead of use
+    const uint32_t nc = uni(r.a.y) >> 16;
+    uint32_t tw0 = 0u, tw1 = 0u;
+    esl::uint2_t hd{idle, 0u};
+    if (nc) {
+        const __attribute__((address_space(1))) uint32_t *cg = gptr(T->rc_cells) + (uni(r.a.w) & 0x3ffffffu) + tid;
+        tw0 = cg[0];
+        tw1 = cg[kWave];
+        if (tid < nc) {
+            const __attribute__((address_space(1))) esl::uint2_t &h = gptr(T->rc_head)[uni(r.a.z) + tid];
+            hd = esl::uint2_t{h.x, h.y};
+        }
+    }
+    red_rows(r, tv0, T->n_tv, rhs0 - tv0 - T->n_tv * 8u, (uint32_t)(uintptr_t)(lp)stc, none);
+    if (nc) {
+        // the pad slots take the indices (the rows above use no pad)
+        uint32_t *pw = reinterpret_cast<uint32_t *>(tv + T->pad_slot);
+        pw[tid] = tw0;
+        pw[kWave + tid] = tw1;
+        wsync();
+        red_chains(hd, uni(r.a.w) >> 26, pw, tv, rhs, stc);
+    }
+}
+
+// Assembly into the tape's factor slots: every chunk evaluates, then its
+// reduce stream adds each target's cells in instance order. A crew of nw
 // wavefronts evaluates nw chunks per round.
-__device__ void assemble(const DeckProg &dp, const TapeProg &T, const double *live, const double *x, double *lim,
+__device__ void assemble(const DeckProg &dp, ctape T, const double *live, const double *x, double *lim,
                          uint32_t lim_stride, double *tv, double *rhs, double *st, uint32_t tid, const Crew &cr,
                          double src = 1.0)
 {
     const uint32_t n = dp.n;
-    for (uint32_t i = tid; i < T.n_tv; i += kWave) tv[i] = 0.0;
+    for (uint32_t i = tid; i < T->n_tv; i += kWave) tv[i] = 0.0;
     for (uint32_t i = tid; i < n; i += kWave) rhs[i] = 0.0;
+    if (tid == 0) rhs[2 * n + 1] = -0.0;
+    using lp = __attribute__((address_space(3))) double *;
+    const uint32_t none = (uint32_t)(uintptr_t)(lp)(rhs + 2 * n + 1);
+    const uint32_t idle = kRedTarget | kRedRhs | (2 * n);
     wsync();
+    RedStream r;
+    red_head(r, T, 0);
     for (uint32_t c0 = 0; c0 < dp.n_chunks; c0 += cr.nw) {
+        const Chunk ch = red_chunk(r);
+        red_load(r, T, tid);
         if (cr.nw > 1) crew_post(cr, c0, false, 0.0, tid, src);
-        eval_chunk(dp, dp.chunks[c0], live, x, lim, lim_stride, st, tid, 0.0, false, src);   // capacitors stage nothing here
+        // capacitors stage nothing here
+        if (ch.kind != kC) eval_chunk(dp, ch, live, x, lim, lim_stride, st, tid, 0.0, false, src);
         if (cr.nw > 1) __syncthreads();
         else wsync();
         const uint32_t c1 = c0 + cr.nw < dp.n_chunks ? c0 + cr.nw : dp.n_chunks;
         for (uint32_t c = c0; c < c1; c++) {
-            if (dp.chunks[c].kind == kC) continue;   // no static stamps
-            double *stc = st + (c - c0) * kStageDoubles;
-            // the stream through a global pointer: its ring of loads must
-            // not hold up the LDS waits of the reduce (flat loads would)
-            const __attribute__((address_space(1))) uint32_t *rs = gptr(T.red) + T.red_off[c] + tid;
-            const uint32_t len = T.red_len[c];
-            // the chains' headers and cell indices load now, ahead of use
-            const uint32_t nc = T.rc_count[c];
-            uint32_t tw0 = 0u, tw1 = 0u;
-            esl::uint2_t hd{red_pad(n), 0u};
-            if (nc) {
-                const __attribute__((address_space(1))) uint32_t *cg = gptr(T.rc_cells) + T.rc_coff[c] + tid;
-                tw0 = cg[0];
-                tw1 = cg[kWave];
-                if (tid < nc) {
-                    const __attribute__((address_space(1))) esl::uint2_t &h = gptr(T.rc_head)[T.rc_off[c] + tid];
-                    hd = esl::uint2_t{h.x, h.y};
-                }
-            }
-            uint32_t q[kRing];
-#pragma unroll
-            for (int k = 0; k < kRing; k++) {
-                q[k] = rs[k * kWave];
-                __builtin_amdgcn_sched_barrier(0);
-            }
-            // Each word's value is read kAhead words before its use, so a
-            // long target's chain of adds waits on the adds, not on an LDS
-            // round trip each. The running sum is stored to the current
-            // target at every word (its final value at the switch to the
-            // next target): a chunk gives each target to one thread, once,
-            // so no other read sees the partial sums. The sums are the
-            // instance-ordered ones of the serial assembly.
-            constexpr int kAhead = kRing / 2;
-            double va[kAhead];
-            double *pa[kAhead];
-#pragma unroll
-            for (int k = 0; k < kAhead; k++) {
-                pa[k] = red_src(q[k], tv, rhs, stc);
-                va[k] = *pa[k];
-            }
-            double *cur = rhs + 2 * n;   // the scratch double
-            double acc = 0.0;
-            for (uint32_t w = 0; w < len; w += kRing) {
-#pragma unroll
-                for (int k = 0; k < kRing; k++) {
-                    const double v = va[k % kAhead];
-                    double *p = pa[k % kAhead];
-                    const bool tgt = (int32_t)q[k] < 0;
-                    *cur = acc;
-                    cur = tgt ? p : cur;
-                    acc = tgt ? v : acc + v;
-                    // word w + k + kAhead: still in the ring (k < kAhead), or
-                    // the refill of the slot used kAhead words ago
-                    pa[k % kAhead] = red_src(q[(k + kAhead) % kRing], tv, rhs, stc);
-                    va[k % kAhead] = *pa[k % kAhead];
-                    q[k] = rs[(w + kRing + k) * kWave];
-                    __builtin_amdgcn_sched_barrier(0);
-                }
-            }
-            *cur = acc;
-            if (nc) {
-                // the pad slots take the indices (the stream above reads no pad)
-                uint32_t *pw = reinterpret_cast<uint32_t *>(tv + T.pad_slot);
-                pw[tid] = tw0;
-                pw[kWave + tid] = tw1;
-                wsync();
-                red_chains(hd, T.rc_blocks[c], pw, tv, rhs, stc);
-            }
+            if (c != c0) red_load(r, T, tid);
+            RedStream nx;
+            red_head(nx, T, 2 * (c + 1));
+            red_stream(r, T, tv, rhs, st + (c - c0) * kStageDoubles, none, idle, tid);
+            r.a = nx.a;
+            r.b = nx.b;
             wsync();
         }
     }
     if (tid == 0) {
-        const uint32_t s0 = T.diag_tv[0];
+        const uint32_t s0 = T->diag_tv[0];
         tv[s0] = tv[s0] + 1.0;
         rhs[0] = rhs[0] + x[0];
     }
@@ -700,6 +734,7 @@ __device__ __forceinline__ uint32_t op_lane(const OpArgs &a, uint32_t lane, doub
     const bool can_priv = kOwnLU && a.priv.cap != 0 && !fp32;
     bool priv = kOwnLU && rs.tape == kPrivTape;
     const TapeProg T = a.tapes[priv ? 0 : rs.tape];   // unused while the lane is on its own LU
+    const ctape Tc = (ctape)(a.tapes + (priv ? 0 : rs.tape));
     double *pap = a.priv.ap + (size_t)lane * dp.nnz;  // the lane's Jacobian for its own LU (pattern order)
     // FP64 solve vector; in FP32 lanes and on the lane's own LU, dx in row order
     double *y = priv ? tv + a.tv_cap : tv + T.n_tv;
@@ -780,7 +815,7 @@ __device__ __forceinline__ uint32_t op_lane(const OpArgs &a, uint32_t lane, doub
             assemble_pattern(dp, live, x, lim, nm, pap, rhs, st, tid, lam);
             add_gmin(g_run, dp, dp.diag_slot, pap, rhs, x, tid);
         } else {
-            assemble(dp, T, live, x, lim, nm, tv, rhs, st, tid, cr, lam);
+            assemble(dp, Tc, live, x, lim, nm, tv, rhs, st, tid, cr, lam);
             add_gmin(g_run, dp, T.diag_tv, tv, rhs, x, tid);
         }
         if (warm == 1) {
@@ -1029,36 +1064,56 @@ __global__ __launch_bounds__(kWave) void op_newton_own(OpArgs a)
 // (src/device/eval.zig:782-922 with the charge planes of LaneSink), the
 // ground pin, then A = G + ag0 C and F += ag0 (q - q1) - ag1 i_prev
 // (lane_kernels.zig:194-215). q1 and i_prev are the lane's rows in global
-// memory. Jacobian entries go to tv[amap[slot]] (amap null: tv[slot], the
-// pattern order). A crew of nw wavefronts evaluates nw chunks per round.
-__device__ void assemble_tran(const DeckProg &dp, const uint32_t *amap, uint32_t n_slots, const double *live,
+// memory. Jacobian entries go to the tape's slots (T null: tv[slot], the pattern
+// order, by the deck's reduce tasks). A crew of nw wavefronts evaluates nw
+// chunks per round.
+__device__ __forceinline__ void assemble_tran(const DeckProg &dp, ctape T, uint32_t n_slots, const double *live,
                               const double *x, double *lim, uint32_t nm, double *tv, double *rhs, double *q,
                               double *cq, double *st, double t, double ag0, double ag1, const double *q1,
                               const double *ip, uint32_t tid, const Crew &cr)
 {
     const uint32_t n = dp.n;
+    const uint32_t *amap = T ? T->amap : nullptr;
     for (uint32_t i = tid; i < n_slots; i += kWave) tv[i] = 0.0;
     for (uint32_t i = tid; i < n; i += kWave) {
         rhs[i] = 0.0;
         q[i] = 0.0;
     }
     for (uint32_t k = tid; k < dp.n_cslot; k += kWave) cq[k] = 0.0;
+    // the reduce streams' scratch pair follows cq
+    if (T && tid == 0) cq[dp.n_cslot + 1] = -0.0;
+    using lp = __attribute__((address_space(3))) double *;
+    const uint32_t none = (uint32_t)(uintptr_t)(lp)(cq + dp.n_cslot + 1);
+    const uint32_t idle = kRedTarget | kRedRhs | (3 * n + dp.n_cslot);
     wsync();
+    RedStream r;
+    if (T) red_head(r, T, 1);
     for (uint32_t c0 = 0; c0 < dp.n_chunks; c0 += cr.nw) {
+        const Chunk ch = T ? red_chunk(r) : dp.chunks[c0];
+        if (T) red_load(r, T, tid);
         if (cr.nw > 1) crew_post(cr, c0, true, t, tid);
-        eval_chunk(dp, dp.chunks[c0], live, x, lim, nm, st, tid, t, true);
+        eval_chunk(dp, ch, live, x, lim, nm, st, tid, t, true);
         if (cr.nw > 1) __syncthreads();
         else wsync();
         const uint32_t c1 = c0 + cr.nw < dp.n_chunks ? c0 + cr.nw : dp.n_chunks;
         for (uint32_t c = c0; c < c1; c++) {
-            const double *stc = st + (c - c0) * kStageDoubles;
-            const uint32_t t1 = dp.chunks[c + 1].task_begin;
-            for (uint32_t k = dp.chunks[c].task_begin + tid; k < t1; k += kWave) {
-                const uint32_t tgt = dp.task_target[k];
-                const uint32_t idx = tgt & kTargetMask;
-                double *d = (tgt & kRhsBit) ? &rhs[idx] : (tgt & kQBit) ? &q[idx] : (tgt & kCBit) ? &cq[idx]
-                                                                                                   : &tv[amap ? amap[tgt] : tgt];
-                *d = add_cells(*d, stc, dp.cells, dp.task_cell[k], dp.task_cell[k + 1]);
+            double *stc = st + (c - c0) * kStageDoubles;
+            if (T) {
+                if (c != c0) red_load(r, T, tid);
+                RedStream nx;
+                red_head(nx, T, 2 * (c + 1) + 1);
+                red_stream(r, T, tv, rhs, stc, none, idle, tid);
+                r.a = nx.a;
+                r.b = nx.b;
+            } else {
+                const uint32_t t1 = dp.chunks[c + 1].task_begin;
+                for (uint32_t k = dp.chunks[c].task_begin + tid; k < t1; k += kWave) {
+                    const uint32_t tgt = dp.task_target[k];
+                    const uint32_t idx = tgt & kTargetMask;
+                    double *d = (tgt & kRhsBit) ? &rhs[idx] : (tgt & kQBit) ? &q[idx] : (tgt & kCBit) ? &cq[idx]
+                                                                                                       : &tv[tgt];
+                    *d = add_cells(*d, stc, dp.cells, dp.task_cell[k], dp.task_cell[k + 1]);
+                }
             }
             wsync();
         }
@@ -1206,6 +1261,7 @@ __device__ __forceinline__ void tran_lane(const TranArgs &ta, uint32_t lane, dou
     const bool can_priv = kOwnLU && a.priv.cap != 0;
     bool priv = kOwnLU && rs.tape == kPrivTape;
     const TapeProg T = a.tapes[priv ? 0 : rs.tape];   // unused while the lane is on its own LU
+    const ctape Tc = (ctape)(a.tapes + (priv ? 0 : rs.tape));
     double *pap = a.priv.ap + (size_t)lane * dp.nnz;  // the lane's Jacobian for its own LU (pattern order)
     double *y = priv ? tv + a.tv_cap : tv + T.n_tv;
     bool staged = true;
@@ -1224,7 +1280,7 @@ __device__ __forceinline__ void tran_lane(const TranArgs &ta, uint32_t lane, dou
     // the lane's own LU
     auto assemble_step = [&](bool own, double tt, double g0, double g1) {
         if (own) assemble_tran(dp, nullptr, dp.nnz, live, x, lim, nm, pap, rhs, q, cq, st, tt, g0, g1, q1, ip, tid, cr);
-        else assemble_tran(dp, T.amap, T.n_tv, live, x, lim, nm, tv, rhs, q, cq, st, tt, g0, g1, q1, ip, tid, cr);
+        else assemble_tran(dp, Tc, T.n_tv, live, x, lim, nm, tv, rhs, q, cq, st, tt, g0, g1, q1, ip, tid, cr);
     };
     for (uint32_t i = tid; i < n; i += kWave) x[i] = a.x[(size_t)lane * n + i];
     wsync();
