@@ -3377,7 +3377,15 @@ extern "C" esl_status esl_op_solve(esl_engine *h, const double *values, size_t c
     // Tiling: explicit, or the autotuner's choice. The autotuner times both
     // tilings once per engine on the first batch of at least 1024 points
     // (kernel time of the first launch over every lane) and keeps the faster;
-    // below that size a batch runs one wavefront per lane.
+    // below that size a batch runs one wavefront per lane. So does a batch
+    // whose trial could not end otherwise: the thread tiling's time hardly
+    // depends on the count (its lanes wait on HBM) and grows with the
+    // unknowns. At 16,384 points, against the wavefront tiling: 0.17 to 0.67
+    // ms at 5 unknowns, 1.30 to 1.38 at 19, but 5.0 to 1.8 at 43, 9.4 to 2.3
+    // at 61 and 210 to 10 at 324: a factor of 4 and more past 48, which twice
+    // as many points do not turn (and the trial cost that first batch 200 ms).
+    constexpr u32 kThreadMost = 48;
+    constexpr size_t kThreadPoints = 32768;
     // the thread tiling runs FP64 lanes from cold or given starts
     // the .op ladder runs on the device in the wavefront kernels (FP64 lanes)
     const bool ladder = (o.flags & ESL_OP_LADDER) && !fp32 && !e->big;
@@ -3401,7 +3409,7 @@ extern "C" esl_status esl_op_solve(esl_engine *h, const double *values, size_t c
     } else if (tiling == ESL_TILING_AUTO) {
         if (e->tuned) {
             tiling = e->tuned;
-        } else if (count >= 1024) {
+        } else if (count >= 1024 && (n <= kThreadMost || count > kThreadPoints)) {
             float ms_w = 0, ms_t = 0;
             if (launch_lpw(*e, a, (u32)count, mode0, lead_cap, ms_w) != ESL_OK) return ESL_DEVICE_UNAVAILABLE;
             HIPCHK(hipMemcpyAsync(e->resume.p, rs.data(), count * sizeof(esl::LaneResume), hipMemcpyHostToDevice, s));
