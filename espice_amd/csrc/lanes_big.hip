@@ -253,6 +253,9 @@ __device__ bool big_refactor(const TapeProg &T, uint32_t n, gdbl *tv, const BigL
     gcu32 *flags = gptr(T.flags), *amap = gptr(T.amap), *void_slots = gptr(T.void_slots);
     LuFlags f{false, 0, 0};
     for (uint32_t v = tid; v < T.n_void; v += kTeamThreads) f.bad |= tv[amap[void_slots[v]]] != 0.0;
+    // a void column's own diagonal is among the void slots: every wavefront
+    // has read it before any sets it
+    if (T.n_void) __syncthreads();
     for (uint32_t k = tid; k < n; k += kTeamThreads)
         if (flags[k] & kVoidBit) tv[T.n_u + k] = 1.0;
     __syncthreads();

@@ -81,3 +81,28 @@ def test_mesh_rejects_fp32_and_batches(lanes, mesh):
         eng.solve_op(vals, precision=lanes.FP32_REFINED)
     with pytest.raises(lanes.EslError):
         lanes.solve_batch([{"engine": eng, "values": vals}])
+
+
+def test_void_unknowns_of_a_big_lane_bitwise(lanes, oracle):
+    """Nodes that only capacitors touch are void in the operating point:
+    their columns and rows hold zeros and their pivots are set to 1 after
+    the replay has found those zeros. 200 of them, so that the slots are
+    read by other wavefronts than set them: every lane keeps its first
+    pivots, bitwise the oracle's, and steps on from there."""
+    fam = circuits.rc_mesh(40)
+    d = fam.deck
+    for k in range(200):
+        d.capacitor(f"cv{k}", f"v{k}", f"v{k + 1}" if k % 3 else 0, 1e-14)
+    vals = fam.sample(17, 5)
+    eng = lanes.Engine(d.arrays())
+    _, _, q = eng.pattern()
+    say(f"mesh 40x40 and 200 void unknowns, n {eng.n}, 5 lanes")
+    got = eng.solve_op(vals)
+    tm = eng.timing()
+    c = oracle.Circuit(d.arrays())
+    ref = c.op(vals, q, threads=5)
+    assert tm.repivots == 0
+    assert (got["reasons"] == 0).all()
+    assert np.array_equal(got["iterations"], ref["iterations"])
+    assert np.array_equal(bits(got["x"]), bits(ref["x"]))
+    eng.close()
