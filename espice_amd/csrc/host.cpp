@@ -2171,6 +2171,62 @@ void build_reduce_streams(const Compiled &c, TapeHostProg &o)
 // Every index a kernel reads is checked on the host before the first launch,
 // so a malformed program is an error here rather than a GPU memory fault.
 
+// Whether the ops of one row may run in any order: the wavefronts of a team
+// read and write the row unordered until its barrier, so no op may read or
+// write a slot that another op of the row writes. words: the row, W of them,
+// x = d | b << 16; third(w): a further slot the op reads. stamp: one entry a
+// slot, last row written; row: unlike any earlier call's on the same stamps.
+template <typename F>
+bool row_independent(const esl::uint2_t *words, u32 W, vector<u32> &stamp, u32 row, F third)
+{
+    for (u32 t = 0; t < W; t++) {
+        const u32 d = words[t].x & 0xffff;
+        if (stamp[d] == row) return false;
+        stamp[d] = row;
+    }
+    for (u32 t = 0; t < W; t++) {
+        const u32 d = words[t].x & 0xffff, b = words[t].x >> 16, c = third(words[t]);
+        if ((b != d && stamp[b] == row) || (c != d && stamp[c] == row)) return false;
+    }
+    return true;
+}
+
+// One block's rows (W words each, over lim slots): kinds, slots, and the
+// independence of each row.
+bool block_rows_ok(const esl::uint2_t *words, u32 rows, u32 W, u32 lim)
+{
+    vector<u32> stamp(lim, NONE);
+    for (u32 r = 0; r < rows; r++) {
+        const esl::uint2_t *row = words + (size_t)r * W;
+        const u32 kind = esl::row_kind(row[0].y);
+        if (kind >= esl::R_KINDS || kind == esl::R_MACZ || kind == esl::R_CHAIN) return false;
+        for (u32 t = 0; t < W; t++) {
+            const esl::uint2_t w = row[t];
+            if (esl::row_kind(w.y) != kind || (w.y >> 22) != 0) return false;
+            if ((w.x & 0xffff) >= lim || (w.x >> 16) >= lim || (w.y & 0xffff) >= lim) return false;
+        }
+        if (!row_independent(row, W, stamp, r, [](const esl::uint2_t &w) { return w.y & 0xffffu; })) return false;
+    }
+    return true;
+}
+
+// The rows of a solve program (W words each) over lim solve-vector slots and
+// n_tv factor slots.
+bool solve_rows_ok(const esl::uint2_t *words, size_t rows, u32 W, u32 lim, u32 n_tv)
+{
+    vector<u32> stamp(lim, NONE);
+    for (size_t r = 0; r < rows; r++) {
+        const esl::uint2_t *row = words + r * W;
+        for (u32 t = 0; t < W; t++) {
+            const esl::uint2_t w = row[t];
+            if ((w.x & 0xffff) >= lim || (w.x >> 16) >= lim || (w.y & ~esl::kSolDiv) >= n_tv) return false;
+            if ((w.y & esl::kSolDiv) != (row[0].y & esl::kSolDiv)) return false;
+        }
+        if (!row_independent(row, W, stamp, (u32)r, [](const esl::uint2_t &w) { return w.x & 0xffffu; })) return false;
+    }
+    return true;
+}
+
 // A big tape's blocks and solve program.
 bool validate_big(const TapeHostProg &o, u32 n, u32 W = esl::kTeamThreads)
 {
@@ -2183,27 +2239,12 @@ bool validate_big(const TapeHostProg &o, u32 n, u32 W = esl::kTeamThreads)
         if ((size_t)b.slot_off + b.m > o.blk_slots.size()) return false;
         if (b.rows == 0 || b.rows % esl::kRing || (size_t)b.row0 + b.rows + esl::kRing > total_rows) return false;
         bm = std::max(bm, b.m);
-        const u32 lim = b.m + W;
-        for (size_t r = b.row0; r < (size_t)b.row0 + b.rows; r++) {
-            const u32 kind = esl::row_kind(o.blk_words[r * W].y);
-            if (kind >= esl::R_KINDS || kind == esl::R_MACZ || kind == esl::R_CHAIN) return false;
-            for (u32 t = 0; t < W; t++) {
-                const esl::uint2_t w = o.blk_words[r * W + t];
-                if (esl::row_kind(w.y) != kind || (w.y >> 22) != 0) return false;
-                const u32 d = w.x & 0xffff, bb = w.x >> 16, c = w.y & 0xffff;
-                if (d >= lim || bb >= lim || c >= lim) return false;
-            }
-        }
+        if (!block_rows_ok(o.blk_words.data() + (size_t)b.row0 * W, b.rows, W, b.m + W)) return false;
     }
     if (bm != P.blk_m) return false;
     for (u32 v : o.blk_slots) if (v >= P.n_tv) return false;
     if (P.sol_rows % esl::kRing || o.sol_w.size() != ((size_t)P.sol_rows + esl::kRing) * W) return false;
-    for (size_t k = 0; k < o.sol_w.size(); k++) {
-        const esl::uint2_t w = o.sol_w[k];
-        if ((w.x & 0xffff) >= n + W || (w.x >> 16) >= n + W || (w.y & ~esl::kSolDiv) >= P.n_tv) return false;
-        if ((w.y & esl::kSolDiv) != (o.sol_w[k - k % W].y & esl::kSolDiv)) return false;
-    }
-    return true;
+    return solve_rows_ok(o.sol_w.data(), (size_t)P.sol_rows + esl::kRing, W, n + W, P.n_tv);
 }
 bool validate_tape(const TapeHostProg &o, u32 n, u32 nnz, u32 ncs = 0)
 {
@@ -2697,21 +2738,38 @@ esl_status esl_debug_profile(esl_engine *h, int enable, unsigned long long *out,
     return ESL_OK;
 }
 
+// Development hook, not part of the drop-in: the check that every row of a
+// big tape's programs passes before it reaches a kernel, on `rows` rows of
+// `width` words x, y (2 u32 each) over `slots` slots: ESL_FAILED when a word
+// is out of range, a row mixes kinds, or an op of a row reads or writes what
+// another op of it writes. solve: rows of the solve program. Needs no device.
+esl_status esl_debug_big_rows(const uint32_t *words, uint32_t rows, uint32_t width, uint32_t slots, int solve)
+{
+    if (!words || width == 0 || slots == 0 || slots > 65536) return ESL_INVALID_ARGUMENT;
+    vector<esl::uint2_t> w((size_t)rows * width);
+    for (size_t k = 0; k < w.size(); k++) w[k] = esl::uint2_t{words[2 * k], words[2 * k + 1]};
+    const bool ok = solve ? solve_rows_ok(w.data(), rows, width, slots, slots)
+                          : block_rows_ok(w.data(), rows, width, slots);
+    return ok ? ESL_OK : ESL_FAILED;
+}
+
 // Development hook, not part of the drop-in: the replay and solves of a
-// big tape (lanes in HBM) run on the CPU exactly as the big-lane kernel runs
-// them (blocks of at most block_slots slots gathered, their rows applied in
-// order, written slots scattered; the solves over the column chunks), for
+// big tape (lanes in HBM) run on the CPU as the big-lane kernel runs them
+// (blocks of at most block_slots slots gathered, their rows of `width` words
+// applied in order, every operand of a row read before any result of it is
+// written, written slots scattered; then the rows of the solve program), for
 // `lanes` matrices a [lanes][nnz] and right-hand sides rhs [lanes][n] on
 // the tape factored from lead_vals. Outputs per lane: L, U, pivots in the
 // tape's order, dx (row order) and the re-pivot flag; sizes: the block
 // count, nnz_l, nnz_u and the rows of all blocks (lanes == 0: only these).
 esl_status esl_debug_big_replay(uint32_t n, const uint32_t *col_ptr, const uint32_t *row_idx,
                                 const double *lead_vals, const uint32_t *q, double pivot_tol, uint32_t block_slots,
-                                const double *a, const double *rhs, uint32_t lanes, double *lx, double *ux,
-                                double *udiag, double *dx, uint32_t *fail, uint32_t *sizes)
+                                uint32_t width, const double *a, const double *rhs, uint32_t lanes, double *lx,
+                                double *ux, double *udiag, double *dx, uint32_t *fail, uint32_t *sizes)
 {
+    const u32 W = width;
     if (!col_ptr || !row_idx || !lead_vals || !q || n == 0 || (block_slots != 0 && block_slots < 3) ||
-        block_slots > kBigSlotLimit)
+        block_slots > kBigSlotLimit || (W != (u32)esl::kWave && W != esl::kTeamThreads))
         return ESL_INVALID_ARGUMENT;
     if (lanes && (!a || !rhs || !lx || !ux || !udiag || !dx || !fail)) return ESL_INVALID_ARGUMENT;
     HostTape t;
@@ -2720,9 +2778,7 @@ esl_status esl_debug_big_replay(uint32_t n, const uint32_t *col_ptr, const uint3
     TapeHostProg o;
     build_tape_prog(t, cp, 1e-12, 1.0 / pivot_tol, o);
     o.big = true;
-    // small blocks (many of them): narrow rows, the same programs otherwise
     if (block_slots == 0) block_slots = kBigBlockSlots;
-    const u32 W = block_slots < 1024 ? (u32)esl::kWave : esl::kTeamThreads;
     if (!build_big_program(t, o, block_slots, W) || !validate_big(o, n, W)) return ESL_FAILED;
     const esl::TapeProg &T = o.prog;
     if (sizes) {
@@ -2733,7 +2789,7 @@ esl_status esl_debug_big_replay(uint32_t n, const uint32_t *col_ptr, const uint3
     }
     const u32 nnz = cp[n];
     for (u32 l = 0; l < lanes; l++) {
-        vector<double> tv(T.n_tv, 0.0), M(T.blk_m + W, 0.0), y(n);
+        vector<double> tv(T.n_tv, 0.0), M(T.blk_m + W, 0.0), y(n + W, 0.0), rd(3 * (size_t)W);
         for (u32 p = 0; p < nnz; p++) tv[o.amap[p]] = a[(size_t)l * nnz + p];
         bool bad = false;
         uint64_t nonfinite = 0, worst = 0;
@@ -2744,17 +2800,23 @@ esl_status esl_debug_big_replay(uint32_t n, const uint32_t *col_ptr, const uint3
             if (o.flags[k] & esl::kVoidBit) tv[T.n_u + k] = 1.0;
         for (const esl::BigBlock &B : o.blk) {
             for (u32 j = 0; j < B.m; j++) M[j] = tv[o.blk_slots[B.slot_off + j]];
-            for (u32 r = B.row0; r < B.row0 + B.rows; r++)
+            for (u32 r = B.row0; r < B.row0 + B.rows; r++) {
+                const esl::uint2_t *row = o.blk_words.data() + (size_t)r * W;
                 for (u32 th = 0; th < W; th++) {
-                    const esl::uint2_t w = o.blk_words[(size_t)r * W + th];
-                    const u32 kind = esl::row_kind(w.y), d = w.x & 0xffff, b = w.x >> 16, c = w.y & 0xffff;
+                    rd[3 * th] = M[row[th].x & 0xffff];
+                    rd[3 * th + 1] = M[row[th].x >> 16];
+                    rd[3 * th + 2] = M[row[th].y & 0xffff];
+                }
+                for (u32 th = 0; th < W; th++) {
+                    const u32 kind = esl::row_kind(row[th].y), d = row[th].x & 0xffff;
+                    const double v = rd[3 * th], A = rd[3 * th + 1];
                     if (kind == esl::R_MAC) {
-                        const double m = M[b] * M[c];
-                        M[d] = M[d] - m;
+                        const double m = A * rd[3 * th + 2];
+                        M[d] = v - m;
                     } else if (kind == esl::R_DIV) {
-                        const double v = M[d], A = M[b], qq = v / A;
+                        const double qq = v / A;
                         M[d] = qq;
-                        const u32 fl = esl::row_flags(w.y);
+                        const u32 fl = esl::row_flags(row[th].y);
                         const bool un = fl & esl::kFlagUnscaled;
                         bad |= un && T.growth > 0 && !(std::fabs(A) >= T.growth * std::fabs(v));
                         nonfinite |= ((un && !(T.growth > 0)) || (fl & esl::kFlagScaled)) ? bits(qq - qq) : 0;
@@ -2762,6 +2824,7 @@ esl_status esl_debug_big_replay(uint32_t n, const uint32_t *col_ptr, const uint3
                         worst = lb > worst ? lb : worst;
                     }
                 }
+            }
             for (u32 j = 0; j < B.w; j++) tv[o.blk_slots[B.slot_off + j]] = M[j];
         }
         for (u32 p = 0; p < T.n_u; p++) nonfinite |= bits(tv[p] - tv[p]);
@@ -2772,15 +2835,18 @@ esl_status esl_debug_big_replay(uint32_t n, const uint32_t *col_ptr, const uint3
         }
         fail[l] = (bad || nonfinite != 0 || !(dbl(worst) <= T.wide)) ? 1u : 0u;
         for (u32 r = 0; r < n; r++) y[o.pinv[r]] = -rhs[(size_t)l * n + r];
-        for (u32 r = 0; r < T.sol_rows; r++)
+        for (u32 r = 0; r < T.sol_rows; r++) {
+            const esl::uint2_t *row = o.sol_w.data() + (size_t)r * W;
             for (u32 th = 0; th < W; th++) {
-                const esl::uint2_t w = o.sol_w[(size_t)r * W + th];
-                const u32 d = w.x & 0xffff, c = w.x >> 16;
-                if (d >= n) continue;
-                const double v = y[d], A = tv[w.y & ~esl::kSolDiv];
-                const double m = A * y[c];
-                y[d] = (w.y & esl::kSolDiv) ? v / A : y[c] != 0.0 ? v - m : v;
+                rd[2 * th] = y[row[th].x & 0xffff];
+                rd[2 * th + 1] = y[row[th].x >> 16];
             }
+            for (u32 th = 0; th < W; th++) {
+                const double v = rd[2 * th], B = rd[2 * th + 1], A = tv[row[th].y & ~esl::kSolDiv];
+                const double m = A * B;
+                y[row[th].x & 0xffff] = (row[th].y & esl::kSolDiv) ? v / A : B != 0.0 ? v - m : v;
+            }
+        }
         for (u32 p = 0; p < T.n_u; p++) ux[(size_t)l * T.n_u + p] = tv[p];
         for (u32 k = 0; k < n; k++) udiag[(size_t)l * n + k] = tv[T.n_u + k];
         for (u32 qq = 0; qq < T.n_l; qq++) lx[(size_t)l * T.n_l + qq] = tv[T.lx0 + qq];

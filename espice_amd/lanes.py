@@ -192,8 +192,10 @@ def load() -> C.CDLL:
     L.esl_last_timing.restype = C.c_uint32
     L.esl_last_timing.argtypes = [vp, C.POINTER(Timing)]
     L.esl_tape_create.restype = C.c_uint32
-    L.esl_debug_big_replay.argtypes = [C.c_uint32, vp, vp, vp, vp, C.c_double, C.c_uint32, vp, vp, C.c_uint32,
-                                       vp, vp, vp, vp, vp, vp]
+    L.esl_debug_big_replay.argtypes = [C.c_uint32, vp, vp, vp, vp, C.c_double, C.c_uint32, C.c_uint32, vp, vp,
+                                       C.c_uint32, vp, vp, vp, vp, vp, vp]
+    L.esl_debug_big_rows.argtypes = [vp, C.c_uint32, C.c_uint32, C.c_uint32, C.c_int]
+    L.esl_debug_big_rows.restype = C.c_int
     L.esl_debug_big_replay.restype = C.c_int
     L.esl_debug_row_replay.argtypes = [C.c_uint32, vp, vp, vp, vp, C.c_double, C.c_uint32, vp, vp, C.c_uint32,
                                        vp, vp, vp, vp, vp, vp]
@@ -494,10 +496,25 @@ def solve_batch(jobs, tiling=TILING_AUTO, tune=False):
     return out, rep
 
 
-def debug_big_replay(col_ptr, row_idx, lead_vals, q, a, rhs, block_slots=4032, pivot_tol=1e-3):
-    """The big-lane kernel's blocked refactor and chunked solves run on the
-    CPU (esl_debug_big_replay) for a [lanes][nnz], rhs [lanes][n]: a
-    development check of the block programs, no device needed."""
+def debug_big_rows(words, slots, solve=False):
+    """Whether rows of a big-lane program ([rows][width][2] words over
+    `slots` slots) pass the check made before a kernel runs them
+    (esl_debug_big_rows): in range, and no op of a row reading or writing
+    what another op of it writes."""
+    w = np.ascontiguousarray(words, dtype=np.uint32)
+    st = load().esl_debug_big_rows(_ptr(w), w.shape[0], w.shape[1], slots, 1 if solve else 0)
+    if st not in (OK, FAILED):
+        _check(st, "big rows")
+    return st == OK
+
+
+def debug_big_replay(col_ptr, row_idx, lead_vals, q, a, rhs, block_slots=4032, pivot_tol=1e-3, width=None):
+    """The big-lane kernel's blocked refactor and row-program solves run on
+    the CPU (esl_debug_big_replay), rows of `width` words (64 or the
+    kernel's 512; by default 64 for blocks of fewer slots than that, whose
+    rows never fill), for a [lanes][nnz], rhs [lanes][n]: a development
+    check of the block programs, no device needed."""
+    width = width or (64 if block_slots < 64 else 512)
     L = load()
     cp, ri, qq = (np.ascontiguousarray(v, dtype=np.uint32) for v in (col_ptr, row_idx, q))
     lead = np.ascontiguousarray(lead_vals, dtype=np.float64)
@@ -505,7 +522,7 @@ def debug_big_replay(col_ptr, row_idx, lead_vals, q, a, rhs, block_slots=4032, p
     rhs = np.ascontiguousarray(np.atleast_2d(rhs), dtype=np.float64)
     n, lanes = len(cp) - 1, a.shape[0]
     sizes = np.zeros(4, np.uint32)
-    args = (n, _ptr(cp), _ptr(ri), _ptr(lead), _ptr(qq), pivot_tol, block_slots)
+    args = (n, _ptr(cp), _ptr(ri), _ptr(lead), _ptr(qq), pivot_tol, block_slots, width)
     _check(L.esl_debug_big_replay(*args, None, None, 0, None, None, None, None, None, _ptr(sizes)), "big replay")
     nl, nu = int(sizes[1]), int(sizes[2])
     out = dict(lx=np.zeros((lanes, nl)), ux=np.zeros((lanes, nu)), udiag=np.zeros((lanes, n)),

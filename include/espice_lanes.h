@@ -484,7 +484,9 @@ esl_status esl_debug_profile(esl_engine *e, int enable, unsigned long long *out,
 
 /* Development hook, not part of the drop-in: the refactor and solves of the
  * kernel for lanes beyond a workgroup's LDS (the replay cut into blocks of
- * at most block_slots slots, the solves in column chunks), run on the CPU
+ * at most block_slots slots, 0: the kernel's, in rows of `width` words, the
+ * solves as rows too), run on the CPU with every operand of a row read before
+ * any result of it is written,
  * for `lanes` matrices a [lanes][nnz] and right-hand sides rhs [lanes][n]
  * on the tape factored from lead_vals with column order q. Writes per lane
  * L [lanes][nnz_l], U [lanes][nnz_u], the pivots [lanes][n], dx [lanes][n]
@@ -496,10 +498,17 @@ esl_status esl_debug_big_replay(uint32_t n, const uint32_t *col_ptr,
                                 const uint32_t *row_idx,
                                 const double *lead_vals, const uint32_t *q,
                                 double pivot_tol, uint32_t block_slots,
-                                const double *a, const double *rhs,
-                                uint32_t lanes, double *lx, double *ux,
-                                double *udiag, double *dx, uint32_t *fail,
-                                uint32_t *sizes);
+                                uint32_t width, const double *a,
+                                const double *rhs, uint32_t lanes, double *lx,
+                                double *ux, double *udiag, double *dx,
+                                uint32_t *fail, uint32_t *sizes);
+
+/* Development hook, not part of the drop-in: the check of those rows (words
+ * in range, one kind a row, no op of a row reading or writing what another op
+ * of it writes) on given words [rows][width][2] over `slots` slots; solve:
+ * rows of the solve program. ESL_FAILED when it does not hold. */
+esl_status esl_debug_big_rows(const uint32_t *words, uint32_t rows,
+                              uint32_t width, uint32_t slots, int solve);
 
 /* Development hook, not part of the drop-in: the refactor and solve row
  * programs of the wavefront kernels (chain rows for runs of at least

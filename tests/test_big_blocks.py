@@ -1,7 +1,8 @@
-"""The blocked refactor and chunked solves of the big-lane kernel, run on
+"""The blocked refactor and row-program solves of the big-lane kernel, run on
 the CPU by the library (esl_debug_big_replay) and compared with the oracle's
 serial replay (lane_kernels.zig:49-143): the blocks gather their slots,
-apply their rows and scatter what they wrote, so L, U, the pivots, dx and
+apply their rows (every operand of a row read before any result of it is
+written) and scatter what they wrote, so L, U, the pivots, dx and
 the re-pivot flag must equal the serial column replay's bit for bit, for
 any block size down to a few slots (many blocks, ops of one target split
 across blocks) and on the peel cases (void column, wide multiplier, growth).
@@ -50,8 +51,8 @@ def grid_laplacian(rng, k):
     return np.array(cp, np.uint32), np.array(ri, np.uint32), np.array(vals)
 
 
-def compare(lanes, oracle, cp, ri, lead, q, a, rhs, block_slots):
-    got = lanes.debug_big_replay(cp, ri, lead, q, a, rhs, block_slots=block_slots)
+def compare(lanes, oracle, cp, ri, lead, q, a, rhs, block_slots, width=None):
+    got = lanes.debug_big_replay(cp, ri, lead, q, a, rhs, block_slots=block_slots, width=width)
     ref = oracle.lu_replay(cp, ri, lead, q, a, rhs)
     assert ref is not None
     assert np.array_equal(got["fail"], ref["fail"])
@@ -109,14 +110,57 @@ def test_peel_cases_fail_as_serial(lanes, oracle):
         assert list(got["fail"]) == [0, 1]
 
 
-@pytest.mark.parametrize("k,block_slots", [(5, 1024), (9, 1500), (14, 2048), (14, 18944)])
+@pytest.mark.parametrize("k,block_slots", [(5, 40), (5, 1024), (9, 64), (9, 1500), (14, 256), (14, 2048), (14, 18944)])
 def test_team_rows_equal_serial(lanes, oracle, k, block_slots):
-    """Blocks run in rows of 512 words (wide blocks) equal the serial replay:
-    one block, several, and rows with more ops than a wavefront holds."""
+    """Blocks run in rows of 512 words equal the serial replay: one block,
+    several, many small ones, and rows with more ops than a wavefront holds."""
     rng = np.random.default_rng(k)
     cp, ri, lead = grid_laplacian(rng, k)
     q = np.arange(k * k, dtype=np.uint32)
     a = lead * (1 + 0.02 * rng.standard_normal((3, len(lead))))
     rhs = rng.standard_normal((3, k * k))
-    got, ok = compare(lanes, oracle, cp, ri, lead, q, a, rhs, block_slots)
+    got, ok = compare(lanes, oracle, cp, ri, lead, q, a, rhs, block_slots, width=512)
     assert ok.all()
+    assert got["blocks"] > 1 or block_slots >= 1024
+
+
+R_NOP, R_MAC, R_DIV = 0, 1, 3
+
+
+def block_row(ops, width, m, kind):
+    """One row of words: ops (d, b, c), the other threads on their pads."""
+    w = np.zeros((width, 2), np.uint32)
+    for t in range(width):
+        d, b, c = ops[t] if t < len(ops) else (m + t,) * 3
+        w[t] = d | (b << 16), c | (kind << 16)
+    return w
+
+
+@pytest.mark.parametrize("ops,ok", [
+    ([(0, 1, 2), (3, 1, 2)], True),        # shared operands
+    ([(0, 1, 2), (3, 0, 2)], False),       # reads what the row writes (b)
+    ([(3, 1, 0), (0, 1, 2)], False),       # the same through c, the writer on a later thread
+    ([(0, 1, 2), (0, 1, 3)], False),       # two ops on one target
+])
+@pytest.mark.parametrize("far", [False, True])
+def test_rows_of_dependent_ops_are_refused(lanes, ops, ok, far):
+    """The wavefronts of a team run a row in any order: a row whose ops
+    depend on one another must not reach the kernel, whichever wavefronts
+    they are on (far: the second op on another one), though a serial walk
+    of the row would give the serial result."""
+    m, width = 8, 512
+    row = block_row(ops, width, m, R_MAC)
+    if far:
+        row[[1, 300]] = row[[300, 1]]
+        row[1] = m + 1 | (m + 1) << 16, m + 1 | R_MAC << 16
+    idle = block_row([], width, m, R_NOP)
+    for rows in ([row], [idle, row], [row, idle, row]):
+        assert lanes.debug_big_rows(np.array(rows), m + width) is ok
+        assert not lanes.debug_big_rows(np.array(rows), m + width - 1)   # the last pad out of range
+    # the solve program's words: x = d | c << 16, y a factor slot
+    sol = row.copy()
+    for t in range(width):
+        d, c = int(row[t, 0]) & 0xffff, int(row[t, 1]) & 0xffff
+        sol[t] = d | c << 16, 0
+    want = ok or ops == [(0, 1, 2), (3, 0, 2)]   # b is no operand there
+    assert lanes.debug_big_rows(np.array([sol]), m + width, solve=True) is want
