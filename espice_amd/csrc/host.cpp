@@ -16,7 +16,9 @@
 #include <cstdio>
 #include <cstring>
 #include <map>
+#include <memory>
 #include <mutex>
+#include <new>
 #include <queue>
 #include <set>
 #include <thread>
@@ -3802,30 +3804,51 @@ esl_status tran_adaptive_rounds(Engine &E, const esl::TranArgs &ta, const esl::P
     HIPCHK(hipMemcpyAsync(iterations, e->iters.p, count * 4, hipMemcpyDeviceToHost, s));
     HIPCHK(hipStreamSynchronize(s));
     // the accepted rows only: the device's rows past them hold whatever the
-    // buffers held before
-    size_t top = 0;
-    for (size_t l = 0; l < count; l++)
-        if (reasons[l] == ESL_REASON_OK) top = std::max<size_t>(top, std::min(st[l].steps, o.max_steps));
-    vector<double> rows;
-    auto take = [&](const double *src, double *dst, size_t w) -> hipError_t {
-        if (!top || !w) return hipSuccess;
-        hipError_t er = e->probe_out.ensure(count * top * w * 8);
-        if (er != hipSuccess) return er;
-        er = esl_launch_pack(src, (size_t)o.max_steps * w, top * w, (u32)count, e->probe_out.as<double>(), s);
-        if (er != hipSuccess) return er;
-        rows.resize(count * top * w);
-        er = hipMemcpyAsync(rows.data(), e->probe_out.p, rows.size() * 8, hipMemcpyDeviceToHost, s);
-        if (er != hipSuccess) return er;
-        er = hipStreamSynchronize(s);
-        if (er != hipSuccess) return er;
-        for (size_t l = 0; l < count; l++)
-            if (reasons[l] == ESL_REASON_OK)
-                memcpy(dst + l * o.max_steps * w, rows.data() + l * top * w,
-                       std::min<size_t>(st[l].steps, top) * w * 8);
-        return hipSuccess;
+    // buffers held before. Slabs of lanes are packed on the device and copied
+    // through two buffers of at most kSlab doubles; rows of a lane that are
+    // long by themselves go to the caller directly.
+    constexpr size_t kSlab = 8u << 20, kLong = 32u << 10;
+    auto rows_of = [&](size_t l) -> size_t {
+        return reasons[l] == ESL_REASON_OK ? std::min(st[l].steps, o.max_steps) : 0;
     };
-    HIPCHK(take(e->ttimes.as<double>(), ar.times, 1));
-    HIPCHK(take(e->tprobes.as<double>(), probe_out, o.n_probes));
+    size_t top_all = 0;
+    for (size_t l = 0; l < count; l++) top_all = std::max(top_all, rows_of(l));
+    std::unique_ptr<double[]> rows;
+    auto take = [&](const double *src, double *dst, size_t w) -> esl_status {
+        if (!top_all || !w) return ESL_OK;
+        const size_t stride = (size_t)o.max_steps * w;
+        if (top_all * w >= kLong) {
+            for (size_t l = 0; l < count; l++)
+                if (rows_of(l))
+                    HIPCHK(hipMemcpyAsync(dst + l * stride, src + l * stride, rows_of(l) * w * 8,
+                                          hipMemcpyDeviceToHost, s));
+            HIPCHK(hipStreamSynchronize(s));
+            return ESL_OK;
+        }
+        const size_t slab = std::min(count, kSlab / (top_all * w));
+        rows.reset(new (std::nothrow) double[slab * top_all * w]);
+        if (!rows) {
+            g_last_error = "no host memory for the accepted rows";
+            return ESL_FAILED;
+        }
+        HIPCHK(e->probe_out.ensure(slab * top_all * w * 8));
+        for (size_t l0 = 0; l0 < count; l0 += slab) {
+            const size_t l1 = std::min(count, l0 + slab);
+            size_t top = 0;
+            for (size_t l = l0; l < l1; l++) top = std::max(top, rows_of(l));
+            if (!top) continue;
+            const size_t k = top * w;
+            HIPCHK(esl_launch_pack(src + l0 * stride, stride, k, (u32)(l1 - l0), e->probe_out.as<double>(), s));
+            HIPCHK(hipMemcpyAsync(rows.get(), e->probe_out.p, (l1 - l0) * k * 8, hipMemcpyDeviceToHost, s));
+            HIPCHK(hipStreamSynchronize(s));
+            for (size_t l = l0; l < l1; l++)
+                if (rows_of(l)) memcpy(dst + l * stride, rows.get() + (l - l0) * k, rows_of(l) * w * 8);
+        }
+        return ESL_OK;
+    };
+    esl_status tr = take(e->ttimes.as<double>(), ar.times, 1);
+    if (tr == ESL_OK) tr = take(e->tprobes.as<double>(), probe_out, o.n_probes);
+    if (tr != ESL_OK) return tr;
     uint64_t lane_it = 0;
     for (size_t l = 0; l < count; l++) {
         if (reasons[l] != ESL_REASON_OK) {   // the operating point failed

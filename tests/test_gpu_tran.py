@@ -240,3 +240,56 @@ def test_lines_take_the_shallow_order_bitwise_against_oracle(lanes, oracle, node
     assert np.array_equal(bits(got["probes"]), bits(ref["probes"]))
     assert np.array_equal(bits(got["x"]), bits(ref["x"]))
     eng.close()
+
+
+@pytest.mark.parametrize("points,probes,steps", [(3, 1, 40), (6000, 160, 40), (2, 4000, 40)])
+def test_adaptive_rows_come_back_by_slabs(lanes, points, probes, steps):
+    """The accepted rows come back packed in slabs of lanes (several of them
+    for 6,000 lanes of 160 probes), or lane by lane where one lane's rows are
+    long; either way each lane's rows are those of a solve of its own, and
+    what lies past them stays the caller's."""
+    fam = circuits.rc_ladder(16, tran=True)
+    vals = fam.sample(21, points)
+    eng = lanes.Engine(fam.deck.arrays())
+    ids = [2 + k % 16 for k in range(probes)]
+    got = eng.solve_tran_adaptive(vals, steps * 1e-11, 1e-11, probes=ids, max_steps=200)
+    assert (got["reasons"] == 0).all()
+    assert got["accepted"].min() >= 10 and got["accepted"].max() < 200
+    words = int(got["accepted"].max()) * probes
+    assert points < 6000 or points * words > 8 << 20   # several slabs
+    assert probes < 4000 or words > 32 << 10           # long rows
+    for l in {0, 1, points // 2, points - 1}:
+        one = eng.solve_tran_adaptive(vals[l:l + 1], steps * 1e-11, 1e-11, probes=ids[:16], max_steps=200)
+        a = int(got["accepted"][l])
+        assert one["accepted"][0] == a
+        assert np.array_equal(bits(got["times"][l]), bits(one["times"][0]))
+        assert np.array_equal(bits(got["probes"][l][:, :16]), bits(one["probes"][0][:, :probes]))
+        assert (got["times"][l, a:] == 0).all() and (got["probes"][l, a:] == 0).all()
+    for k in range(16, probes, 16):   # the further probes repeat the first 16
+        assert np.array_equal(got["probes"][:, :, k:k + 16], got["probes"][:, :, :16])
+    eng.close()
+
+
+def test_adaptive_rows_take_no_second_copy_on_the_device(lanes):
+    """A run whose lanes fill max_steps holds its rows once on the device:
+    the slabs they come back through are of a fixed size."""
+    import ctypes
+
+    def free():
+        f, t = ctypes.c_size_t(), ctypes.c_size_t()
+        assert lanes.load().hipMemGetInfo(ctypes.byref(f), ctypes.byref(t)) == 0
+        return f.value
+
+    fam = circuits.rc_ladder(16, tran=True)
+    eng = lanes.Engine(fam.deck.arrays())
+    ids = [2 + k % 16 for k in range(128)]
+    steps = int(eng.solve_tran_adaptive(fam.sample(22, 1), 4e-10, 1e-11, probes=ids, max_steps=200)["accepted"][0])
+    vals = np.repeat(fam.sample(22, 1), 16 * 1024, axis=0)   # 16 MB a step
+    free0 = free()
+    got = eng.solve_tran_adaptive(vals, 4e-10, 1e-11, probes=ids, max_steps=steps)
+    used = free0 - free()
+    rows = vals.shape[0] * steps * len(ids) * 8
+    say(f"  {steps} steps, rows {rows / 2**20:.0f} MB, device memory taken {used / 2**20:.0f} MB")
+    assert (got["accepted"] == steps).all()
+    assert used < 1.5 * rows
+    eng.close()
