@@ -312,11 +312,8 @@ bool gp_factor(u32 n, const u32 *col_ptr, const u32 *row_idx, const double *vals
     return true;
 }
 
-// Minimum degree on the pattern of A + A^T (ties to the lowest index).
-// shallow: the next vertex is instead the one of least 2 * degree + level,
-// level being the longest elimination path that ends in it. depth: the
-// longest path of the order; fill: the entries of L (and of U).
-vector<u32> min_degree(u32 n, const vector<u32> &col_ptr, const vector<u32> &row_idx, bool shallow, u32 &depth, size_t &fill)
+// The neighbours of each unknown in the pattern of A + A^T, ascending.
+vector<vector<u32>> sym_pattern(u32 n, const vector<u32> &col_ptr, const vector<u32> &row_idx)
 {
     vector<vector<u32>> adj(n);
     for (u32 j = 0; j < n; j++)
@@ -330,39 +327,74 @@ vector<u32> min_degree(u32 n, const vector<u32> &col_ptr, const vector<u32> &row
         std::sort(a.begin(), a.end());
         a.erase(std::unique(a.begin(), a.end()), a.end());
     }
+    return adj;
+}
+
+// An elimination order of a symmetric pattern. depth: its longest path;
+// fill: the entries of L (and of U). Empty q: the order passed a limit.
+struct Order {
+    vector<u32> q;
+    u32 depth = 0;
+    size_t fill = 0;
+};
+
+// Minimum degree (ties to the lowest index). shallow: the next vertex is
+// instead the one of least 2 * degree + level, level being the longest
+// elimination path that ends in it; given up once it passes max_depth or
+// max_fill. The next vertex comes off a heap of (key, vertex); an entry
+// whose vertex is gone or has another key by now is dropped when it
+// surfaces (with a scan of all vertices a step, creating the engine of a
+// line of 2,048 nodes took 3.6 ms, and 10.8 ms with both orders; it takes
+// 2.5 ms).
+Order min_degree(vector<vector<u32>> adj, bool shallow = false, u32 max_depth = NONE, size_t max_fill = SIZE_MAX)
+{
+    const u32 n = (u32)adj.size();
+    Order o;
     vector<char> gone(n, 0);
     vector<u32> level(n, 0);
-    fill = 0;
-    vector<u32> q;
-    q.reserve(n);
-    vector<u32> merged;
-    for (u32 step = 0; step < n; step++) {
-        u32 best = NONE;
-        size_t bd = SIZE_MAX;
-        for (u32 v = 0; v < n; v++) {
-            const size_t key = shallow ? 2 * adj[v].size() + level[v] : adj[v].size();
-            if (!gone[v] && key < bd) {
-                bd = key;
-                best = v;
-            }
-        }
-        const u32 v = best;
-        q.push_back(v);
+    using Entry = std::pair<size_t, u32>;
+    auto key = [&](u32 v) { return shallow ? 2 * adj[v].size() + level[v] : adj[v].size(); };
+    vector<Entry> init(n);
+    for (u32 v = 0; v < n; v++) init[v] = {key(v), v};
+    std::priority_queue<Entry, vector<Entry>, std::greater<Entry>> heap(std::greater<Entry>(), std::move(init));
+    vector<u32> merged, nb;
+    o.q.reserve(n);
+    while (o.q.size() < n) {
+        const Entry top = heap.top();
+        heap.pop();
+        const u32 v = top.second;
+        if (gone[v] || top.first != key(v)) continue;
+        o.q.push_back(v);
         gone[v] = 1;
-        const vector<u32> nb = adj[v];
-        fill += nb.size();
-        for (u32 u : nb) {
-            level[u] = std::max(level[u], level[v] + 1);
-            merged.clear();
-            std::set_union(adj[u].begin(), adj[u].end(), nb.begin(), nb.end(), std::back_inserter(merged));
-            adj[u].clear();
-            for (u32 w : merged)
-                if (w != u && !gone[w]) adj[u].push_back(w);
+        nb.clear();
+        nb.swap(adj[v]);
+        o.fill += nb.size();
+        if (!nb.empty()) o.depth = std::max(o.depth, level[v] + 1);
+        if (o.depth > max_depth || o.fill > max_fill) {
+            o.q.clear();
+            return o;
         }
-        adj[v].clear();
+        for (u32 u : nb) {
+            const size_t before = key(u);
+            vector<u32> &au = adj[u];
+            level[u] = std::max(level[u], level[v] + 1);
+            // the union of u's and v's neighbours without the two
+            merged.clear();
+            size_t i = 0, j = 0;
+            while (i < au.size() || j < nb.size()) {
+                u32 x;
+                if (j == nb.size() || (i < au.size() && au[i] < nb[j])) x = au[i++];
+                else {
+                    x = nb[j++];
+                    if (i < au.size() && au[i] == x) i++;
+                }
+                if (x != u && x != v) merged.push_back(x);
+            }
+            au.assign(merged.begin(), merged.end());
+            if (key(u) != before) heap.push({key(u), u});
+        }
     }
-    depth = *std::max_element(level.begin(), level.end());
-    return q;
+    return o;
 }
 
 // The column order of a deck. Plain minimum degree eats a line of resistors
@@ -377,15 +409,17 @@ vector<u32> min_degree(u32 n, const vector<u32> &col_ptr, const vector<u32> &row
 // where two-terminal decks agree to rounding in any order.
 vector<u32> deck_order(u32 n, const vector<u32> &col_ptr, const vector<u32> &row_idx, bool transistors)
 {
-    u32 d0 = 0, d1 = 0;
-    size_t f0 = 0, f1 = 0;
-    vector<u32> q = min_degree(n, col_ptr, row_idx, false, d0, f0);
-    if (transistors || 8 * (size_t)d0 < n) return q;   // a path of n / 8 columns: nothing like a line
-    vector<u32> q1 = min_degree(n, col_ptr, row_idx, true, d1, f1);
-    // a lane holds its factors and about eight n-vectors in LDS: the extra
-    // fill must not cost it the LDS of half a workgroup
-    if ((n + 2 * f1 + 8 * (size_t)n) * 8 > 80 * 1024) return q;
-    return 2 * d1 <= d0 ? q1 : q;
+    const vector<vector<u32>> adj = sym_pattern(n, col_ptr, row_idx);
+    Order plain = min_degree(adj);
+    if (transistors || 8 * (size_t)plain.depth < n) return plain.q;   // a path of n / 8 columns: nothing like a line
+    // a lane holds its factors (n + 2 fill) and about eight n-vectors in
+    // LDS: the shallow one may take half of a workgroup's, which keeps two
+    // lanes on a CU (measured at 182 nodes; a line of more than about 800
+    // nodes keeps the plain order, whatever that takes itself)
+    constexpr size_t kHalf = 80 * 1024 / 8;
+    if (9 * (size_t)n > kHalf) return plain.q;
+    Order sh = min_degree(adj, true, plain.depth / 2, (kHalf - 9 * (size_t)n) / 2);
+    return sh.q.empty() ? plain.q : sh.q;
 }
 
 // Row programs. Every update of the refactor or the solve is one op
@@ -1235,8 +1269,6 @@ struct Compiled {
     // deck program host arrays
     vector<esl::Chunk> chunks;
     vector<u32> task_target, task_cell;
-    vector<u32> rt_round, rt_target, rt_cell;   // the tasks of rounds of kTeam chunks
-    vector<uint16_t> rt_cells;
     vector<uint16_t> cells;
     vector<u32> r_t, v_t, i_t, m_t;
     vector<double> r_val, v_val, i_val, m_par;
@@ -1743,30 +1775,6 @@ bool compile_deck(const esl_deck *d, Compiled &c, std::string &err)
     }
     c.task_cell.push_back((u32)c.cells.size());
     c.chunks.push_back(esl::Chunk{0, 0, 0, (u32)c.task_target.size()});
-    // rounds of kTeam chunks: each target's cells in chunk order
-    const u32 nch = (u32)c.chunks.size() - 1;
-    for (u32 c0 = 0; c0 < nch; c0 += esl::kTeam) {
-        c.rt_round.push_back((u32)c.rt_target.size());
-        std::map<u32, u32> at;   // target -> position in `lists`
-        vector<std::pair<u32, vector<u32>>> lists;
-        for (u32 k = c0; k < std::min(nch, c0 + esl::kTeam); k++)
-            for (u32 tk = c.chunks[k].task_begin; tk < c.chunks[k + 1].task_begin; tk++) {
-                auto it = at.emplace(c.task_target[tk], (u32)lists.size());
-                if (it.second) lists.push_back({c.task_target[tk], {}});
-                for (u32 cc = c.task_cell[tk]; cc < c.task_cell[tk + 1]; cc++)
-                    lists[it.first->second].second.push_back((k - c0) * esl::kStageDoubles + c.cells[cc]);
-            }
-        // threads take the lists in turn: the longest first
-        std::stable_sort(lists.begin(), lists.end(),
-                         [](auto &a, auto &b) { return a.second.size() > b.second.size(); });
-        for (auto &l : lists) {
-            c.rt_target.push_back(l.first);
-            c.rt_cell.push_back((u32)c.rt_cells.size());
-            for (u32 v : l.second) c.rt_cells.push_back((uint16_t)v);
-        }
-    }
-    c.rt_round.push_back((u32)c.rt_target.size());
-    c.rt_cell.push_back((u32)c.rt_cells.size());
     return true;
 }
 
@@ -1776,7 +1784,8 @@ struct Engine {
     Compiled c;
     DevBuf deck_buf;
     esl::DeckProg dp{};
-    // the reduce tasks by rounds, in deck_buf (BigArgs)
+    // a big engine's reduce tasks by rounds (BigArgs), from its first launch on
+    DevBuf rounds_buf;
     u32 n_rounds = 0;
     const u32 *rt_round = nullptr, *rt_target = nullptr, *rt_cell = nullptr;
     const uint16_t *rt_cells = nullptr;
@@ -1831,8 +1840,7 @@ hipError_t upload_deck(Engine &e)
     Compiled &c = e.c;
     Packer pk;
     size_t o_chunks = pk.add(c.chunks), o_tt = pk.add(c.task_target), o_tc = pk.add(c.task_cell),
-           o_rtr = pk.add(c.rt_round), o_rtt = pk.add(c.rt_target), o_rtc = pk.add(c.rt_cell),
-           o_rts = pk.add(c.rt_cells), o_cells = pk.add(c.cells), o_diag = pk.add(c.diag), o_cur = pk.add(c.current_row),
+           o_cells = pk.add(c.cells), o_diag = pk.add(c.diag), o_cur = pk.add(c.current_row),
            o_rt = pk.add(c.r_t), o_rv = pk.add(c.r_val), o_rb = pk.add(c.r_bind), o_vt = pk.add(c.v_t),
            o_vv = pk.add(c.v_val), o_vb = pk.add(c.v_bind), o_it = pk.add(c.i_t), o_iv = pk.add(c.i_val),
            o_ib = pk.add(c.i_bind), o_mt = pk.add(c.m_t), o_mp = pk.add(c.m_par), o_mbv = pk.add(c.m_bind_vto),
@@ -1897,11 +1905,6 @@ hipError_t upload_deck(Engine &e)
     dp.chunks = reinterpret_cast<const esl::Chunk *>(b + o_chunks);
     dp.task_target = reinterpret_cast<const u32 *>(b + o_tt);
     dp.task_cell = reinterpret_cast<const u32 *>(b + o_tc);
-    e.n_rounds = (u32)c.rt_round.size() - 1;
-    e.rt_round = reinterpret_cast<const u32 *>(b + o_rtr);
-    e.rt_target = reinterpret_cast<const u32 *>(b + o_rtt);
-    e.rt_cell = reinterpret_cast<const u32 *>(b + o_rtc);
-    e.rt_cells = reinterpret_cast<const uint16_t *>(b + o_rts);
     dp.cells = reinterpret_cast<const uint16_t *>(b + o_cells);
     dp.diag_slot = reinterpret_cast<const u32 *>(b + o_diag);
     dp.current_row = reinterpret_cast<const uint8_t *>(b + o_cur);
@@ -2084,13 +2087,17 @@ void build_reduce_streams(const Compiled &c, TapeHostProg &o)
             }
             if (!rows) return std::max<size_t>((words + esl::kWave - 1) / esl::kWave, left.empty() ? 0 : left[0]);
             at.assign(left.size(), 0);
+            vector<u32> pick;
+            auto most = [&](u32 a, u32 b) { return left[a] != left[b] ? left[a] > left[b] : a < b; };
             for (size_t done = 0; done < words;) {
-                vector<u32> pick;
+                pick.clear();
                 for (u32 k = 0; k < left.size(); k++)
                     if (left[k]) pick.push_back(k);
-                std::stable_sort(pick.begin(), pick.end(), [&](u32 a, u32 b) { return left[a] > left[b]; });
-                if (pick.size() > (size_t)esl::kWave) pick.resize(esl::kWave);
+                const size_t take = std::min<size_t>(pick.size(), esl::kWave);
+                std::partial_sort(pick.begin(), pick.begin() + take, pick.end(), most);
+                pick.resize(take);
                 vector<std::pair<u32, u32>> row;
+                row.reserve(take);
                 for (u32 k : pick) {
                     row.push_back({order[first + k], at[k]++});
                     left[k]--;
@@ -2428,10 +2435,6 @@ bool validate_deck(const Compiled &c)
     }
     for (u32 v : c.cslot_pat) if (v >= nnz) return false;
     for (u32 v : c.cells) if (v >= (u32)(esl::kWave * esl::kStageEntries)) return false;
-    if (c.rt_round.empty() || c.rt_round.front() != 0 || c.rt_round.back() != c.rt_target.size()) return false;
-    if ((c.rt_round.size() - 1) * esl::kTeam < c.chunks.size() - 1) return false;
-    if (c.rt_cell.size() != c.rt_target.size() + 1 || c.rt_cell.back() != c.rt_cells.size()) return false;
-    for (u32 v : c.rt_cells) if (v >= esl::kTeam * esl::kStageDoubles) return false;
     auto terms_ok = [&](const vector<u32> &t) {
         for (u32 v : t) if (v >= n) return false;
         return true;
@@ -3097,9 +3100,63 @@ u32 big_lds(const Engine &e)
     return esl::big_lds_doubles(e.c.n, bm);
 }
 
+// The reduce tasks of a big engine by rounds of kTeam chunks (BigArgs), on
+// the device: a round's targets, each with its cells in chunk order, the
+// longest first (the threads take them in turn). The deck's tasks and cells
+// were checked when the engine was created.
+esl_status big_rounds(Engine &e)
+{
+    if (e.n_rounds) return ESL_OK;
+    const Compiled &c = e.c;
+    const u32 nch = (u32)c.chunks.size() - 1, n = c.n, nnz = c.nnz, ncs = (u32)c.cslot_pat.size();
+    vector<u32> round, target, cell, at((size_t)nnz + 2 * n + ncs, NONE);
+    vector<uint16_t> cells;
+    auto place = [&](u32 t) {
+        const u32 idx = t & esl::kTargetMask;
+        return (t & esl::kRhsBit) ? nnz + idx : (t & esl::kQBit) ? nnz + n + idx : (t & esl::kCBit) ? nnz + 2 * n + idx : idx;
+    };
+    vector<std::pair<u32, vector<u32>>> lists;
+    for (u32 c0 = 0; c0 < nch; c0 += esl::kTeam) {
+        round.push_back((u32)target.size());
+        lists.clear();
+        for (u32 k = c0; k < std::min(nch, c0 + esl::kTeam); k++)
+            for (u32 tk = c.chunks[k].task_begin; tk < c.chunks[k + 1].task_begin; tk++) {
+                u32 &a = at[place(c.task_target[tk])];
+                if (a == NONE) {
+                    a = (u32)lists.size();
+                    lists.push_back({c.task_target[tk], {}});
+                }
+                for (u32 cc = c.task_cell[tk]; cc < c.task_cell[tk + 1]; cc++)
+                    lists[a].second.push_back((k - c0) * esl::kStageDoubles + c.cells[cc]);
+            }
+        for (auto &l : lists) at[place(l.first)] = NONE;
+        std::stable_sort(lists.begin(), lists.end(),
+                         [](auto &a, auto &b) { return a.second.size() > b.second.size(); });
+        for (auto &l : lists) {
+            target.push_back(l.first);
+            cell.push_back((u32)cells.size());
+            for (u32 v : l.second) cells.push_back((uint16_t)v);
+        }
+    }
+    static_assert(esl::kTeam * esl::kStageDoubles <= 65536, "16-bit cell indices");
+    round.push_back((u32)target.size());
+    cell.push_back((u32)cells.size());
+    Packer pk;
+    const size_t o_r = pk.add(round), o_t = pk.add(target), o_c = pk.add(cell), o_s = pk.add(cells);
+    HIPCHK(e.rounds_buf.ensure(pk.blob.size()));
+    HIPCHK(hipMemcpy(e.rounds_buf.p, pk.blob.data(), pk.blob.size(), hipMemcpyHostToDevice));
+    const unsigned char *b = e.rounds_buf.as<unsigned char>();
+    e.rt_round = reinterpret_cast<const u32 *>(b + o_r);
+    e.rt_target = reinterpret_cast<const u32 *>(b + o_t);
+    e.rt_cell = reinterpret_cast<const u32 *>(b + o_c);
+    e.rt_cells = reinterpret_cast<const uint16_t *>(b + o_s);
+    e.n_rounds = (u32)round.size() - 1;
+    return ESL_OK;
+}
+
 // The workspace of a big engine's launch over `lanes` lanes with up to
-// tv_cap factor slots each, and the kernel's LDS limit (set ahead of graph
-// capture).
+// tv_cap factor slots each, the kernel's LDS limit and the rounds (ahead of
+// graph capture).
 esl_status big_room(Engine &e, size_t lanes, u32 tv_cap)
 {
     const size_t stride = esl::big_stride(tv_cap, e.c.n, (u32)e.c.cslot_pat.size());
@@ -3110,7 +3167,7 @@ esl_status big_room(Engine &e, size_t lanes, u32 tv_cap)
         return ESL_FAILED;
     }
     HIPCHK(esl_big_attrs(lds));
-    return ESL_OK;
+    return big_rounds(e);
 }
 
 esl::BigArgs big_args(Engine &e, const esl::TranArgs &t, u32 lanes, u32 tran)

@@ -329,3 +329,51 @@ def test_ladder_matches_oracle_bitwise(lanes, oracle, stages, host_repivot):
     assert all(same_x)
     assert np.array_equal(got["iterations"], ref["iterations"])
     eng.close()
+
+
+def elimination_order(cp, ri, n, shallow):
+    """Minimum degree on the pattern of A + A^T as a scan of every vertex at
+    every step (ties to the lowest index); shallow: least 2 * degree +
+    level. Returns the order, its longest path and its fill."""
+    adj = [set() for _ in range(n)]
+    for j in range(n):
+        for i in ri[cp[j]:cp[j + 1]]:
+            if i != j:
+                adj[i].add(j)
+                adj[j].add(int(i))
+    level, gone, q, fill = [0] * n, [False] * n, [], 0
+    for _ in range(n):
+        v = min((v for v in range(n) if not gone[v]),
+                key=lambda v: (2 * len(adj[v]) + level[v] if shallow else len(adj[v]), v))
+        q.append(v)
+        gone[v] = True
+        nb, adj[v] = adj[v], set()
+        fill += len(nb)
+        for u in nb:
+            level[u] = max(level[u], level[v] + 1)
+            adj[u] = (adj[u] | nb) - {u, v}
+    return q, max(level), fill
+
+
+@pytest.mark.parametrize("fam,shallow", [
+    (circuits.rc_ladder(2), False), (circuits.diode_stack(3), True), (circuits.diode_stack(24), True),
+    (circuits.rc_ladder(97), True), (circuits.rc_mesh(9), False), (circuits.rc_mesh(14), False),
+    (circuits.inverter_chain(7), False), (circuits.ota_array(3), False), (circuits.diffpair_array(5), False),
+    (circuits.rc_ladder(780), True), (circuits.rc_ladder(900), False)], ids=lambda f: getattr(f, "name", f))
+def test_column_order_is_the_stated_one(lanes, fam, shallow):
+    """The engine's column order against a plain statement of it: minimum
+    degree, or for decks without transistors the shallow order where it at
+    least halves the longest path and leaves a lane half of a workgroup's
+    LDS (10,240 doubles for n + 2 fill + 8 n)."""
+    eng = lanes.Engine(fam.deck.arrays())
+    cp, ri, q = eng.pattern()
+    want, depth, _ = elimination_order(cp, ri, eng.n, False)
+    if not any(k in (5, 6) for k in fam.deck.kind) and 8 * depth >= eng.n:
+        q1, d1, f1 = elimination_order(cp, ri, eng.n, True)
+        took = 2 * d1 <= depth and 9 * eng.n + 2 * f1 <= 10240
+        assert took == shallow
+        want = q1 if took else want
+    else:
+        assert not shallow
+    assert list(q) == want
+    eng.close()
