@@ -205,15 +205,16 @@ __host__ __device__ inline uint32_t tran_doubles(uint32_t tv_cap, uint32_t n, ui
 }
 
 // A lane beyond a workgroup's LDS (a big lane) runs on a team of kTeam
-// wavefronts, one workgroup; its row programs are kTeamThreads wide.
+// wavefronts, one workgroup, or on one wavefront where its elimination is
+// narrow; its row programs are as wide as the team (kTeamThreads at most).
 constexpr uint32_t kTeam = 8;
 constexpr uint32_t kTeamThreads = kTeam * kWave;
 
 // One block of a big tape's replay: a run of consecutive ops of the row
 // program order whose slots fit LDS. The block gathers its m slots
 // (blk_slots[slot_off ...]) into LDS positions 0..m-1, runs its rows (words
-// [row][kTeamThreads] from row row0 of blk_words, indices into [m slots |
-// kTeamThreads pads]), then scatters the first w positions (the slots it
+// [row][team threads] from row row0 of blk_words, indices into [m slots |
+// a pad a thread]), then scatters the first w positions (the slots it
 // writes) back.
 struct BigBlock {
     uint32_t slot_off, m, w, rows;   // rows: a multiple of kRing
@@ -257,12 +258,12 @@ struct TapeProg {
     const uint32_t *li;         // [n_l] row (pivot step) of each L entry
     // big tapes (lanes whose slots live in HBM): the replay in blocks of at
     // most blk_m slots, and the solves as sol_rows rows of words
-    // [row][kTeamThreads] (kRing idle rows follow both programs)
+    // [row][team threads] (kRing idle rows follow both programs)
     uint32_t n_blk, blk_m, sol_rows, pad5;
     uint32_t pad6, pad7, pad8, pad9;
     const BigBlock *blk;        // [n_blk]
     const uint32_t *blk_slots;  // tv slots of each block's LDS positions
-    const uint2_t *blk_words;   // rows of all blocks, [row][kTeamThreads]
+    const uint2_t *blk_words;   // rows of all blocks, [row][team threads]
     const uint2_t *sol_w;
     const uint2_t *sol_pad;
     // chain segments of the refactor and solve programs: (word offset into
@@ -496,7 +497,7 @@ struct LptArgs {
 };
 
 // Arguments of the kernel for lanes whose working set is beyond a
-// workgroup's LDS (big_lanes): workgroup g, a team of kTeam wavefronts, runs
+// workgroup's LDS (big_lanes): workgroup g, `team` wavefronts (kTeam or 1), runs
 // lane ta.op.lane_ids[g], .op (tran == 0: the OpArgs of ta, modes 0-2, dump)
 // or transient steps (tran == 1). The lane's vectors and factor slots live
 // in HBM at ws + g * ws_stride: tv [tv_cap], then rhs, x, xold, sdiag, q [n
@@ -509,11 +510,11 @@ struct BigArgs {
     uint64_t ws_stride;
     uint32_t N, tran;
     uint32_t tv_cap, lds;
-    // the deck's reduce tasks by rounds of kTeam chunks: targets
+    // the deck's reduce tasks by rounds of `team` chunks: targets
     // rt_target[rt_round[r] .. rt_round[r + 1]), their cells from
     // rt_cell[...] on in instance order, cell indices chunk in the round *
     // kStageDoubles + staging index
-    uint32_t n_rounds, pad;
+    uint32_t n_rounds, team;
     const uint32_t *rt_round, *rt_target, *rt_cell;
     const uint16_t *rt_cells;
 };
@@ -522,15 +523,15 @@ __host__ __device__ inline size_t big_stride(uint32_t tv_cap, uint32_t n, uint32
     const size_t d = (size_t)tv_cap + 5 * (size_t)n + n_cslot;
     return (d + 15) / 16 * 16;   // 128-byte aligned lanes
 }
-// the LDS of a big lane: the staging cells of kTeam chunks, a replay block
-// of blk_m slots and its pads, or the solve vector and its pads; then the
-// reduction scratch
-constexpr uint32_t kTeamScratch = 2 * kTeam;
-__host__ __device__ inline uint32_t big_lds_doubles(uint32_t n, uint32_t blk_m)
+// the LDS of a big lane: the staging cells of a round's chunks, a replay
+// block of blk_m slots and its pads, or the solve vector and its pads; then
+// the reduction scratch
+__host__ __device__ constexpr uint32_t team_scratch(uint32_t team) { return 2 * team; }
+__host__ __device__ inline uint32_t big_lds_doubles(uint32_t n, uint32_t blk_m, uint32_t team)
 {
     uint32_t d = blk_m > n ? blk_m : n;
-    d += kTeamThreads;
-    return (kTeam * kStageDoubles > d ? kTeam * kStageDoubles : d) + kTeamScratch;
+    d += team * kWave;
+    return (team * kStageDoubles > d ? team * kStageDoubles : d) + team_scratch(team);
 }
 
 // Arguments of the LU-only replay (tape_replay).

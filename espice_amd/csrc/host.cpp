@@ -42,7 +42,7 @@ extern "C" hipError_t esl_launch_tran_steps(const void *ta, uint32_t grid, uint3
 extern "C" hipError_t esl_launch_batch(const void *b, uint32_t grid, uint32_t lds_bytes, hipStream_t s);
 extern "C" hipError_t esl_batch_occupancy(uint32_t lds_bytes, int *blocks_per_cu);
 extern "C" hipError_t esl_launch_big(const void *b, hipStream_t s);
-extern "C" hipError_t esl_big_attrs(uint32_t lds_bytes);
+extern "C" hipError_t esl_big_attrs(uint32_t team, uint32_t lds_bytes);
 extern "C" hipError_t esl_launch_pack(const double *src, size_t stride, size_t k, uint32_t count, double *out,
                                       hipStream_t s);
 extern "C" hipError_t esl_launch_gather(const double *x, uint32_t n, const uint32_t *ids, uint32_t k, uint32_t count,
@@ -331,11 +331,12 @@ vector<vector<u32>> sym_pattern(u32 n, const vector<u32> &col_ptr, const vector<
 }
 
 // An elimination order of a symmetric pattern. depth: its longest path;
-// fill: the entries of L (and of U). Empty q: the order passed a limit.
+// fill: the entries of L (and of U); work: the multiply-subtracts of a
+// factor. Empty q: the order passed a limit.
 struct Order {
     vector<u32> q;
     u32 depth = 0;
-    size_t fill = 0;
+    size_t fill = 0, work = 0;
 };
 
 // Minimum degree (ties to the lowest index). shallow: the next vertex is
@@ -369,6 +370,7 @@ Order min_degree(vector<vector<u32>> adj, bool shallow = false, u32 max_depth = 
         nb.clear();
         nb.swap(adj[v]);
         o.fill += nb.size();
+        o.work += nb.size() * nb.size();
         if (!nb.empty()) o.depth = std::max(o.depth, level[v] + 1);
         if (o.depth > max_depth || o.fill > max_fill) {
             o.q.clear();
@@ -407,19 +409,19 @@ Order min_degree(vector<vector<u32>> adj, bool shallow = false, u32 max_depth = 
 // order too: their stages have gain, so the rounding of another order can
 // move a point's iteration count (inverter chains: 60 % of the points),
 // where two-terminal decks agree to rounding in any order.
-vector<u32> deck_order(u32 n, const vector<u32> &col_ptr, const vector<u32> &row_idx, bool transistors)
+Order deck_order(u32 n, const vector<u32> &col_ptr, const vector<u32> &row_idx, bool transistors)
 {
     const vector<vector<u32>> adj = sym_pattern(n, col_ptr, row_idx);
     Order plain = min_degree(adj);
-    if (transistors || 8 * (size_t)plain.depth < n) return plain.q;   // a path of n / 8 columns: nothing like a line
+    if (transistors || 8 * (size_t)plain.depth < n) return plain;   // a path of n / 8 columns: nothing like a line
     // a lane holds its factors (n + 2 fill) and about eight n-vectors in
     // LDS: the shallow one may take half of a workgroup's, which keeps two
     // lanes on a CU (measured at 182 nodes; a line of more than about 800
     // nodes keeps the plain order, whatever that takes itself)
     constexpr size_t kHalf = 80 * 1024 / 8;
-    if (9 * (size_t)n > kHalf) return plain.q;
+    if (9 * (size_t)n > kHalf) return plain;
     Order sh = min_degree(adj, true, plain.depth / 2, (kHalf - 9 * (size_t)n) / 2);
-    return sh.q.empty() ? plain.q : sh.q;
+    return sh.q.empty() ? plain : sh;
 }
 
 // Row programs. Every update of the refactor or the solve is one op
@@ -752,6 +754,7 @@ struct TapeHostProg {
     // lanes beyond a workgroup's LDS: the replay in blocks and the solves in
     // chunks instead of whole-tape row programs and reduce streams
     bool big = false;
+    u32 width = 0;   // threads of a big lane: words a row
     vector<esl::BigBlock> blk;
     vector<u32> blk_slots;
     vector<esl::uint2_t> blk_words, sol_w;
@@ -967,13 +970,14 @@ void build_row_programs(const HostTape &t, TapeHostProg &o, u32 min_chain = kMin
 // 10,700 rows of 512 at 18,000. The solves: one program over the solve
 // vector, each factor entry read from its slot. False when a flop's target
 // lies outside its column.
-constexpr u32 kBigBlockSlots = 18944;
+constexpr u32 kBigBlockSlots = 18944, kNarrowBlockSlots = 4032;
 constexpr u32 kBigSlotLimit = 65536 - esl::kTeamThreads;   // 16-bit row-word indices
 
-bool build_big_program(const HostTape &t, TapeHostProg &o, u32 block_slots = kBigBlockSlots,
-                       u32 W = esl::kTeamThreads)
+bool build_big_program(const HostTape &t, TapeHostProg &o, u32 block_slots, u32 W)
 {
     const u32 n = t.n, nu = t.nnz_u;
+    o.big = true;
+    o.width = W;
     const esl::TapeProg &P = o.prog;
     const u32 lx0 = P.lx0, discard = P.discard;
     o.blk.clear();
@@ -1268,6 +1272,8 @@ struct Compiled {
     u32 kind_first[esl::kKinds + 1] = {};
     // deck program host arrays
     vector<esl::Chunk> chunks;
+    u32 order_depth = 0;     // of the column order: its longest path and the
+    size_t order_work = 0;   // multiply-subtracts of a factor
     vector<u32> task_target, task_cell;
     vector<uint16_t> cells;
     vector<u32> r_t, v_t, i_t, m_t;
@@ -1616,9 +1622,12 @@ bool compile_deck(const esl_deck *d, Compiled &c, std::string &err)
         else if (in.kind == esl::kQ)
             for (int e = 0; e < 12; e++) in.slot[e] = find_slot(c, in.t[BJT_ENT[e][0]], in.t[BJT_ENT[e][1]]);
     }
-    c.q = deck_order(n, c.col_ptr, c.row_idx,
-                     c.kind_first[esl::kMos] != c.kind_first[esl::kMos + 1] ||
-                         c.kind_first[esl::kQ] != c.kind_first[esl::kQ + 1]);
+    Order order = deck_order(n, c.col_ptr, c.row_idx,
+                             c.kind_first[esl::kMos] != c.kind_first[esl::kMos + 1] ||
+                                 c.kind_first[esl::kQ] != c.kind_first[esl::kQ + 1]);
+    c.order_depth = order.depth;
+    c.order_work = order.work;
+    c.q = std::move(order.q);
 
     // per-kind instance arrays
     for (auto &in : c.inst) {
@@ -1784,11 +1793,16 @@ struct Engine {
     Compiled c;
     DevBuf deck_buf;
     esl::DeckProg dp{};
-    // a big engine's reduce tasks by rounds (BigArgs), from its first launch on
-    DevBuf rounds_buf;
-    u32 n_rounds = 0;
-    const u32 *rt_round = nullptr, *rt_target = nullptr, *rt_cell = nullptr;
-    const uint16_t *rt_cells = nullptr;
+    // a big engine: the wavefronts of a lane in the solve that runs (set_team),
+    // and its reduce tasks by rounds (BigArgs) for kTeam wavefronts and for one,
+    // each from the first launch that needs it on
+    u32 team = 1;
+    struct Rounds {
+        DevBuf buf;
+        u32 count = 0;
+        const u32 *round = nullptr, *target = nullptr, *cell = nullptr;
+        const uint16_t *cells = nullptr;
+    } rounds[2];
     vector<TapeHostProg *> tapes;
     std::map<vector<u32>, u32> tape_index;
     DevBuf tape_table;
@@ -2237,8 +2251,10 @@ bool solve_rows_ok(const esl::uint2_t *words, size_t rows, u32 W, u32 lim, u32 n
 }
 
 // A big tape's blocks and solve program.
-bool validate_big(const TapeHostProg &o, u32 n, u32 W = esl::kTeamThreads)
+bool validate_big(const TapeHostProg &o, u32 n)
 {
+    const u32 W = o.width;
+    if (W != (u32)esl::kWave && W != esl::kTeamThreads) return false;
     const esl::TapeProg &P = o.prog;
     if (P.n_blk != o.blk.size() || o.blk_words.size() % W || n > kBigSlotLimit) return false;
     const size_t total_rows = o.blk_words.size() / W;
@@ -2493,13 +2509,16 @@ TapeHostProg *build_tape(const Engine &e, const HostTape &t, const char *&err)
     const bool fits = lds_bytes_for(tp->prog.n_tv, n) <= e.lds_limit && tp->prog.n_tv + n < 65536;
     err = nullptr;
     if (e.big || (!fits && e.tapes.empty())) {
-        tp->big = true;
         tp->diag_tv.assign(n, 0);
         for (u32 i = 0; i < n; i++) tp->diag_tv[i] = tp->amap[e.c.diag[i]];
-        // blocks as large as the LDS holds beside their pads
-        const u32 room = e.lds_limit / 8 - esl::kTeamThreads - esl::kTeamScratch;
-        if (!build_big_program(t, *tp, std::min(kBigSlotLimit, room))) err = "tape program failed validation";
-        else if ((size_t)esl::big_lds_doubles(n, tp->prog.blk_m) * 8 > e.lds_limit)
+        // a team's blocks are as large as the LDS holds beside their pads; a
+        // wavefront's leave room for three more lanes on its CU, unless its
+        // solve vector takes that anyway
+        const u32 W = e.team * esl::kWave;
+        const u32 room = e.lds_limit / 8 - W - esl::team_scratch(e.team);
+        const u32 slots = e.team == 1 ? std::max(kNarrowBlockSlots, n) : kBigSlotLimit;
+        if (!build_big_program(t, *tp, std::min(slots, room), W)) err = "tape program failed validation";
+        else if ((size_t)esl::big_lds_doubles(n, tp->prog.blk_m, e.team) * 8 > e.lds_limit)
             err = "too many unknowns for a lane's solve vector in LDS";
     } else if (!fits) {
         err = "lane state exceeds the LDS of one workgroup";
@@ -2521,10 +2540,12 @@ TapeHostProg *build_tape(const Engine &e, const HostTape &t, const char *&err)
     return tp;
 }
 
-vector<u32> tape_key(const HostTape &t)
+// A tape's pivot sequence, and for a big engine the team its programs are for.
+vector<u32> tape_key(const Engine &e, const HostTape &t)
 {
     vector<u32> key = t.pinv;
     key.insert(key.end(), t.flags.begin(), t.flags.end());
+    key.push_back(e.big ? e.team : 0);
     return key;
 }
 
@@ -2560,7 +2581,7 @@ esl_status register_tape(Engine &e, vector<u32> key, TapeHostProg *tp, u32 &id)
 // Registers a tape program (deduplicated by pivot sequence and flags).
 esl_status add_tape(Engine &e, const HostTape &t, u32 &id)
 {
-    vector<u32> key = tape_key(t);
+    vector<u32> key = tape_key(e, t);
     auto it = e.tape_index.find(key);
     if (it != e.tape_index.end()) {
         id = it->second;
@@ -2572,6 +2593,7 @@ esl_status add_tape(Engine &e, const HostTape &t, u32 &id)
         g_last_error = err;
         return ESL_FAILED;
     }
+    if (tp->big) key.back() = e.team;   // (this tape may be what makes the engine big)
     esl_status st = register_tape(e, std::move(key), tp, id);
     if (st != ESL_OK) return st;
     return upload_tape_table(e);
@@ -2782,9 +2804,8 @@ esl_status esl_debug_big_replay(uint32_t n, const uint32_t *col_ptr, const uint3
     vector<u32> cp(col_ptr, col_ptr + n + 1);
     TapeHostProg o;
     build_tape_prog(t, cp, 1e-12, 1.0 / pivot_tol, o);
-    o.big = true;
     if (block_slots == 0) block_slots = kBigBlockSlots;
-    if (!build_big_program(t, o, block_slots, W) || !validate_big(o, n, W)) return ESL_FAILED;
+    if (!build_big_program(t, o, block_slots, W) || !validate_big(o, n)) return ESL_FAILED;
     const esl::TapeProg &T = o.prog;
     if (sizes) {
         sizes[0] = T.n_blk;
@@ -3091,24 +3112,26 @@ esl_status launch_lpt(Engine &e, const HostOpArgs &a, u32 lanes, u32 mode, float
     return ESL_OK;
 }
 
-// The LDS of a big engine's lanes: the staging cells, its tapes' largest
-// replay block, or the solve vector.
+// The LDS of a big engine's lanes: the staging cells, the largest replay block
+// of its tapes for this team, or the solve vector.
 u32 big_lds(const Engine &e)
 {
     u32 bm = 0;
-    for (const TapeHostProg *t : e.tapes) bm = std::max(bm, t->prog.blk_m);
-    return esl::big_lds_doubles(e.c.n, bm);
+    for (const TapeHostProg *t : e.tapes)
+        if (t->width == e.team * esl::kWave) bm = std::max(bm, t->prog.blk_m);
+    return esl::big_lds_doubles(e.c.n, bm, e.team);
 }
 
-// The reduce tasks of a big engine by rounds of kTeam chunks (BigArgs), on
+// The reduce tasks of a big engine by rounds of its team's chunks (BigArgs), on
 // the device: a round's targets, each with its cells in chunk order, the
 // longest first (the threads take them in turn). The deck's tasks and cells
 // were checked when the engine was created.
 esl_status big_rounds(Engine &e)
 {
-    if (e.n_rounds) return ESL_OK;
+    Engine::Rounds &R = e.rounds[e.team == 1];
+    if (R.count) return ESL_OK;
     const Compiled &c = e.c;
-    const u32 nch = (u32)c.chunks.size() - 1, n = c.n, nnz = c.nnz, ncs = (u32)c.cslot_pat.size();
+    const u32 nch = (u32)c.chunks.size() - 1, n = c.n, nnz = c.nnz, ncs = (u32)c.cslot_pat.size(), team = e.team;
     vector<u32> round, target, cell, at((size_t)nnz + 2 * n + ncs, NONE);
     vector<uint16_t> cells;
     auto place = [&](u32 t) {
@@ -3116,10 +3139,10 @@ esl_status big_rounds(Engine &e)
         return (t & esl::kRhsBit) ? nnz + idx : (t & esl::kQBit) ? nnz + n + idx : (t & esl::kCBit) ? nnz + 2 * n + idx : idx;
     };
     vector<std::pair<u32, vector<u32>>> lists;
-    for (u32 c0 = 0; c0 < nch; c0 += esl::kTeam) {
+    for (u32 c0 = 0; c0 < nch; c0 += team) {
         round.push_back((u32)target.size());
         lists.clear();
-        for (u32 k = c0; k < std::min(nch, c0 + esl::kTeam); k++)
+        for (u32 k = c0; k < std::min(nch, c0 + team); k++)
             for (u32 tk = c.chunks[k].task_begin; tk < c.chunks[k + 1].task_begin; tk++) {
                 u32 &a = at[place(c.task_target[tk])];
                 if (a == NONE) {
@@ -3143,14 +3166,14 @@ esl_status big_rounds(Engine &e)
     cell.push_back((u32)cells.size());
     Packer pk;
     const size_t o_r = pk.add(round), o_t = pk.add(target), o_c = pk.add(cell), o_s = pk.add(cells);
-    HIPCHK(e.rounds_buf.ensure(pk.blob.size()));
-    HIPCHK(hipMemcpy(e.rounds_buf.p, pk.blob.data(), pk.blob.size(), hipMemcpyHostToDevice));
-    const unsigned char *b = e.rounds_buf.as<unsigned char>();
-    e.rt_round = reinterpret_cast<const u32 *>(b + o_r);
-    e.rt_target = reinterpret_cast<const u32 *>(b + o_t);
-    e.rt_cell = reinterpret_cast<const u32 *>(b + o_c);
-    e.rt_cells = reinterpret_cast<const uint16_t *>(b + o_s);
-    e.n_rounds = (u32)round.size() - 1;
+    HIPCHK(R.buf.ensure(pk.blob.size()));
+    HIPCHK(hipMemcpy(R.buf.p, pk.blob.data(), pk.blob.size(), hipMemcpyHostToDevice));
+    const unsigned char *b = R.buf.as<unsigned char>();
+    R.round = reinterpret_cast<const u32 *>(b + o_r);
+    R.target = reinterpret_cast<const u32 *>(b + o_t);
+    R.cell = reinterpret_cast<const u32 *>(b + o_c);
+    R.cells = reinterpret_cast<const uint16_t *>(b + o_s);
+    R.count = (u32)round.size() - 1;
     return ESL_OK;
 }
 
@@ -3166,7 +3189,7 @@ esl_status big_room(Engine &e, size_t lanes, u32 tv_cap)
         g_last_error = "too many unknowns for a lane's solve vector in LDS";
         return ESL_FAILED;
     }
-    HIPCHK(esl_big_attrs(lds));
+    HIPCHK(esl_big_attrs(e.team, lds));
     return big_rounds(e);
 }
 
@@ -3180,11 +3203,13 @@ esl::BigArgs big_args(Engine &e, const esl::TranArgs &t, u32 lanes, u32 tran)
     b.tran = tran;
     b.tv_cap = t.op.tv_cap;
     b.lds = big_lds(e);
-    b.n_rounds = e.n_rounds;
-    b.rt_round = e.rt_round;
-    b.rt_target = e.rt_target;
-    b.rt_cell = e.rt_cell;
-    b.rt_cells = e.rt_cells;
+    const Engine::Rounds &R = e.rounds[e.team == 1];
+    b.team = e.team;
+    b.n_rounds = R.count;
+    b.rt_round = R.round;
+    b.rt_target = R.target;
+    b.rt_cell = R.cell;
+    b.rt_cells = R.cells;
     return b;
 }
 
@@ -3231,6 +3256,29 @@ esl_status launch_lpw(Engine &e, HostOpArgs a, u32 lanes, u32 mode, u32 tv_cap, 
     return ESL_OK;
 }
 
+// The wavefronts of a lane of a big engine in a solve of `count` points.
+// Eight take one lane to its end soonest where the elimination is wide
+// enough to feed them (width: multiply-subtracts a column of its longest
+// path); one leaves a CU room for four lanes at once, so with more points than
+// CUs a team has to be that much faster. The lines lie where the two meet.
+// Kernel ms of an operating point and two steps, one wavefront : eight, at 64
+// and at 1,024 points (RC lines, strips and meshes of 1,600 to 4,100 unknowns):
+//   width    1 (line of 3,000)   47.5 : 74.4     58.3 : 299
+//   width   19 (4 x 900)         15.1 : 18.2     20.3 : 73.3
+//   width  141 (8 x 450)         12.4 :  8.7     18.1 : 35.5
+//   width  488 (12 x 300)        13.9 :  6.8     20.6 : 28.1
+//   width 1274 (16 x 220)        16.6 :  6.1     25.0 : 25.8
+//   width 2984 (40 x 40)         35.1 :  9.2     50.2 : 37.3
+//   width 9102 (64 x 64)          226 : 47.0      351 : 215
+u32 big_team(const Engine &e, size_t count)
+{
+    const size_t cu = std::max<size_t>(1, device_cu_count());
+    const size_t lds = 8 * (size_t)esl::big_lds_doubles(e.c.n, std::max(kNarrowBlockSlots, e.c.n), 1);
+    const size_t lanes = std::min<size_t>(4, std::max<size_t>(1, e.lds_limit / lds));
+    const size_t k = std::min((count + cu - 1) / cu, lanes);
+    return e.c.order_work >= 80 * k * k * e.c.order_depth ? esl::kTeam : 1;
+}
+
 // The solve's uploads, start vectors and Newton arguments, and the lead
 // tape (point 0's first Jacobian, factored on the host; lead_singular when
 // that matrix is singular).
@@ -3242,6 +3290,7 @@ esl_status op_prepare(Engine &E, const double *values, size_t count, const esl_o
     const Compiled &c = e->c;
     const u32 n = c.n, nnz = c.nnz, P = c.n_live;
     e->timing = esl_timing{};
+    if (e->big || e->tapes.empty()) e->team = big_team(*e, count);   // (the lead tape may make it big)
     HIPCHK(e->live.ensure(std::max<size_t>(1, count * P) * 8));
     HIPCHK(e->live_t.ensure(std::max<size_t>(1, count * P) * 8));
     HIPCHK(e->x.ensure(count * n * 8));
@@ -4664,7 +4713,7 @@ esl_status batch_item_repivot(BatchItemRun &r, vector<esl::BatchJob> &resume_job
     vector<size_t> build;
     for (size_t k = 0; k < na; k++) {
         if (!ok[k]) continue;
-        keys[k] = tape_key(ht[k]);
+        keys[k] = tape_key(*e, ht[k]);
         if (e->tape_index.count(keys[k])) continue;
         auto f = fresh.find(keys[k]);
         if (f != fresh.end()) {

@@ -510,10 +510,10 @@ def debug_big_rows(words, slots, solve=False):
 
 def debug_big_replay(col_ptr, row_idx, lead_vals, q, a, rhs, block_slots=4032, pivot_tol=1e-3, width=None):
     """The big-lane kernel's blocked refactor and row-program solves run on
-    the CPU (esl_debug_big_replay), rows of `width` words (64 or the
-    kernel's 512; by default 64 for blocks of fewer slots than that, whose
-    rows never fill), for a [lanes][nnz], rhs [lanes][n]: a development
-    check of the block programs, no device needed."""
+    the CPU (esl_debug_big_replay), rows of `width` words (64 for lanes on
+    one wavefront, 512 on eight; by default 64 for blocks of fewer slots
+    than that, whose rows never fill), for a [lanes][nnz], rhs [lanes][n]: a
+    development check of the block programs, no device needed."""
     width = width or (64 if block_slots < 64 else 512)
     L = load()
     cp, ri, qq = (np.ascontiguousarray(v, dtype=np.uint32) for v in (col_ptr, row_idx, q))
