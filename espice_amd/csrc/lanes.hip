@@ -1656,31 +1656,29 @@ __device__ inline BatchJob uni_job(const BatchJob &g)
 
 // One job on the lane's leader (nw > 1: with a crew): the operating point,
 // then, for a transient job whose point converged, the hand-over to the
-// transient tape and the steps.
+// transient tape and the steps; or a transient resumed at its saved step and
+// iterate (no .op arguments).
 __device__ __forceinline__ void run_job(const BatchArgs &b, const BatchJob &jb, double *base, uint32_t nw,
                                         uint32_t avail)
 {
-    const uint32_t tid = threadIdx.x % kWave;
-    if (jb.op == kNoArgs) {
-        // a transient resumed at its saved step and iterate
-        tran_lane<true>(b.trans[jb.tran], jb.lane, base, nw, avail);
-        return;
+    if (jb.op != kNoArgs) {
+        const uint32_t tid = threadIdx.x % kWave;
+        const OpArgs &oa = b.ops[jb.op];
+        const uint32_t st = op_lane<true>(oa, jb.lane, base, nw, avail);
+        if (jb.tran == kNoArgs || st != kConverged) return;
+        const TranArgs &ta = b.trans[jb.tran];
+        if (tid == 0) {
+            LaneResume r{};
+            r.tape = ta.tran_tape;
+            r.limit = 1e9;
+            ta.op.resume[jb.lane] = r;
+            ta.op.status[jb.lane] = kTranRunning;
+            ta.op.iterations[jb.lane] = 0;
+            ta.step[jb.lane] = 0;
+        }
+        wsync();
     }
-    const OpArgs &oa = b.ops[jb.op];
-    const uint32_t st = op_lane<true>(oa, jb.lane, base, nw, avail);
-    if (jb.tran == kNoArgs || st != kConverged) return;
-    const TranArgs &ta = b.trans[jb.tran];
-    if (tid == 0) {
-        LaneResume r{};
-        r.tape = ta.tran_tape;
-        r.limit = 1e9;
-        ta.op.resume[jb.lane] = r;
-        ta.op.status[jb.lane] = kTranRunning;
-        ta.op.iterations[jb.lane] = 0;
-        ta.step[jb.lane] = 0;
-    }
-    wsync();
-    tran_lane<true>(ta, jb.lane, base, nw, avail);
+    tran_lane<true>(b.trans[jb.tran], jb.lane, base, nw, avail);
 }
 
 __device__ __forceinline__ void follow_job(const BatchArgs &b, const BatchJob &jb, double *base, uint32_t wv)
@@ -1702,42 +1700,40 @@ __global__ __launch_bounds__(kWave * kCrew) void batch_run(BatchArgs b)
     __shared__ uint32_t claim;
     const uint32_t wv = threadIdx.x / kWave, tid = threadIdx.x % kWave;
     double *mine = sm + (size_t)wv * b.wave_doubles;
-    for (;;) {
-        uint32_t j = 0;
-        if (tid == 0) j = atomicAdd(b.next + 2, 1u);
-        j = uni(j);
-        if (j >= b.n_lead) break;
-        const uint64_t t0 = wall_clock64();
-        run_job(b, uni_job(b.wave_jobs[j]), mine, 1, b.wave_doubles);
-        if (b.wave_ticks && tid == 0) b.wave_ticks[j] = wall_clock64() - t0;
-    }
-    __syncthreads();
-    // lane per block: the whole workgroup on one lane at a time
-    for (;;) {
-        if (threadIdx.x == 0) claim = atomicAdd(b.next, 1u);
-        __syncthreads();
-        const uint32_t j = claim;
-        __syncthreads();
-        if (j >= b.n_block) break;
-        const BatchJob jb = uni_job(b.block_jobs[j]);
-        if (wv == 0) {
+    // lane per wavefront: each wavefront on its own lanes in its share of the
+    // LDS, first the lead jobs and at last the others (one loop for both: a
+    // copy of the job costs the build as much as a kernel)
+#pragma unroll 1
+    for (uint32_t last = 0; last < 2; last++) {
+        const uint32_t n_jobs = last ? b.n_wave : b.n_lead;
+        for (;;) {
+            uint32_t j = 0;
+            if (tid == 0) j = atomicAdd(b.next + (last ? 1 : 2), 1u);
+            j = uni(j);
+            if (j >= n_jobs) break;
             const uint64_t t0 = wall_clock64();
-            run_job(b, jb, sm, kCrew, kCrew * b.wave_doubles);
-            crew_done(tid);
-            if (b.block_ticks && tid == 0) b.block_ticks[j] = wall_clock64() - t0;
-        } else {
-            follow_job(b, jb, sm, wv);
+            run_job(b, uni_job(b.wave_jobs[j]), mine, 1, b.wave_doubles);
+            if (b.wave_ticks && tid == 0) b.wave_ticks[j] = wall_clock64() - t0;
         }
-    }
-    // lane per wavefront: each wavefront on its own lanes in its share of the LDS
-    for (;;) {
-        uint32_t j = 0;
-        if (tid == 0) j = atomicAdd(b.next + 1, 1u);
-        j = uni(j);
-        if (j >= b.n_wave) break;
-        const uint64_t t0 = wall_clock64();
-        run_job(b, uni_job(b.wave_jobs[j]), mine, 1, b.wave_doubles);
-        if (b.wave_ticks && tid == 0) b.wave_ticks[j] = wall_clock64() - t0;
+        if (last) break;
+        __syncthreads();
+        // lane per block: the whole workgroup on one lane at a time
+        for (;;) {
+            if (threadIdx.x == 0) claim = atomicAdd(b.next, 1u);
+            __syncthreads();
+            const uint32_t j = claim;
+            __syncthreads();
+            if (j >= b.n_block) break;
+            const BatchJob jb = uni_job(b.block_jobs[j]);
+            if (wv == 0) {
+                const uint64_t t0 = wall_clock64();
+                run_job(b, jb, sm, kCrew, kCrew * b.wave_doubles);
+                crew_done(tid);
+                if (b.block_ticks && tid == 0) b.block_ticks[j] = wall_clock64() - t0;
+            } else {
+                follow_job(b, jb, sm, wv);
+            }
+        }
     }
 }
 
