@@ -167,11 +167,10 @@ constexpr uint32_t kRedTarget = 0x80000000u, kRedRhs = 0x40000000u;
 // Reduce rows: words {x = target | c0 << 16, y = c1 | c2 << 16}, one per
 // thread of a row: the target takes the staged cells c0, c1, c2 in that
 // order; a target with more cells continues in later rows. target: a factor
-// slot below n_tv, n_tv + i for the double at rhs + i. kRedNone: no cell (it
-// reads as -0, which leaves any sum unchanged). Idle threads add nothing to
-// a scratch double behind the lane's working set, which holds two: that one
-// and the -0.
-constexpr uint32_t kRedNone = 0xffffu;
+// slot below n_tv, n_tv + i for the double at rhs + i. kRedNone (negative as
+// 16 bits): no cell; it reads the discard slot, which holds -0 during the
+// assembly and leaves any sum unchanged. Idle threads add that to itself.
+constexpr uint32_t kRedNone = 0x8000u;
 constexpr int kRedCells = 3;
 constexpr int kRedRing = 4;    // rows of words in flight; a stream is a multiple of it
 constexpr int kRing = 16;      // rows in flight; streams carry kRing pad rows
@@ -181,9 +180,9 @@ constexpr uint32_t kRedChainCells = 256;
 
 // Doubles of a lane's working set in LDS: tv_cap factor slots, the Y block
 // (y, sdiag, xold after the assembly; during it the stamp staging areas,
-// one per wavefront of the lane's crew), rhs, x, and the assembly reduce's
-// scratch pair. A transient lane's Y block holds y and xold, and q and the
-// charge-Jacobian cells follow x, then the scratch pair.
+// one per wavefront of the lane's crew), rhs, x, and a scratch pair (the
+// refinement's idle threads write its first). A transient lane's Y block holds
+// y and xold, and q and the charge-Jacobian cells follow x.
 constexpr uint32_t kStageDoubles = kWave * kStageEntries;
 __host__ __device__ inline uint32_t lds_y_block(uint32_t n, uint32_t nw = 1)
 {
@@ -201,7 +200,7 @@ __host__ __device__ inline uint32_t tran_y_block(uint32_t n, uint32_t nw = 1)
 }
 __host__ __device__ inline uint32_t tran_doubles(uint32_t tv_cap, uint32_t n, uint32_t n_cslot, uint32_t nw = 1)
 {
-    return tv_cap + tran_y_block(n, nw) + 3 * n + n_cslot + 2;
+    return tv_cap + tran_y_block(n, nw) + 3 * n + n_cslot;
 }
 
 // A lane beyond a workgroup's LDS (a big lane) runs on a team of kTeam

@@ -2071,7 +2071,7 @@ void build_reduce_streams(const Compiled &c, TapeHostProg &o)
     o.rc_coff.clear();
     o.rc_blocks.clear();
     const size_t nch = c.chunks.size() - 1;
-    const u32 n = c.n, n_tv = o.prog.n_tv, ncs = (u32)c.cslot_pat.size();
+    const u32 n = c.n, n_tv = o.prog.n_tv;
     for (size_t si = 0; si < 2 * nch; si++) {
         const size_t ci = si / 2;
         const bool tran = si % 2 != 0;
@@ -2145,7 +2145,7 @@ void build_reduce_streams(const Compiled &c, TapeHostProg &o)
         const size_t L = (rows.size() + esl::kRedRing - 1) / esl::kRedRing * esl::kRedRing;
         o.red_off.push_back((u32)o.red.size());
         o.red_len.push_back((u32)L);
-        const u32 idle = n_tv + (tran ? 3 * n + ncs : 2 * n);
+        const u32 idle = o.prog.discard;
         const size_t base = o.red.size();
         o.red.resize(base + (L + esl::kRedRing) * esl::kWave,
                      esl::uint2_t{idle | (esl::kRedNone << 16), esl::kRedNone | (esl::kRedNone << 16)});
@@ -2374,17 +2374,17 @@ bool validate_tape(const TapeHostProg &o, u32 n, u32 nnz, u32 ncs = 0)
     if (!rows_ok(o.rch, false) || !rows_ok(o.sch, true)) return false;
     for (u32 v : o.rsrc) if (v >= P.n_tv) return false;
     if (!o.red_off.empty()) {
-        // up to the transient's scratch double, and 16-bit targets
+        // up to the transient's last charge cell, and 16-bit targets
         const u32 lim = P.n_tv + 3 * n + ncs;
         if (o.red_len.size() != o.red_off.size() || o.red_off.size() % 2 || lim >= 0xffff) return false;
         if (o.red_h.size() != 2 * o.red_off.size() + 4 || o.rc_cells.size() >= (1u << 26)) return false;
         for (size_t si = 0; si < o.red_off.size(); si++) {
-            const u32 top = si % 2 ? lim : P.n_tv + 2 * n;   // the idle threads' scratch double
+            const u32 top = si % 2 ? lim : P.n_tv + n;
             const size_t rows = (size_t)o.red_len[si] + esl::kRedRing;
             if (o.red_len[si] > 0xffff || o.red_len[si] % esl::kRedRing || o.red_off[si] + rows * esl::kWave > o.red.size()) return false;
             for (size_t k = o.red_off[si]; k < o.red_off[si] + rows * esl::kWave; k++) {
                 const u32 cl[3] = {o.red[k].x >> 16, o.red[k].y & 0xffff, o.red[k].y >> 16};
-                if ((o.red[k].x & 0xffff) > top) return false;
+                if ((o.red[k].x & 0xffff) >= top) return false;
                 for (u32 v : cl)
                     if (v >= esl::kStageDoubles && v != esl::kRedNone) return false;
             }

@@ -203,7 +203,8 @@ __device__ inline void red_load(RedStream &r, ctape T, uint32_t tid)
 
 // Runs a stream on the staged cells at st0 (LDS addresses; tv0: the factor
 // slots, rhs8: what a rhs-side index adds to its slot number's address,
-// none: the double holding -0, above every staging cell). A row is bound by
+// none: the double holding -0, below every staging cell; a cell index is
+// signed and kRedNone's address lies below it). A row is bound by
 // its target's LDS round trip and three dependent adds, for up to three
 // cells a thread, where a stream of one word a cell took a round trip for
 // each cell. With the headers read a chunk ahead, cycles an iteration:
@@ -213,9 +214,9 @@ __device__ inline void red_load(RedStream &r, ctape T, uint32_t tid)
 __device__ inline void red_rows(RedStream &r, uint32_t tv0, uint32_t n_tv, uint32_t rhs8, uint32_t st0, uint32_t none)
 {
     using lp = __attribute__((address_space(3))) double *;
-    auto cell = [&](uint32_t c) {
-        const uint32_t a = st0 + c * 8u;
-        return *(lp)(uintptr_t)(a < none ? a : none);
+    auto cell = [&](int32_t c) {
+        const int32_t a = (int32_t)st0 + c * 8;
+        return *(lp)(uintptr_t)(uint32_t)(a > (int32_t)none ? a : (int32_t)none);
     };
     for (uint32_t row = 0; row < r.len; row += kRedRing) {
         r.w += kRedRing * kWave;
@@ -224,7 +225,7 @@ __device__ inline void red_rows(RedStream &r, uint32_t tv0, uint32_t n_tv, uint3
             const esl::uint2_t w = r.q[k];
             const uint32_t t = w.x & 0xffffu;
             const lp d = (lp)(uintptr_t)(tv0 + t * 8u + (t >= n_tv ? rhs8 : 0u));
-            const double v = *d, a0 = cell(w.x >> 16), a1 = cell(w.y & 0xffffu), a2 = cell(w.y >> 16);
+            const double v = *d, a0 = cell((int32_t)w.x >> 16), a1 = cell((int16_t)w.y), a2 = cell((int32_t)w.y >> 16);
             r.q[k] = esl::uint2_t{r.w[k * kWave].x, r.w[k * kWave].y};
             double acc = v + a0;
             acc = acc + a1;
@@ -281,17 +282,16 @@ __device__ inline void red_chains(esl::uint2_t hd, uint32_t nb, const uint32_t *
     *tgt = acc;
 }
 
-// One stream of a staged chunk: its rows, then its chains. idle: the header
-// of a thread without a chain (the scratch double).
-__device__ inline void red_stream(RedStream &r, ctape T, double *tv, double *rhs, double *stc, uint32_t none,
-                                  uint32_t idle, uint32_t tid)
+// One stream of a staged chunk: its rows, then its chains (a thread without
+// one adds nothing to the discard slot).
+__device__ inline void red_stream(RedStream &r, ctape T, double *tv, double *rhs, double *stc, uint32_t tid)
 {
     using lp = __attribute__((address_space(3))) double *;
     const uint32_t tv0 = (uint32_t)(uintptr_t)(lp)tv, rhs0 = (uint32_t)(uintptr_t)(lp)rhs;
     // the chains' cell indices load now, ahead of use
     const uint32_t nc = uni(r.a.y) >> 16;
     uint32_t tw0 = 0u, tw1 = 0u;
-    esl::uint2_t hd{idle, 0u};
+    esl::uint2_t hd{kRedTarget | T->discard, 0u};
     if (nc) {
         const __attribute__((address_space(1))) uint32_t *cg = gptr(T->rc_cells) + (uni(r.a.w) & 0x3ffffffu) + tid;
         tw0 = cg[0];
@@ -301,7 +301,7 @@ __device__ inline void red_stream(RedStream &r, ctape T, double *tv, double *rhs
             hd = esl::uint2_t{h.x, h.y};
         }
     }
-    red_rows(r, tv0, T->n_tv, rhs0 - tv0 - T->n_tv * 8u, (uint32_t)(uintptr_t)(lp)stc, none);
+    red_rows(r, tv0, T->n_tv, rhs0 - tv0 - T->n_tv * 8u, (uint32_t)(uintptr_t)(lp)stc, tv0 + T->discard * 8u);
     if (nc) {
         // the pad slots take the indices (the rows above use no pad)
         uint32_t *pw = reinterpret_cast<uint32_t *>(tv + T->pad_slot);
@@ -322,11 +322,8 @@ __device__ void assemble(const DeckProg &dp, ctape T, const double *live, const 
     const uint32_t n = dp.n;
     for (uint32_t i = tid; i < T->n_tv; i += kWave) tv[i] = 0.0;
     for (uint32_t i = tid; i < n; i += kWave) rhs[i] = 0.0;
-    if (tid == 0) rhs[2 * n + 1] = -0.0;
-    using lp = __attribute__((address_space(3))) double *;
-    const uint32_t none = (uint32_t)(uintptr_t)(lp)(rhs + 2 * n + 1);
-    const uint32_t idle = kRedTarget | kRedRhs | (2 * n);
     wsync();
+    if (tid == 0) tv[T->discard] = -0.0;   // no cell (kRedNone)
     RedStream r;
     red_head(r, T, 0);
     for (uint32_t c0 = 0; c0 < dp.n_chunks; c0 += cr.nw) {
@@ -342,7 +339,7 @@ __device__ void assemble(const DeckProg &dp, ctape T, const double *live, const 
             if (c != c0) red_load(r, T, tid);
             RedStream nx;
             red_head(nx, T, 2 * (c + 1));
-            red_stream(r, T, tv, rhs, st + (c - c0) * kStageDoubles, none, idle, tid);
+            red_stream(r, T, tv, rhs, st + (c - c0) * kStageDoubles, tid);
             r.a = nx.a;
             r.b = nx.b;
             wsync();
@@ -1080,12 +1077,8 @@ __device__ __forceinline__ void assemble_tran(const DeckProg &dp, ctape T, uint3
         q[i] = 0.0;
     }
     for (uint32_t k = tid; k < dp.n_cslot; k += kWave) cq[k] = 0.0;
-    // the reduce streams' scratch pair follows cq
-    if (T && tid == 0) cq[dp.n_cslot + 1] = -0.0;
-    using lp = __attribute__((address_space(3))) double *;
-    const uint32_t none = (uint32_t)(uintptr_t)(lp)(cq + dp.n_cslot + 1);
-    const uint32_t idle = kRedTarget | kRedRhs | (3 * n + dp.n_cslot);
     wsync();
+    if (T && tid == 0) tv[T->discard] = -0.0;   // no cell (kRedNone)
     RedStream r;
     if (T) red_head(r, T, 1);
     for (uint32_t c0 = 0; c0 < dp.n_chunks; c0 += cr.nw) {
@@ -1102,7 +1095,7 @@ __device__ __forceinline__ void assemble_tran(const DeckProg &dp, ctape T, uint3
                 if (c != c0) red_load(r, T, tid);
                 RedStream nx;
                 red_head(nx, T, 2 * (c + 1) + 1);
-                red_stream(r, T, tv, rhs, stc, none, idle, tid);
+                red_stream(r, T, tv, rhs, stc, tid);
                 r.a = nx.a;
                 r.b = nx.b;
             } else {

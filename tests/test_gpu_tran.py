@@ -293,3 +293,61 @@ def test_adaptive_rows_take_no_second_copy_on_the_device(lanes):
     assert (got["accepted"] == steps).all()
     assert used < 1.5 * rows
     eng.close()
+
+
+def test_a_lane_that_just_fills_a_workgroups_lds_runs(lanes, oracle):
+    """A transient lane's working set is its factor slots, the larger of two
+    n-vectors and the staging cells, three n-vectors and the charge cells,
+    and nothing beside: the lane that takes the last double of a workgroup's
+    LDS runs, bitwise the oracle's, and one double more is refused."""
+    import ctypes
+
+    static = ctypes.c_uint32()
+    assert lanes.load().esl_kernel_static_lds(ctypes.byref(static)) == 0
+    limit = (160 * 1024 - (static.value + 255) // 256 * 256) // 8
+
+    def line(nodes, caps):
+        """A line of resistors with `caps` of its nodes capacitive to ground."""
+        d = circuits.Deck(f"line_{nodes}_{caps}")
+        d.vsource("vs", "src", 0, 0.0, step_to=1.0, step_at=0.0)
+        prev = "src"
+        for k in range(nodes):
+            d.resistor(f"r{k}", prev, f"n{k}", 1e3)
+            d.bind(f"r{k}", 0, f"r{k}")
+            if k < caps:
+                d.capacitor(f"c{k}", f"n{k}", 0, 30e-15)
+            prev = f"n{k}"
+        return d
+
+    def doubles(eng, caps):
+        eng.solve_op(np.full((1, eng.n_live), 1e3))
+        n = eng.n
+        n_tv = eng.info().lds_bytes // 8 - max(3 * n, 1024) - 2 * n - 2
+        return n_tv + max(2 * n, 1024) + 3 * n + caps   # (a charge cell for each capacitor to ground)
+
+    # the longest line that fits, and as many capacitors as then fit
+    nodes = 2540
+    while True:
+        eng = lanes.Engine(line(nodes, 0).arrays())
+        caps = limit - doubles(eng, 0)
+        eng.close()
+        if caps > 0:
+            break
+        nodes -= 1
+    say(f"  limit {limit} doubles, line of {nodes} with {caps} capacitors")
+    assert caps < nodes
+    for extra in (0, 1):
+        d = line(nodes, caps + extra)
+        eng = lanes.Engine(d.arrays())
+        assert doubles(eng, caps + extra) == limit + extra
+        vals = 1e3 * (1 + 0.05 * np.random.default_rng(3).standard_normal((2, eng.n_live)))
+        if extra:
+            with pytest.raises(lanes.EslError):
+                eng.solve_tran(vals, 1e-12, 3, probes=[2, 3])
+        else:
+            _, _, q = eng.pattern()
+            got = eng.solve_tran(vals, 1e-12, 3, probes=[2, 3])
+            ref = oracle.tran(oracle.Circuit(d.arrays()), vals, q, 1e-12, 3, probes=[2, 3], threads=2)
+            assert np.array_equal(got["iterations"], ref["iterations"])
+            assert np.array_equal(bits(got["x"]), bits(ref["x"]))
+        eng.close()
