@@ -377,3 +377,57 @@ def test_column_order_is_the_stated_one(lanes, fam, shallow):
         assert not shallow
     assert list(q) == want
     eng.close()
+
+
+def chain_with_floats(stages, floats):
+    """An inverter chain and `floats` nodes that only capacitors touch: void
+    unknowns of its operating point."""
+    fam = circuits.inverter_chain(stages)
+    for k in range(floats):
+        fam.deck.capacitor(f"cf{k}", f"f{k}", 0, 1e-14)
+    return fam
+
+
+@pytest.mark.parametrize("stages,floats", [(2, 0), (58, 0), (59, 0), (60, 0), (20, 3), (56, 3)])
+def test_own_lu_of_small_lanes_bitwise(lanes, oracle, stages, floats):
+    """Lanes that re-pivot hold their own factors dense in LDS up to 64
+    unknowns where it has room (a few lanes), and sparse beyond (65
+    unknowns), with void unknowns, and where many lanes leave no room: the
+    same bits on every path, the oracle's."""
+    fam = chain_with_floats(stages, floats)
+    eng = lanes.Engine(fam.deck.arrays())
+    assert eng.n == stages + 5 + floats
+    vals = fam.sample(78, 4500)
+    _, _, q = eng.pattern()
+    t = lanes.default_options().tol
+    t.max_iter = 150
+    few = eng.solve_op(vals[:48], tiling=lanes.TILING_WAVE, tol=t)
+    own = eng.timing().device_repivot_lanes
+    ref = oracle.Circuit(fam.deck.arrays()).op(vals[:48], q, threads=8,
+                                               tol=oracle.Tol(t.reltol, t.abstol, t.vntol, t.residual_tol, 150, 0))
+    say(f"  n {eng.n}: {own} of 48 lanes on their own LU, converged {(ref['reasons'] == 0).sum()}/48")
+    assert stages < 16 or own > 0
+    many = eng.solve_op(vals, tiling=lanes.TILING_WAVE, tol=t)
+    assert stages < 16 or eng.timing().device_repivot_lanes > 2048   # eight and more a CU
+    for got in (few, many):
+        assert np.array_equal(got["reasons"][:48], ref["reasons"])
+        assert np.array_equal(got["iterations"][:48], ref["iterations"])
+        assert np.array_equal(bits(got["x"][:48]), bits(ref["x"]))
+    eng.close()
+
+
+@pytest.mark.parametrize("stages,count,tuned", [(43, 1024, True), (43, 1023, False), (44, 1024, False)])
+def test_the_tilings_are_tried_up_to_48_unknowns(lanes, stages, count, tuned):
+    """48 and 49 unknowns: a first batch of 1,024 points times both tilings
+    up to 48 unknowns and runs one wavefront a lane beyond; the results are
+    the wavefront tiling's either way."""
+    fam = circuits.inverter_chain(stages)
+    eng = lanes.Engine(fam.deck.arrays())
+    assert eng.n == stages + 5
+    vals = fam.sample(79, count)
+    got = eng.solve_op(vals)
+    assert (eng.info().tiling != 0) == tuned
+    ref = eng.solve_op(vals, tiling=lanes.TILING_WAVE)
+    assert np.array_equal(got["iterations"], ref["iterations"])
+    assert np.array_equal(bits(got["x"]), bits(ref["x"]))
+    eng.close()

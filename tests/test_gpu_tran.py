@@ -351,3 +351,47 @@ def test_a_lane_that_just_fills_a_workgroups_lds_runs(lanes, oracle):
             assert np.array_equal(got["iterations"], ref["iterations"])
             assert np.array_equal(bits(got["x"]), bits(ref["x"]))
         eng.close()
+
+
+@pytest.mark.parametrize("kind,count", [("r", 16), ("r", 17), ("r", 63), ("r", 64), ("r", 65), ("r", 200), ("c", 64),
+                                        ("d", 40), ("d", 64), ("m", 33), ("m", 64), ("q", 17), ("q", 64)])
+def test_rails_of_many_devices_step_bitwise(lanes, oracle, kind, count):
+    """A rail that every device of a kind hangs from: its Jacobian entry,
+    residual row and charge collect up to 64 cells a chunk, as chains where
+    they are long (slots and residuals of more than 16 cells) and as rows of
+    three cells a word otherwise. The sums keep the device order: operating
+    points and steps are bitwise the oracle's."""
+    d = circuits.Deck(f"rail_{kind}_{count}")
+    d.vsource("vs", "src", 0, 0.6, step_to=0.7, step_at=0.0)
+    d.resistor("rs", "src", "rail", 10.0)
+    for k in range(count):
+        a = f"a{k % 7}"   # a few nodes share many devices too
+        if kind == "r":
+            d.resistor(f"x{k}", "rail", a, 1e3 * (1 + 0.01 * k))
+        elif kind == "c":
+            d.capacitor(f"x{k}", "rail", a, 1e-14 * (1 + 0.01 * k))
+        elif kind == "d":
+            d.diode(f"x{k}", "rail", a, {"is": 1e-15 * (1 + 0.01 * k), "cjo": 1e-14})
+        elif kind == "m":
+            d.mos1(f"x{k}", "rail", "rail", a, 0, {"type": 1, "vto": 0.2 + 0.001 * k, "kp": 2e-4, "cgso": 1e-10}, w=1e-6, l=1e-7)
+        else:
+            d.bjt(f"x{k}", "rail", "rail", a, 0, {"type": 1, "is": 1e-16 * (1 + 0.01 * k), "bf": 100.0})
+    for k in range(7):
+        d.resistor(f"g{k}", f"a{k}", 0, 500.0)
+        d.bind(f"g{k}", 0, f"g{k}")
+        d.capacitor(f"h{k}", f"a{k}", 0, 1e-14)
+    d.capacitor("cr", "rail", 0, 1e-14)
+    vals = 500.0 * (1 + 0.1 * np.random.default_rng(4).standard_normal((9, 7)))
+    eng = lanes.Engine(d.arrays())
+    _, _, q = eng.pattern()
+    c = oracle.Circuit(d.arrays())
+    op = eng.solve_op(vals)
+    ref = c.op(vals, q, threads=8)
+    assert (op["reasons"] == 0).all()
+    assert np.array_equal(op["iterations"], ref["iterations"]) and np.array_equal(bits(op["x"]), bits(ref["x"]))
+    got = eng.solve_tran(vals, 1e-12, 5, probes=[2, 3])
+    ref = oracle.tran(c, vals, q, 1e-12, 5, probes=[2, 3], threads=8)
+    assert np.array_equal(got["reasons"], ref["reasons"]) and np.array_equal(got["iterations"], ref["iterations"])
+    assert np.array_equal(bits(got["probes"]), bits(ref["probes"]))
+    assert np.array_equal(bits(got["x"]), bits(ref["x"]))
+    eng.close()
