@@ -3426,6 +3426,10 @@ esl_status op_repivot(Engine &E, const HostOpArgs &a, size_t count, vector<u32> 
             e->timing.fp64_lanes += (u32)to64.size();
             HIPCHK(hipMemcpyAsync(e->lane64.p, lane64.data(), count, hipMemcpyHostToDevice, s));
         }
+        // the tapes the lanes stand on, for the launch's room too (a lane that
+        // only goes on in FP64 keeps its own, whatever it is)
+        HIPCHK(hipMemcpyAsync(rs.data(), e->resume.p, count * sizeof(esl::LaneResume), hipMemcpyDeviceToHost, s));
+        HIPCHK(hipStreamSynchronize(s));
         vector<u32> next = to64;
         if (!again.empty()) {
         HIPCHK(e->a_out.ensure(again.size() * nnz * 8));
@@ -3445,7 +3449,6 @@ esl_status op_repivot(Engine &E, const HostOpArgs &a, size_t count, vector<u32> 
         if (r != ESL_OK) return r;
         vector<double> A(again.size() * (size_t)nnz);
         HIPCHK(hipMemcpyAsync(A.data(), e->a_out.p, A.size() * 8, hipMemcpyDeviceToHost, s));
-        HIPCHK(hipMemcpyAsync(rs.data(), e->resume.p, count * sizeof(esl::LaneResume), hipMemcpyDeviceToHost, s));
         HIPCHK(hipStreamSynchronize(s));
         for (size_t k = 0; k < again.size(); k++) {
             const u32 l = again[k];

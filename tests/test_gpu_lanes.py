@@ -431,3 +431,27 @@ def test_the_tilings_are_tried_up_to_48_unknowns(lanes, stages, count, tuned):
     assert np.array_equal(got["iterations"], ref["iterations"])
     assert np.array_equal(bits(got["x"]), bits(ref["x"]))
     eng.close()
+
+
+@pytest.mark.parametrize("stages", [12, 24, 40])
+def test_fp32_lanes_that_stall_on_a_later_tape_go_on_in_fp64(lanes, stages):
+    """Lanes whose refinement stalls go on in FP64 on the tape they stand on.
+    Here the engine's first tape has fewer factor slots than this solve's
+    lead: the launch must have room for the lead's, and the results are the
+    FP64 lanes' bit for bit."""
+    fam = circuits.inverter_chain(stages)
+    vals = fam.sample(3, 4)
+    eng = lanes.Engine(fam.deck.arrays())
+    eng.solve_op(vals)
+    first = eng.info().lds_bytes
+    x0 = np.random.default_rng(5).uniform(-0.2, 1.2, (4, eng.n))
+    x0[:, 0] = 0
+    t = lanes.default_options().tol
+    t.max_iter = 400
+    got = eng.solve_op(vals, x0=x0, precision=lanes.FP32_REFINED, refine_tol=0.0, refine_max=1, tol=t)
+    assert eng.timing().fp64_lanes == 4 and eng.info().lds_bytes > first
+    ref = eng.solve_op(vals, x0=x0, tiling=lanes.TILING_WAVE, tol=t)
+    assert (ref["reasons"] == 0).all()
+    assert np.array_equal(got["iterations"], ref["iterations"])
+    assert np.array_equal(bits(got["x"]), bits(ref["x"]))
+    eng.close()
