@@ -40,9 +40,8 @@ __device__ inline double wave_fmax(double v)
 }
 
 // Keeps a value in a vector register at this point: its computation is
-// neither moved past here nor speculated above it. Only 32-bit operands: the
-// "v" constraint may give a 64-bit one a register pair that starts at an odd
-// register, which gfx950 instructions cannot address.
+// neither moved past here nor speculated above it. A double is pinned by its
+// low word, which whatever uses the value then waits for.
 __device__ inline void pin(uint32_t &v)
 {
 #if defined(__HIP_DEVICE_COMPILE__)

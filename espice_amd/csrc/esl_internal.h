@@ -259,12 +259,10 @@ struct TapeProg {
     // most blk_m slots, and the solves as sol_rows rows of words
     // [row][team threads] (kRing idle rows follow both programs)
     uint32_t n_blk, blk_m, sol_rows, pad5;
-    uint32_t pad6, pad7, pad8, pad9;
     const BigBlock *blk;        // [n_blk]
     const uint32_t *blk_slots;  // tv slots of each block's LDS positions
     const uint2_t *blk_words;   // rows of all blocks, [row][team threads]
     const uint2_t *sol_w;
-    const uint2_t *sol_pad;
     // chain segments of the refactor and solve programs: (word offset into
     // the terms, blocks) each, and their terms
     const uint2_t *rseg, *sseg;

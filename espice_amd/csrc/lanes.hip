@@ -1063,7 +1063,10 @@ __global__ __launch_bounds__(kWave) void op_newton_own(OpArgs a)
 // (lane_kernels.zig:194-215). q1 and i_prev are the lane's rows in global
 // memory. Jacobian entries go to the tape's slots (T null: tv[slot], the pattern
 // order, by the deck's reduce tasks). A crew of nw wavefronts evaluates nw
-// chunks per round.
+// chunks per round. Inlined: as a call it costs the step loop its registers (16
+// bipolar pairs 5.3 -> 11.6 ms, an RC line of 182 nodes 10.3 -> 14.3 ms), and
+// the compiler refuses that kernel (it moves a 64-bit spill reload onto an odd
+// register pair) unless its copy propagation is off.
 __device__ __forceinline__ void assemble_tran(const DeckProg &dp, ctape T, uint32_t n_slots, const double *live,
                               const double *x, double *lim, uint32_t nm, double *tv, double *rhs, double *q,
                               double *cq, double *st, double t, double ag0, double ag1, const double *q1,
