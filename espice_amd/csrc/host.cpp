@@ -4421,26 +4421,27 @@ struct BatchItemRun {
 };
 
 // Model of one job's time before any measurement: the rows a Newton
-// iteration runs (refactor, solves, assembly reduce) times a typical
-// iteration count; the lane-per-block tiling evaluates devices on four
+// iteration runs (refactor, solves, the analysis' own assembly reduce) times a
+// typical iteration count; the lane-per-block tiling evaluates devices on four
 // wavefronts.
 void model_job_ns(const BatchItemRun &r, double out[2])
 {
     const Engine &e = *r.e;
-    auto rows = [&](u32 tape) {
+    auto rows = [&](u32 tape, bool tran) {   // red_len: an .op and a transient stream a chunk
         const TapeHostProg &t = *e.tapes[tape];
         double red = 0;
-        for (size_t k = 0; k < t.red_len.size(); k += 2) red += t.red_len[k];
+        for (size_t k = tran ? 1 : 0; k < t.red_len.size(); k += 2) red += t.red_len[k];
         return (double)t.prog.rw_rows + t.prog.sw_rows + red;
     };
     const double chunks = (double)e.c.chunks.size() - 1;
-    double w = (rows(e.lead_id) + 40.0 * chunks) * 8.0, b = (rows(e.lead_id) + 10.0 * chunks) * 8.0;
+    const double per_op = rows(e.lead_id, false);
+    double w = (per_op + 40.0 * chunks) * 8.0, b = (per_op + 10.0 * chunks) * 8.0;
     if (r.tran && !r.tran_singular) {
-        const double per = rows(r.ta.tran_tape);
+        const double per = rows(r.ta.tran_tape, true);
         w += (per + 40.0 * chunks) * 3.0 * r.ta.steps;
         b += (per + 10.0 * chunks) * 3.0 * r.ta.steps;
     }
-    out[0] = 100.0 * w;   // ~100 ns per row of a latency-bound wavefront
+    out[0] = 100.0 * w;   // ~100 ns per row of a latency-bound wavefront (a row program's 95, a reduce row's 60)
     out[1] = 100.0 * b;
 }
 
