@@ -167,9 +167,11 @@ constexpr uint32_t kRedTarget = 0x80000000u, kRedRhs = 0x40000000u;
 // Reduce rows: words {x = target | c0 << 16, y = c1 | c2 << 16}, one per
 // thread of a row: the target takes the staged cells c0, c1, c2 in that
 // order; a target with more cells continues in later rows. target: a factor
-// slot below n_tv, n_tv + i for the double at rhs + i. kRedNone (negative as
-// 16 bits): no cell; it reads the discard slot, which holds -0 during the
-// assembly and leaves any sum unchanged. Idle threads add that to itself.
+// slot below n_tv, n_tv + i for the double at rhs + i. kRedNone (far from any
+// cell, as a signed index and as an unsigned one): no cell; it reads a double
+// that holds -0 during the assembly and leaves any sum unchanged: the scratch
+// pair's second of an operating point, the discard slot of a transient. Idle
+// threads have no cells and the discard slot for a target.
 constexpr uint32_t kRedNone = 0x8000u;
 constexpr int kRedCells = 3;
 constexpr int kRedRing = 4;    // rows of words in flight; a stream is a multiple of it
@@ -180,8 +182,8 @@ constexpr uint32_t kRedChainCells = 256;
 
 // Doubles of a lane's working set in LDS: tv_cap factor slots, the Y block
 // (y, sdiag, xold after the assembly; during it the stamp staging areas,
-// one per wavefront of the lane's crew), rhs, x, and a scratch pair (the
-// refinement's idle threads write its first). A transient lane's Y block holds
+// one per wavefront of the lane's crew), rhs, x, and a scratch pair (what idle
+// threads write; the assembly reduce's -0). A transient lane's Y block holds
 // y and xold, and q and the charge-Jacobian cells follow x.
 constexpr uint32_t kStageDoubles = kWave * kStageEntries;
 __host__ __device__ inline uint32_t lds_y_block(uint32_t n, uint32_t nw = 1)

@@ -203,20 +203,27 @@ __device__ inline void red_load(RedStream &r, ctape T, uint32_t tid)
 
 // Runs a stream on the staged cells at st0 (LDS addresses; tv0: the factor
 // slots, rhs8: what a rhs-side index adds to its slot number's address,
-// none: the double holding -0, below every staging cell; a cell index is
-// signed and kRedNone's address lies below it). A row is bound by
+// none: the double holding -0; kBelow: below every staging cell, the cell
+// indices read as signed, kRedNone's address below it; otherwise above them,
+// read as unsigned, kRedNone's above it). A row is bound by
 // its target's LDS round trip and three dependent adds, for up to three
 // cells a thread, where a stream of one word a cell took a round trip for
 // each cell. With the headers read a chunk ahead, cycles an iteration:
 // assembly of the 64-OTA array 106.9 k -> 86.3 k, of the mirror tree of
 // depth 6 109.6 k -> 66.9 k, of 8 diodes 15.9 k -> 9.9 k; the transient of
 // 16 bipolar pairs, whose reduce walked task tables, 7.28 -> 6.42 ms.
+template <bool kBelow>
 __device__ inline void red_rows(RedStream &r, uint32_t tv0, uint32_t n_tv, uint32_t rhs8, uint32_t st0, uint32_t none)
 {
     using lp = __attribute__((address_space(3))) double *;
-    auto cell = [&](int32_t c) {
-        const int32_t a = (int32_t)st0 + c * 8;
-        return *(lp)(uintptr_t)(uint32_t)(a > (int32_t)none ? a : (int32_t)none);
+    auto cell = [&](uint32_t c) {
+        if constexpr (kBelow) {
+            const int32_t a = (int32_t)st0 + (int16_t)c * 8;
+            return *(lp)(uintptr_t)(uint32_t)(a > (int32_t)none ? a : (int32_t)none);
+        } else {
+            const uint32_t a = st0 + c * 8u;
+            return *(lp)(uintptr_t)(a < none ? a : none);
+        }
     };
     for (uint32_t row = 0; row < r.len; row += kRedRing) {
         r.w += kRedRing * kWave;
@@ -225,7 +232,7 @@ __device__ inline void red_rows(RedStream &r, uint32_t tv0, uint32_t n_tv, uint3
             const esl::uint2_t w = r.q[k];
             const uint32_t t = w.x & 0xffffu;
             const lp d = (lp)(uintptr_t)(tv0 + t * 8u + (t >= n_tv ? rhs8 : 0u));
-            const double v = *d, a0 = cell((int32_t)w.x >> 16), a1 = cell((int16_t)w.y), a2 = cell((int32_t)w.y >> 16);
+            const double v = *d, a0 = cell(w.x >> 16), a1 = cell(w.y & 0xffffu), a2 = cell(w.y >> 16);
             r.q[k] = esl::uint2_t{r.w[k * kWave].x, r.w[k * kWave].y};
             double acc = v + a0;
             acc = acc + a1;
@@ -282,16 +289,18 @@ __device__ inline void red_chains(esl::uint2_t hd, uint32_t nb, const uint32_t *
     *tgt = acc;
 }
 
-// One stream of a staged chunk: its rows, then its chains (a thread without
-// one adds nothing to the discard slot).
-__device__ inline void red_stream(RedStream &r, ctape T, double *tv, double *rhs, double *stc, uint32_t tid)
+// One stream of a staged chunk: its rows, then its chains. none: the address of
+// the -0 (red_rows); idle: the header of a thread without a chain.
+template <bool kBelow>
+__device__ inline void red_stream(RedStream &r, ctape T, double *tv, double *rhs, double *stc, uint32_t none,
+                                  uint32_t idle, uint32_t tid)
 {
     using lp = __attribute__((address_space(3))) double *;
     const uint32_t tv0 = (uint32_t)(uintptr_t)(lp)tv, rhs0 = (uint32_t)(uintptr_t)(lp)rhs;
     // the chains' cell indices load now, ahead of use
     const uint32_t nc = uni(r.a.y) >> 16;
     uint32_t tw0 = 0u, tw1 = 0u;
-    esl::uint2_t hd{kRedTarget | T->discard, 0u};
+    esl::uint2_t hd{idle, 0u};
     if (nc) {
         const __attribute__((address_space(1))) uint32_t *cg = gptr(T->rc_cells) + (uni(r.a.w) & 0x3ffffffu) + tid;
         tw0 = cg[0];
@@ -301,7 +310,7 @@ __device__ inline void red_stream(RedStream &r, ctape T, double *tv, double *rhs
             hd = esl::uint2_t{h.x, h.y};
         }
     }
-    red_rows(r, tv0, T->n_tv, rhs0 - tv0 - T->n_tv * 8u, (uint32_t)(uintptr_t)(lp)stc, tv0 + T->discard * 8u);
+    red_rows<kBelow>(r, tv0, T->n_tv, rhs0 - tv0 - T->n_tv * 8u, (uint32_t)(uintptr_t)(lp)stc, none);
     if (nc) {
         // the pad slots take the indices (the rows above use no pad)
         uint32_t *pw = reinterpret_cast<uint32_t *>(tv + T->pad_slot);
@@ -322,8 +331,13 @@ __device__ void assemble(const DeckProg &dp, ctape T, const double *live, const 
     const uint32_t n = dp.n;
     for (uint32_t i = tid; i < T->n_tv; i += kWave) tv[i] = 0.0;
     for (uint32_t i = tid; i < n; i += kWave) rhs[i] = 0.0;
+    // no cell (kRedNone): the second of the scratch pair behind x, which an
+    // operating point has anyway (the cheaper form by 1.7 % of a small solve)
+    if (tid == 0) rhs[2 * n + 1] = -0.0;
+    using lp = __attribute__((address_space(3))) double *;
+    const uint32_t none = (uint32_t)(uintptr_t)(lp)(rhs + 2 * n + 1);
+    const uint32_t idle = kRedTarget | kRedRhs | (2 * n);
     wsync();
-    if (tid == 0) tv[T->discard] = -0.0;   // no cell (kRedNone)
     RedStream r;
     red_head(r, T, 0);
     for (uint32_t c0 = 0; c0 < dp.n_chunks; c0 += cr.nw) {
@@ -339,7 +353,7 @@ __device__ void assemble(const DeckProg &dp, ctape T, const double *live, const 
             if (c != c0) red_load(r, T, tid);
             RedStream nx;
             red_head(nx, T, 2 * (c + 1));
-            red_stream(r, T, tv, rhs, st + (c - c0) * kStageDoubles, tid);
+            red_stream<false>(r, T, tv, rhs, st + (c - c0) * kStageDoubles, none, idle, tid);
             r.a = nx.a;
             r.b = nx.b;
             wsync();
@@ -1072,7 +1086,7 @@ __device__ __forceinline__ void assemble_tran(const DeckProg &dp, ctape T, uint3
                               double *cq, double *st, double t, double ag0, double ag1, const double *q1,
                               const double *ip, uint32_t tid, const Crew &cr)
 {
-    const uint32_t n = dp.n;
+    const uint32_t n = dp.n, disc = T ? T->discard : 0u;
     const uint32_t *amap = T ? T->amap : nullptr;
     for (uint32_t i = tid; i < n_slots; i += kWave) tv[i] = 0.0;
     for (uint32_t i = tid; i < n; i += kWave) {
@@ -1080,8 +1094,11 @@ __device__ __forceinline__ void assemble_tran(const DeckProg &dp, ctape T, uint3
         q[i] = 0.0;
     }
     for (uint32_t k = tid; k < dp.n_cslot; k += kWave) cq[k] = 0.0;
+    // no cell (kRedNone): the discard slot, so that the working set ends with cq
+    if (T && tid == 0) tv[disc] = -0.0;
+    using lp = __attribute__((address_space(3))) double *;
+    const uint32_t none = (uint32_t)(uintptr_t)(lp)(tv + disc), idle = kRedTarget | disc;
     wsync();
-    if (T && tid == 0) tv[T->discard] = -0.0;   // no cell (kRedNone)
     RedStream r;
     if (T) red_head(r, T, 1);
     for (uint32_t c0 = 0; c0 < dp.n_chunks; c0 += cr.nw) {
@@ -1098,7 +1115,7 @@ __device__ __forceinline__ void assemble_tran(const DeckProg &dp, ctape T, uint3
                 if (c != c0) red_load(r, T, tid);
                 RedStream nx;
                 red_head(nx, T, 2 * (c + 1) + 1);
-                red_stream(r, T, tv, rhs, stc, tid);
+                red_stream<true>(r, T, tv, rhs, stc, none, idle, tid);
                 r.a = nx.a;
                 r.b = nx.b;
             } else {
