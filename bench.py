@@ -439,7 +439,7 @@ def run_mesh(args):
         "data": "synthetic (seeded R, C and IS draws per point)",
         "config": {"workload": f"rc_mesh 64x64 + 5% diode clamps, {len(vals)} points, {steps} trapezoid steps "
                                f"of 1 ps", "n": n, "nnz": nnz, "nnz_l": nl, "nnz_u": nu,
-                   "flops_F": int(info.flops), "tiling": "lane per wavefront, factors and vectors in HBM, "
+                   "flops_F": int(info.flops), "tiling": "lane per workgroup of eight wavefronts, factors and vectors in HBM, "
                                                          "replay blocks staged in LDS"},
         "kernel_ms_per_step": round(kern / args.steps, 1),
         "transient_iterations_per_point": round(lane_it / max(conv, 1) / args.steps, 2),

@@ -751,8 +751,8 @@ struct TapeHostProg {
     vector<esl::uint4_t> red_h;
     vector<u32> rsrc;   // the factor slot of each position of the packed FP64 Jacobian
     uint64_t flops = 0;
-    // lanes beyond a workgroup's LDS: the replay in blocks and the solves in
-    // chunks instead of whole-tape row programs and reduce streams
+    // lanes beyond a workgroup's LDS: the replay in blocks and the solves as rows
+    // of their own width instead of whole-tape row programs and reduce streams
     bool big = false;
     u32 width = 0;   // threads of a big lane: words a row
     vector<esl::BigBlock> blk;
@@ -957,19 +957,19 @@ void build_row_programs(const HostTape &t, TapeHostProg &o, u32 min_chain = kMin
 }
 
 // The programs of a big tape (lanes whose factor slots live in HBM), rows of
-// kTeamThreads words. The replay: the ops of the refactor row program in
-// the order build_row_programs adds them (column by column; in a column each
-// target's multiply-subtracts in the order of the column replay, an L target
-// then its pivot division), cut into runs that touch at most block_slots
-// slots; each run is scheduled into rows of its own over LDS positions (the
-// slots it writes first), padded to a multiple of kRing. The runs' rows are
-// stored back to back (a run's prefetches past its end load the next run's
-// words), kRing idle rows after the last. A block as large as a workgroup's
-// LDS leaves the scheduler more columns at once: the 64x64 mesh (2.84 M ops)
-// takes 592 blocks and 87,000 rows of 64 at 4,032 slots, 43 blocks and
-// 10,700 rows of 512 at 18,000. The solves: one program over the solve
-// vector, each factor entry read from its slot. False when a flop's target
-// lies outside its column.
+// W words, one a thread of the lane. The replay: the ops of the refactor row
+// program in the order build_row_programs adds them (column by column; in a
+// column each target's multiply-subtracts in the order of the column replay,
+// an L target then its pivot division), cut into runs that touch at most
+// block_slots slots; each run is scheduled into rows of its own over LDS
+// positions (the slots it writes first), padded to a multiple of kRing. The
+// runs' rows are stored back to back (a run's prefetches past its end load the
+// next run's words), kRing idle rows after the last. A block as large as a
+// workgroup's LDS leaves the scheduler more columns at once: the 64x64 mesh
+// (2.84 M ops) takes 581 blocks and 91,400 rows of 64 at 4,099 slots, 39 blocks
+// and 10,300 rows of 512 at 18,944, 35 and 9,600 at 19,920. The solves: one program
+// over the solve vector, each factor entry read from its slot. False when a
+// flop's target lies outside its column.
 constexpr u32 kBigBlockSlots = 18944, kNarrowBlockSlots = 4032;
 constexpr u32 kBigSlotLimit = 65536 - esl::kTeamThreads;   // 16-bit row-word indices
 
@@ -2029,10 +2029,10 @@ u32 device_cu_count();
 
 // LDS of one lane in a launch of the own-LU kernels over `grid` lanes: when
 // the launch leaves LDS idle (few lanes per CU), room (up to what is idle)
-// past the working set
-// for the lanes' own factor values and the replay's records (room for
-// twice the lead factor's entries, and for the dense form of lanes of at
-// most 64 unknowns), so that their replays and solves run out of LDS; otherwise the working set alone.
+// past the working set for the lanes' own factor values and the replay's
+// records (room for twice the lead factor's entries, and for the dense form of
+// lanes of at most 64 unknowns), so that their replays and solves run out of
+// LDS; otherwise the working set alone.
 u32 own_lds_bytes(u32 lds, u32 grid, u32 n, u32 nnz, u32 nnz_l, u32 nnz_u)
 {
     const u32 cu = device_cu_count();
@@ -2690,7 +2690,7 @@ esl_status esl_engine_create(const esl_deck *deck, esl_engine **out, char *diag,
         return ESL_FAILED;
     }
     // a deck whose Jacobian alone exceeds a workgroup's LDS runs its lanes
-    // one per thread, working sets in HBM
+    // one per workgroup, working sets in HBM
     e->lds_limit = device_lds_max();
     e->big = lds_bytes_for(e->c.nnz + 1, e->c.n) > e->lds_limit;
     hipError_t er = upload_deck(*e);
@@ -3559,8 +3559,9 @@ extern "C" esl_status esl_op_solve(esl_engine *h, const double *values, size_t c
     // depends on the count (its lanes wait on HBM) and grows with the
     // unknowns. At 16,384 points, against the wavefront tiling: 0.17 to 0.67
     // ms at 5 unknowns, 1.30 to 1.38 at 19, but 5.0 to 1.8 at 43, 9.4 to 2.3
-    // at 61 and 210 to 10 at 324: a factor of 4 and more past 48, which twice
-    // as many points do not turn (and the trial cost that first batch 200 ms).
+    // at 61 and 210 to 10 at 324: a factor of 2.8 at 43 and growing (about 3.2
+    // at 49), which twice as many points do not turn (and the trial cost that
+    // first batch 200 ms).
     constexpr u32 kThreadMost = 48;
     constexpr size_t kThreadPoints = 32768;
     // the thread tiling runs FP64 lanes from cold or given starts
@@ -3576,8 +3577,8 @@ extern "C" esl_status esl_op_solve(esl_engine *h, const double *values, size_t c
     }
     u32 tiling = wave_only ? (u32)ESL_TILING_WAVE : o.tiling;
     if (e->big) {
-        // lanes beyond a workgroup's LDS: FP64 from a cold or given start,
-        // one wavefront per lane with the factors in HBM
+        // lanes beyond a workgroup's LDS: FP64 from a cold or given start, one
+        // workgroup per lane with the factors in HBM
         if (fp32 || net) {
             g_last_error = "FP32 factors and learned starts need lanes that fit a workgroup's LDS";
             return ESL_INVALID_ARGUMENT;

@@ -12,11 +12,12 @@
 //   column replay, lane_kernels.zig:49-118) and scatters what it wrote;
 // - solves: the solve vector in LDS, the factor entries read from their
 //   slots ahead of use (lane_kernels.zig:123-143).
-// A team has the whole LDS of a CU: the mesh is 43 blocks and 10,700 rows of
-// 512, each an LDS round trip and a barrier (about 360 cycles; the refactor
-// is 5.1 M of an iteration's 6.1 M cycles). On one wavefront with a quarter
-// of the LDS (four lanes a CU) its blocks hold a few columns at a time, whose
-// dependency chains leave half of 64 threads idle over 81,000 rows. Measured,
+// A team has the whole LDS of a CU: the mesh is 35 blocks and 9,600 rows of
+// 512, each an LDS round trip and a barrier (about 530 cycles with its share
+// of the gathers; the refactor is 5.1 M of an iteration's 6.1 M cycles). On
+// one wavefront with a quarter of the LDS (four lanes a CU) its blocks hold a
+// few columns at a time, whose dependency chains leave half of 64 threads idle
+// over 91,400 rows. Measured,
 // 64 x 64 mesh, an operating point and two steps: 355 ms on one wavefront with
 // the solves in column chunks, 226 ms with the solves as rows, 47 ms on
 // eight (64 lanes; 1,662 and 844 ms for 4,096). A line of 3,000 nodes: 76,

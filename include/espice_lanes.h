@@ -141,7 +141,8 @@ enum {
     ESL_FP32_REFINED = 1   /* FP32 factors, FP64 residual + refinement */
 };
 /* esl_op_options.tiling: how a lane maps onto the GPU. AUTO times both
- * tilings on the engine's first large batch and keeps the faster. */
+ * tilings on the engine's first large batch and keeps the faster (up to 48
+ * unknowns, or past 32,768 points: otherwise a wavefront a lane always wins). */
 enum {
     ESL_TILING_AUTO = 0,
     ESL_TILING_WAVE = 1,    /* one wavefront per lane, factors in LDS */
