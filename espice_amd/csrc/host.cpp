@@ -1013,17 +1013,19 @@ bool build_big_program(const HostTape &t, TapeHostProg &o, u32 block_slots, u32 
         b.rows = ((u32)rows.size() + esl::kRing - 1) / esl::kRing * esl::kRing;
         b.row0 = rows_total;
         rows_total += b.rows;
+        const size_t base = o.blk_words.size();
+        o.blk_words.resize(base + (size_t)b.rows * W);
         for (u32 r = 0; r < b.rows; r++) {
             const u32 cnt = r < rows.size() ? (u32)rows[r].size() : 0u;
             const u32 kind = cnt ? g.op(rows[r][0]).kind : (u32)esl::R_NOP;
-            for (u32 th = 0; th < W; th++) {
+            esl::uint2_t *w = o.blk_words.data() + base + (size_t)r * W;
+            for (u32 th = 0; th < cnt; th++) {
+                const SchedOp &op = g.op(rows[r][th]);
+                w[th] = esl::uint2_t{op.d | (op.b << 16), op.c | (op.kind << 16) | (op.flags << 20)};
+            }
+            for (u32 th = cnt; th < W; th++) {
                 const u32 pad = m + th;
-                esl::uint2_t w{pad | (pad << 16), pad | (kind << 16)};
-                if (th < cnt) {
-                    const SchedOp &op = g.op(rows[r][th]);
-                    w = esl::uint2_t{op.d | (op.b << 16), op.c | (op.kind << 16) | (op.flags << 20)};
-                }
-                o.blk_words.push_back(w);
+                w[th] = esl::uint2_t{pad | (pad << 16), pad | (kind << 16)};
             }
         }
         for (u32 k = b.slot_off; k < (u32)o.blk_slots.size(); k++) local[o.blk_slots[k]] = NONE;
@@ -2543,7 +2545,9 @@ TapeHostProg *build_tape(const Engine &e, const HostTape &t, const char *&err)
 // A tape's pivot sequence, and for a big engine the team its programs are for.
 vector<u32> tape_key(const Engine &e, const HostTape &t)
 {
-    vector<u32> key = t.pinv;
+    vector<u32> key;
+    key.reserve(t.pinv.size() + t.flags.size() + 1);
+    key.insert(key.end(), t.pinv.begin(), t.pinv.end());
     key.insert(key.end(), t.flags.begin(), t.flags.end());
     key.push_back(e.big ? e.team : 0);
     return key;
